@@ -18,6 +18,8 @@ LIB = os.path.join(OUT_DIR, "libpdq.so")
 UNITS = [
     "pdq_capi.hip",
     "pdq_coop.hip",
+    "pdq_coop_wave_filter.hip",
+    "pdq_coop_wave_smoother.hip",
     "pdq_lane.hip",
     "pdq_lane_filter.hip",
     "pdq_lane_fixedpoint.hip",

@@ -62,6 +62,10 @@ int num_cus();
 
 // Launchers (one per translation unit, compiled in parallel).
 int launch_coop(KArgs& a, int G, hipStream_t st);
+void launch_zero_queue(int* queue, hipStream_t st);
+// The same for fixed shapes at 64 lanes per instance (pdq_coop_wave_*.hip).
+int launch_coop_wave_filter(KArgs& a, hipStream_t st);
+int launch_coop_wave_smoother(KArgs& a, hipStream_t st);
 // Lane-per-instance isotropic kernel (pdq_lane.hip): shapes (N = nu + 1, d)
 // it is instantiated for and its launcher.
 bool lane_supported(int N, int D);

@@ -1915,6 +1915,10 @@ __global__ void zero_queue(int* p) {
   if (threadIdx.x == 0) p[0] = 0;
 }
 
+void launch_zero_queue(int* queue, hipStream_t st) {
+  hipLaunchKernelGGL(zero_queue, dim3(1), dim3(64), 0, st, queue);
+}
+
 int launch_taylor_tangents(int vf, int d, int np, int n_inst, int num, int ntan, const double* params,
                            const double* y0, const double* t0, double* out, hipStream_t st) {
   hipLaunchKernelGGL(taylor_tangent_kernel, dim3((n_inst + 63) / 64), dim3(64), 0, st, vf, d, np, n_inst, num, ntan,
@@ -1943,7 +1947,7 @@ int launch_coop_g(KArgs& a, hipStream_t st) {
   const long need = ((long)a.n_inst + ipw - 1) / ipw;
   const long cap = (long)per_cu * num_cus();
   const int grid = (int)std::max<long>(1, std::min(need, cap));
-  hipLaunchKernelGGL(zero_queue, dim3(1), dim3(64), 0, st, a.queue);
+  launch_zero_queue(a.queue, st);
   hipLaunchKernelGGL(kern, dim3(grid), dim3(64), lds, st, a);
   PDQ_HIP_TRY(hipGetLastError());
   return PDQ_OK;
@@ -1979,7 +1983,23 @@ int launch_offgrid_coop(OffgridCoopArgs& o, int G, hipStream_t st) {
   return host_error(PDQ_ERR_INVALID, "lanes per query must be one of 4, 8, 16, 32, 64 (got %d)", G);
 }
 
+// The solves the fixed-shape kernels (pdq_coop_wave.h) take over: one instance
+// per wavefront, d = 2, the shapes instantiated, the options they hold.  Their
+// arithmetic is this file's at 64 lanes per instance, so the choice does not
+// show in the results.
+static bool coop_wave_supported(const KArgs& a) {
+  const pdq_config& c = a.cfg;
+  if (a.mode == MODE_LML || a.lay.d != 2 || a.lay.expo) return false;
+  if (c.error_estimator != PDQ_ERROR_RESIDUAL_STD || c.error_re_linearize || c.re_linearize_after_calibration)
+    return false;
+  if (c.factorisation == PDQ_DENSE) return a.lay.N >= 3 && a.lay.N <= 6;
+  return c.factorisation == PDQ_ISOTROPIC && (a.lay.N == 3 || a.lay.N == 6) &&
+         (c.constraint == PDQ_TS0 || c.jacobian == PDQ_JAC_EXACT);
+}
+
 int launch_coop(KArgs& a, int G, hipStream_t st) {
+  if (G == 64 && coop_wave_supported(a))
+    return a.cfg.strategy == PDQ_FILTER ? launch_coop_wave_filter(a, st) : launch_coop_wave_smoother(a, st);
   switch (G) {
     case 4: return launch_coop_g<4>(a, st);
     case 8: return launch_coop_g<8>(a, st);

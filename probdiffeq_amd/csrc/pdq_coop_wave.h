@@ -1,0 +1,942 @@
+// The cooperative solver for fixed shapes: one IVP instance per wavefront,
+// every matrix size a compile-time constant, the QR in registers (pdq_wave.h).
+//
+// It computes what the run-time-shape kernel (pdq_coop.hip) computes with 64
+// lanes per instance, in the same order of operations, so that for finite
+// data every output is the same bit for bit.  What bounds both is the latency
+// of one instance's serial chain (a few QRs of 10 to 24 rows per attempt; a
+// batch of 1024 has one wavefront per SIMD).  The run-time-shape kernel spends
+// that chain on LDS round trips: every operand of every reflector, with
+// run-time loop bounds.  Here
+// * lane j holds column j of a stack in registers and builds it there from the
+//   factors in LDS (lane i then also owns row i of the resulting factor);
+// * the zeros of the stacks (triangular factors, the IWP transition kron(A, I),
+//   the observation's two derivatives) are skipped at compile time;
+// * the loop is a state machine whose operations share one prediction: an
+//   attempt and the two halves of an interpolation (as in pdq_lane.h), so that
+//   a kernel holds each piece of code once;
+// * the solve's scalars (t, dt, output scale, counts) are wave-uniform
+//   registers, and every loop and branch on them is a scalar one.
+// Measured on one MI355X, the same outputs bit for bit: 1024 dense
+// Lotka-Volterra solves (nu = 4, filter, 200 points) 71.3 -> 14.3 ms, one such
+// solve 32.3 -> 5.7 ms, 1024 stiff van der Pol solves (nu = 5, ts1) 20.9 -> 3.2 ms.
+// Configurations it does not hold (error_state_std, re-linearisation, Monte
+// Carlo Jacobians, the LML) stay with the run-time-shape kernel.
+#pragma once
+
+#include "pdq_args.h"
+#include "pdq_wave.h"
+
+namespace pdq {
+
+// A fixed shape: N = nu + 1, d, dense or isotropic, smoother or filter.
+template <int N_, int D_, bool DENSE_, bool SMOOTHER_>
+struct WShape {
+  static constexpr int N = N_, d = D_;
+  static constexpr bool dense = DENSE_, smoother = SMOOTHER_;
+  static constexpr int nc = dense ? N * d : N, mc = dense ? 1 : d, ko = dense ? d : 1;
+  static constexpr int st = dense ? d : 1;  // stride of the IWP transition's non-zeros
+  static constexpr int nn = nc * nc, ms = nc * mc;
+  // LDS (doubles): the transition, then the instance
+  static constexpr int oA = 0, oQ = oA + nn;
+  static constexpr int oP = oQ + nn, oPI = oP + nc;
+  static constexpr int oUm = oPI + nc, oPm = oUm + ms, oPL = oPm + ms, oTmp = oPL + nn;
+  // a conditional: A, mean, factor, to_latent, to_observed
+  static constexpr int cA = 0, cm = cA + nn, cL = cm + ms, ctl = cL + nn, cto = ctl + nc, csize = cto + nc;
+  static constexpr int oB = oTmp + ms, oE = oB + (smoother ? csize : 0);
+  // three solution slots: mean, factor, conditional
+  static constexpr int sm = 0, sL = sm + ms, sC = sL + nn, ssize = sC + (smoother ? csize : 0);
+  static constexpr int oS = oE + (smoother ? csize : 0);
+  static constexpr int oPrm = oS + 3 * ssize;
+  static constexpr int fixed_size = oPrm;  // + n_params
+  static_assert(2 * nc <= 32, "a column of the revert block per lane, a power per half wavefront");
+  static_assert(N >= 2 && d <= 2, "the observation's rows and the columns' sums");
+};
+
+// The stacks' patterns (WaveQrPlan).
+template <class SH>
+struct WPatStack {  // [dense; upper triangle]
+  static constexpr int nc = SH::nc, M = 2 * nc, NP = nc, MROWS = M;
+  static constexpr int row(int r) { return r; }
+  static constexpr bool nz(int r, int c) { return r < nc || r - nc <= c; }
+};
+template <class SH>
+struct WPatRevert {  // [[upper triangle, 0], [dense, upper triangle]]
+  static constexpr int nc = SH::nc, M = 2 * nc, NP = M, MROWS = M;
+  static constexpr int row(int r) { return r; }
+  static constexpr bool nz(int r, int c) { return c < nc ? (r >= nc || r <= c) : (r >= nc && r - nc <= c - nc); }
+};
+template <class SH>
+struct WPatUpdate {  // [[diagonal, 0], [(H L)^T, L^T]]: H reads derivatives 0 and 1, the first 2 ko rows of L
+  static constexpr int nc = SH::nc, ko = SH::ko, M = ko + nc, NP = M, MROWS = M;
+  static constexpr int row(int r) { return r; }
+  static constexpr bool nz(int r, int c) { return r < ko ? r == c : (c < ko ? r - ko < 2 * ko : r - ko <= c - ko); }
+};
+template <class SH>
+struct WPatFx {  // [(H L)^T; diagonal], without (H L)^T's zero rows
+  static constexpr int nc = SH::nc, ko = SH::ko, M = 3 * ko, NP = ko, MROWS = nc + ko;
+  static constexpr int row(int r) { return r < 2 * ko ? r : nc + r - 2 * ko; }
+  static constexpr bool nz(int r, int c) { return r < 2 * ko || r - 2 * ko == c; }
+};
+
+// Orders the wavefront's LDS accesses.
+__device__ __forceinline__ void wave_sync() { Grp<64>{}.sync(); }
+
+template <int n>
+__device__ __forceinline__ void wave_copy(int l, double* dst, const double* src) {
+#pragma unroll
+  for (int e0 = 0; e0 < n; e0 += 64) {
+    const int e = e0 + l;
+    if (e < n) dst[e] = src[e];
+  }
+}
+
+// A solution's scalars.
+struct WScal {
+  double t, os, nsteps, mle_run, mle_n;
+  bool ident;
+};
+
+// The linearisation: the operator's non-zero block J (ko x 2 ko, derivatives 0
+// and 1; ts1 only) and b (ko x mc), in every lane.
+template <class SH>
+struct WLin {
+  double J[SH::ko * 2 * SH::ko], b[SH::ko * SH::mc];
+};
+
+// The step's quantities that its parts hand on (uniform).
+struct WErr {
+  double oL[4];  // the error model's observed factor (ko x ko)
+  double sigma;
+};
+
+template <class SH>
+struct WCtx {
+  const KArgs* a;
+  double* lds;
+  int l, inst;
+  __device__ __forceinline__ double* P() const { return lds + SH::oP; }
+  __device__ __forceinline__ double* PI() const { return lds + SH::oPI; }
+  __device__ __forceinline__ const double* A() const { return lds + SH::oA; }
+  __device__ __forceinline__ const double* Q() const { return lds + SH::oQ; }
+  __device__ __forceinline__ const double* prm() const { return lds + SH::oPrm; }
+  __device__ __forceinline__ double* slot(int s) const { return lds + SH::oS + s * SH::ssize; }
+  __device__ __forceinline__ bool ts1() const { return a->cfg.constraint == PDQ_TS1; }
+};
+
+// preconditioner_taylor (utilities.py:74-84) into P and PI, and dt^nord (in
+// every lane): one evaluation of pow, lanes 0.. the powers, lanes 32.. their
+// inverses, lane 31 dt^nord.
+template <class SH>
+__device__ __forceinline__ double w_precon(const WCtx<SH>& c, double dt, int nord) {
+  const int i = c.l & 31, pw = i < SH::nc ? SH::N - 1 - (SH::dense ? i / SH::d : i) : 0;
+  const int ex = c.l == 31 ? nord : (c.l < 32 ? pw : -pw);
+  const double s = factorial_d(pw), p = pow(dt, (double)ex);
+  if (i < SH::nc) (c.l < 32 ? c.P() : c.PI())[i] = c.l < 32 ? p / s : p * s;
+  wave_sync();
+  return wave_bcast(p, 31);
+}
+
+template <class SH>
+__device__ __forceinline__ double w_noise_scale(const WCtx<SH>& c, double dt, double s) {
+  if (SH::dense) return sqrt(fabs(dt)) * s;
+  return sqrt(fabs(dt)) * c.a->cfg.base_output_scale * s;
+}
+
+// Row i's lane: lane i < nc (the others repeat row nc - 1 and write nothing).
+template <class SH>
+__device__ __forceinline__ int w_row(const WCtx<SH>& c) {
+  return c.l < SH::nc ? c.l : SH::nc - 1;
+}
+
+// The entries A[i][k] of row i of the transition in ascending k: f(A[i][k], k).
+template <class SH, class F>
+__device__ __forceinline__ void w_prior_terms(const WCtx<SH>& c, int i, F f) {
+  const int k0 = SH::st == 1 ? 0 : i % SH::st;
+#pragma unroll
+  for (int q = 0; q < SH::N; ++q) {
+    const int k = q * SH::st + k0;
+    f(c.A()[i * SH::nc + k], k);
+  }
+}
+
+// Column i of (A (|p| * L))^T: a[r] = sum_k A[i][k] (|p_k| L[k][r]), L lower
+// triangular (p is positive but for non-finite steps).
+template <class SH>
+__device__ __forceinline__ void w_prior_column(const WCtx<SH>& c, int i, const double* L, bool abs_p, double* a) {
+  const int k0 = SH::st == 1 ? 0 : i % SH::st;
+#pragma unroll
+  for (int r = 0; r < SH::nc; ++r) a[r] = 0.0;
+#pragma unroll
+  for (int q = 0; q < SH::N; ++q) {
+    const int k = q * SH::st + k0;
+    const double ak = c.A()[i * SH::nc + k], p = c.PI()[k], pk = abs_p ? fabs(p) : p;
+#pragma unroll
+    for (int r = 0; r < (q + 1) * SH::st; ++r) a[r] += ak * (pk * L[k * SH::nc + r]);
+  }
+}
+
+// apply_flat of the transition to a mean x: out = p * (A (p^-1 * x)) (dense)
+// or (p * A) (p^-1 * x) (isotropic).
+template <class SH>
+__device__ __forceinline__ void w_apply_flat_mean(const WCtx<SH>& c, const double* x, double* out) {
+  const int i = w_row(c);
+  double acc[SH::mc] = {};
+  w_prior_terms(c, i, [&](double ak, int k) {
+#pragma unroll
+    for (int col = 0; col < SH::mc; ++col) {
+      if (SH::dense) acc[col] += ak * (c.PI()[k] * x[k * SH::mc + col]);
+      else acc[col] += (c.P()[i] * ak) * (c.PI()[k] * x[k * SH::mc + col]);
+    }
+  });
+  if (c.l < SH::nc)
+#pragma unroll
+    for (int col = 0; col < SH::mc; ++col)
+      out[i * SH::mc + col] = SH::dense ? c.P()[i] * (acc[col] + 0.0) : acc[col] + 0.0;
+  wave_sync();
+}
+
+// ts0 / ts1 linearisation at the mean Xm (ssm_impl_dense.py:237-334,
+// ssm_impl_isotropic.py:298-355 with the exact trace).
+template <class SH>
+__device__ __forceinline__ void w_linearize(const WCtx<SH>& c, const double* Xm, double t, WLin<SH>& lin) {
+  constexpr int d = SH::d, ko = SH::ko, K2 = 2 * SH::ko;
+  const int id = c.a->cfg.vector_field;
+  double y[d];
+#pragma unroll
+  for (int j = 0; j < d; ++j) y[j] = Xm[j];
+  double f[d];
+#pragma unroll
+  for (int j = 0; j < d; ++j) f[j] = vf_component(id, d, y, c.prm(), t, j);
+  if (!c.ts1()) {
+#pragma unroll
+    for (int j = 0; j < d; ++j) lin.b[j] = wave_rounded(-f[j]);
+#pragma unroll
+    for (int e = 0; e < ko * K2; ++e) lin.J[e] = 0.0;
+    return;
+  }
+  if constexpr (SH::dense) {
+#pragma unroll
+    for (int i = 0; i < ko; ++i) {
+#pragma unroll
+      for (int j = 0; j < K2; ++j)
+        lin.J[i * K2 + j] = j < d ? -vf_jac(id, d, y, c.prm(), i, j < d ? j : 0) : (j == d + i ? 1.0 : 0.0);
+      double jm = 0.0;
+#pragma unroll
+      for (int k = 0; k < K2; ++k) jm += lin.J[i * K2 + k] * Xm[k];
+      lin.b[i] = wave_rounded((Xm[d + i] - f[i]) - jm);
+    }
+  } else {
+    double tr = 0.0;
+#pragma unroll
+    for (int j = 0; j < d; ++j) tr += -vf_jac(id, d, y, c.prm(), j, j);
+    const double h0 = tr / (double)d;
+    lin.J[0] = h0;
+    lin.J[1] = 1.0;
+#pragma unroll
+    for (int j = 0; j < d; ++j) {
+      const double r = Xm[d + j] - f[j];
+      lin.b[j] = wave_rounded(r - (h0 * Xm[j] + Xm[d + j]));
+    }
+  }
+}
+
+// Entry (o, col) of H X for a mean X.
+template <class SH>
+__device__ __forceinline__ double w_hm(const WCtx<SH>& c, const WLin<SH>& lin, const double* X, int o, int col) {
+  constexpr int K2 = 2 * SH::ko;
+  if (!c.ts1()) return X[(SH::ko + o) * SH::mc + col];
+  double acc = 0.0;
+#pragma unroll
+  for (int k = 0; k < K2; ++k) acc += lin.J[o * K2 + k] * X[k * SH::mc + col];
+  return acc;
+}
+
+// Column r of row o (the lane's) of H L for a lower-triangular factor given by
+// its entries L(k, r).
+template <class SH, class LF>
+__device__ __forceinline__ double w_hl(const WCtx<SH>& c, const WLin<SH>& lin, LF L, int o, int r) {
+  constexpr int K2 = 2 * SH::ko;
+  if (!c.ts1()) return L(SH::ko + o, r);
+  double acc = 0.0;
+#pragma unroll
+  for (int k = 0; k < K2; ++k) {
+    double j = lin.J[k];
+#pragma unroll
+    for (int q = 1; q < SH::ko; ++q) j = o == q ? lin.J[q * K2 + k] : j;
+    acc += j * L(k, r);
+  }
+  return acc;
+}
+
+// residual_whitened_rms against zero data (ssm_impl_dense.py:156-160,
+// isotropic :203-207) of an observed marginal held by every lane.
+template <class SH>
+__device__ __forceinline__ double w_rms_zero(const double* om, const double* oL) {
+  constexpr int k = SH::ko, m = SH::mc;
+  double sum[m];
+#pragma unroll
+  for (int col = 0; col < m; ++col) {
+    double x[k], sq = 0.0;
+#pragma unroll
+    for (int i = 0; i < k; ++i) {
+      double s = SH::dense ? (0.0 - om[i * m + col]) : om[i * m + col];
+#pragma unroll
+      for (int j = 0; j < i; ++j) s -= oL[i * k + j] * x[j];
+      x[i] = s / oL[i * k + i];
+      sq = wave_add_square(sq, x[i]);
+    }
+    sum[col] = sq;
+  }
+  double tot = sum[0];
+  if constexpr (m == 2) tot = wave_add(sum[0], sum[1]);
+  return sqrt(tot) / sqrt((double)(k * m));
+}
+
+// The error model's observed marginal at the extrapolation Um with output
+// scale 1 (fx.marginalise of (Um, |p| (s1 Q))): oL and sigma, in every lane.
+template <class SH>
+__device__ __forceinline__ void w_calibrate(const WCtx<SH>& c, const WLin<SH>& lin, const double* Um, double s1,
+                                            WErr& err) {
+  constexpr int k = SH::ko, m = SH::mc;
+  const int o = c.l < k ? c.l : k - 1;
+  const double damp = c.a->cfg.damp;
+  double a[3 * k], om[k * m];
+#pragma unroll
+  for (int r = 0; r < 2 * k; ++r)
+    a[r] = w_hl(c, lin, [&](int q, int col) { return wave_rounded(fabs(c.P()[q]) * (s1 * c.Q()[q * SH::nc + col])); }, o, r);
+#pragma unroll
+  for (int r = 0; r < k; ++r) a[2 * k + r] = r == o ? damp : 0.0;
+#pragma unroll
+  for (int i = 0; i < k; ++i)
+#pragma unroll
+    for (int col = 0; col < m; ++col) om[i * m + col] = w_hm(c, lin, Um, i, col) + lin.b[i * m + col];
+  wave_qr<WPatFx<SH>>(a, c.l);
+#pragma unroll
+  for (int i = 0; i < k; ++i)
+#pragma unroll
+    for (int j = 0; j < k; ++j) err.oL[i * k + j] = j <= i ? wave_bcast(a[j], i) : 0.0;
+  err.sigma = w_rms_zero<SH>(om, err.oL);
+}
+
+// marginalise of the transition (ssm_impl_dense.py:24-33, isotropic :81-89).
+template <class SH>
+__device__ __forceinline__ void w_marginalise_prior(const WCtx<SH>& c, double s, const double* Xm, const double* XL,
+                                                    double* Ym, double* YL) {
+  constexpr int n = SH::nc, m = SH::mc;
+  const int i = w_row(c);
+  double a[2 * n], acc[m] = {};
+  w_prior_column(c, i, XL, false, a);
+#pragma unroll
+  for (int r = 0; r < n; ++r) a[n + r] = wave_rounded(s * c.Q()[i * n + r]);
+  w_prior_terms(c, i, [&](double ak, int k) {
+#pragma unroll
+    for (int col = 0; col < m; ++col) acc[col] += ak * (c.PI()[k] * Xm[k * m + col]);
+  });
+  wave_qr<WPatStack<SH>>(a, c.l);
+  const double p = c.P()[i];
+  if (c.l < n) {
+#pragma unroll
+    for (int col = 0; col < m; ++col) Ym[i * m + col] = p * (acc[col] + 0.0);
+#pragma unroll
+    for (int j = 0; j < n; ++j) YL[i * n + j] = fabs(p) * wave_r(a, j, i);
+  }
+  wave_sync();
+}
+
+// revert of the transition (ssm_impl_dense.py:51-77, isotropic :107-133,
+// cholesky_util.py:27-82): X -> observed (Ym, YL) and backward conditional B.
+template <class SH>
+__device__ __forceinline__ void w_revert_prior(const WCtx<SH>& c, double s, const double* Xm, const double* XL,
+                                               double* Ym, double* YL, double* B, double* tmp) {
+  constexpr int n = SH::nc, m = SH::mc;
+  // lanes 0..n-1: the left columns, lanes n..2n-1: the right ones (the others repeat the last)
+  const bool right = c.l >= n;
+  const int i = right ? (c.l < 2 * n ? c.l - n : n - 1) : c.l;
+  double a[2 * n], acc[m] = {};
+  const double p = c.P()[i], pi = c.PI()[i];
+  {
+    double left[n];
+    w_prior_column(c, i, XL, true, left);
+#pragma unroll
+    for (int r = 0; r < n; ++r) {
+      const double x = wave_rounded(fabs(pi) * XL[i * n + r]), q = wave_rounded(s * c.Q()[i * n + r]);
+      a[r] = right ? 0.0 : q;
+      a[n + r] = right ? x : left[r];
+    }
+  }
+  // mean_observed = A (p^-1 * m)
+  w_prior_terms(c, i, [&](double ak, int k) {
+#pragma unroll
+    for (int col = 0; col < m; ++col) acc[col] += ak * (c.PI()[k] * Xm[k * m + col]);
+  });
+  double xm[m];
+#pragma unroll
+  for (int col = 0; col < m; ++col) {
+    xm[col] = Xm[i * m + col];
+    if (!right) tmp[i * m + col] = acc[col] + 0.0;
+  }
+  wave_sync();
+  wave_qr<WPatRevert<SH>>(a, c.l);
+  // the gain's row i: back substitution of the right column with R_Y
+  double gn[n];
+  wave_backsolve<n>(a, c.l, gn);
+  if (right && c.l < 2 * n) {
+#pragma unroll
+    for (int k = 0; k < n; ++k) B[SH::cA + i * n + k] = gn[k];
+#pragma unroll
+    for (int col = 0; col < m; ++col) {
+      double ac = 0.0;
+#pragma unroll
+      for (int k = 0; k < n; ++k) ac += gn[k] * tmp[k * m + col];
+      B[SH::cm + i * m + col] = pi * xm[col] - ac;
+    }
+#pragma unroll
+    for (int j = 0; j < n; ++j) B[SH::cL + i * n + j] = j <= i ? a[n + j] : 0.0;
+    B[SH::ctl + i] = 1.0 / p;
+    B[SH::cto + i] = 1.0 / pi;
+  }
+  if (!right) {
+#pragma unroll
+    for (int col = 0; col < m; ++col) Ym[i * m + col] = p * tmp[i * m + col];
+#pragma unroll
+    for (int j = 0; j < n; ++j) YL[i * n + j] = fabs(p) * wave_r(a, j, i);
+  }
+  wave_sync();
+}
+
+// merge (ssm_impl_dense.py:35-49, isotropic :91-105): R = F o B, F possibly the
+// identity (then exactly the rescaled B).  R may not share storage with F or B.
+template <class SH>
+__device__ __forceinline__ void w_merge(const WCtx<SH>& c, bool ident, const double* F, const double* B, double* R) {
+  constexpr int n = SH::nc, m = SH::mc;
+  const double *oA = B + SH::cA, *om = B + SH::cm, *oL = B + SH::cL, *oto = B + SH::cto;
+  const int i = w_row(c);
+  if (ident) {
+#pragma unroll
+    for (int e0 = 0; e0 < n * n; e0 += 64) {
+      const int e = e0 + c.l;
+      if (e < n * n) {
+        const double T = 1.0 * oto[e / n];
+        R[SH::cA + e] = T * oA[e];
+        R[SH::cL + e] = fabs(T) * oL[e];
+      }
+    }
+    if (c.l < n) {
+#pragma unroll
+      for (int col = 0; col < m; ++col) R[SH::cm + i * m + col] = (1.0 * oto[i]) * om[i * m + col] + 0.0;
+      R[SH::ctl + i] = B[SH::ctl + i];
+      R[SH::cto + i] = 1.0;
+    }
+    wave_sync();
+    return;
+  }
+  const double *sA = F + SH::cA, *sm = F + SH::cm, *sL = F + SH::cL, *stl = F + SH::ctl;
+  double a[2 * n], acc[m] = {};
+#pragma unroll
+  for (int r = 0; r < n; ++r) {
+    a[r] = 0.0;
+    a[n + r] = sL[i * n + r];  // R2 = C1^T
+  }
+  // R1 = (A1 (|T| o C2))^T with C2 lower triangular, and m = A1 (T o m2) + m1
+#pragma unroll
+  for (int k = 0; k < n; ++k) {
+    const double T = stl[k] * oto[k], g = sA[i * n + k];
+#pragma unroll
+    for (int r = 0; r <= k; ++r) a[r] += g * (fabs(T) * oL[k * n + r]);
+#pragma unroll
+    for (int col = 0; col < m; ++col) acc[col] += g * (T * om[k * m + col]);
+  }
+  // A = A1 (T o A2), spread over all lanes
+#pragma unroll
+  for (int e0 = 0; e0 < n * n; e0 += 64) {
+    const int e = e0 + c.l < n * n ? e0 + c.l : n * n - 1, ei = e / n, ej = e % n;
+    double ac = 0.0;
+#pragma unroll
+    for (int k = 0; k < n; ++k) ac += sA[ei * n + k] * ((stl[k] * oto[k]) * oA[k * n + ej]);
+    if (e0 + c.l < n * n) R[SH::cA + e] = ac;
+  }
+  wave_qr<WPatStack<SH>>(a, c.l);
+  if (c.l < n) {
+#pragma unroll
+    for (int col = 0; col < m; ++col) R[SH::cm + i * m + col] = acc[col] + sm[i * m + col];
+#pragma unroll
+    for (int j = 0; j < n; ++j) R[SH::cL + i * n + j] = wave_r(a, j, i);
+    R[SH::ctl + i] = B[SH::ctl + i];
+    R[SH::cto + i] = F[SH::cto + i];
+  }
+  wave_sync();
+}
+
+// marginalise of a backward conditional C (estimators_and_losses.py:156-178).
+// Y may share storage with X: a lane reads its inputs before the QR.
+template <class SH>
+__device__ __forceinline__ void w_marginalise_cond(const WCtx<SH>& c, const double* C, const double* Xm,
+                                                   const double* XL, double* Ym, double* YL) {
+  constexpr int n = SH::nc, m = SH::mc;
+  const int i = w_row(c);
+  double a[2 * n], acc[m] = {};
+#pragma unroll
+  for (int r = 0; r < n; ++r) {
+    a[r] = 0.0;
+    a[n + r] = C[SH::cL + i * n + r];
+  }
+#pragma unroll
+  for (int k = 0; k < n; ++k) {
+    const double g = C[SH::cA + i * n + k], tl = C[SH::ctl + k];
+#pragma unroll
+    for (int r = 0; r <= k; ++r) a[r] += g * (tl * XL[k * n + r]);
+#pragma unroll
+    for (int col = 0; col < m; ++col) acc[col] += g * (tl * Xm[k * m + col]);
+  }
+  wave_sync();
+  wave_qr<WPatStack<SH>>(a, c.l);
+  const double to = C[SH::cto + i];
+  if (c.l < n) {
+#pragma unroll
+    for (int col = 0; col < m; ++col) Ym[i * m + col] = to * (acc[col] + C[SH::cm + i * m + col]);
+#pragma unroll
+    for (int j = 0; j < n; ++j) YL[i * n + j] = fabs(to) * wave_r(a, j, i);
+  }
+  wave_sync();
+}
+
+// fx.revert(pred) and apply_flat(data) (ssm_impl_api.py:112-132):
+// (Pm, PL) -> (Xm, XL); `obs` receives the observed marginal's mean and factor.
+template <class SH>
+__device__ __forceinline__ void w_update(const WCtx<SH>& c, const WLin<SH>& lin, const double* Pm, const double* PL,
+                                         double* Xm, double* XL, double* om, double* oL) {
+  constexpr int n = SH::nc, k = SH::ko, m = SH::mc;
+  const double damp = c.a->cfg.damp;
+  // lanes 0..k-1: the observation's columns, lanes k..k+n-1: the state's (the others repeat the last)
+  const bool state = c.l >= k;
+  const int o = state ? k - 1 : c.l;
+  const int i = state ? (c.l < k + n ? c.l - k : n - 1) : 0;
+  double a[k + n];
+#pragma unroll
+  for (int r = 0; r < k; ++r) a[r] = !state && r == o ? damp : 0.0;
+#pragma unroll
+  for (int r = 0; r < n; ++r) {
+    const double x = PL[i * n + r];
+    double h = 0.0;
+    if (r < 2 * k) h = w_hl(c, lin, [&](int q, int col) { return PL[q * n + col]; }, o, r);
+    a[k + r] = state ? x : h;
+  }
+#pragma unroll
+  for (int r = 0; r < k; ++r)
+#pragma unroll
+    for (int col = 0; col < m; ++col) om[r * m + col] = w_hm(c, lin, Pm, r, col) + lin.b[r * m + col];
+  wave_qr<WPatUpdate<SH>>(a, c.l);
+  double gn[k];
+  wave_backsolve<k>(a, c.l, gn);
+  if (state && c.l < k + n) {
+#pragma unroll
+    for (int col = 0; col < m; ++col) {
+      double acc = 0.0;
+#pragma unroll
+      for (int r = 0; r < k; ++r) acc += gn[r] * om[r * m + col];
+      Xm[i * m + col] = Pm[i * m + col] - acc;
+    }
+#pragma unroll
+    for (int j = 0; j < n; ++j) XL[i * n + j] = j <= i ? a[k + j] : 0.0;
+  }
+#pragma unroll
+  for (int i2 = 0; i2 < k; ++i2)
+#pragma unroll
+    for (int j = 0; j < k; ++j) oL[i2 * k + j] = j <= i2 ? wave_bcast(a[j], i2) : 0.0;
+  wave_sync();
+}
+
+// error_residual_std.estimate_error_norm (solvers.py:925-996); dtn = dt^nord.
+// Lane k < d takes dimension k.
+template <class SH>
+__device__ __forceinline__ double w_error_power(const WCtx<SH>& c, const WErr& err, const double* prev_m,
+                                                const double* prop_m, double dtn, int nord) {
+  constexpr int k = SH::ko, d = SH::d;
+  const pdq_config& cfg = c.a->cfg;
+  const double fact = nord == 1 ? 1.0 : 2.0;
+  const int q = c.l < d ? c.l : d - 1;
+  // std of the lane's rescaled observed row: dense per-row qr_r (|beta| of
+  // dlarfg), isotropic vector_norm
+  const int r = k == 1 ? 0 : q;
+  double row[k];
+#pragma unroll
+  for (int j = 0; j < k; ++j) {
+    row[j] = err.oL[j];
+#pragma unroll
+    for (int x = 1; x < k; ++x) row[j] = r == x ? err.oL[x * k + j] : row[j];
+  }
+  double ss = 0.0;
+#pragma unroll
+  for (int j = 1; j < k; ++j) {
+    const double x = err.sigma * row[j];
+    ss += x * x;
+  }
+  const double alpha = err.sigma * row[0];
+  double std;
+  if (SH::dense) std = ss == 0.0 ? fabs(alpha) : fabs(hypot(alpha, sqrt(ss)));
+  else std = sqrt(alpha * alpha + ss);
+  const double e = std * dtn / fact;
+  const double ref = fmax(fabs(prev_m[q]), fabs(prop_m[q]));
+  double norm;
+  if (cfg.error_norm == PDQ_NORM_SCALE_THEN_RMS) {
+    const double rr = e / (cfg.atol + cfg.rtol * fabs(ref));
+    double tot = 0.0;
+#pragma unroll
+    for (int x = 0; x < d; ++x) {
+      const double rx = wave_bcast(rr, x);
+      tot = wave_add_square(tot, rx);
+    }
+    norm = sqrt(tot) / sqrt((double)d);
+  } else {
+    double sa = 0.0, sr = 0.0;
+#pragma unroll
+    for (int x = 0; x < k; ++x) {
+      const double ex = wave_bcast(e, x);
+      sa = wave_add_square(sa, ex);
+    }
+#pragma unroll
+    for (int x = 0; x < d; ++x) {
+      const double rx = wave_bcast(ref, x);
+      sr = wave_add_square(sr, rx);
+    }
+    norm = (sqrt(sa) / sqrt((double)k)) / (cfg.atol + cfg.rtol * (sqrt(sr) / sqrt((double)d)));
+  }
+  return pow(norm, -1.0 / (double)SH::N);
+}
+
+// controllers.py:66-84 / :24-63
+__device__ __forceinline__ double w_control(const pdq_config& cfg, double dt, double& cstate, double ep) {
+  if (cfg.control == PDQ_CONTROL_INTEGRAL) {
+    const double ratio = cfg.safety * ep;
+    return fmax(cfg.factor_min, fmin(ratio, cfg.factor_max)) * dt;
+  }
+  const double gi = pow(ep, cfg.exponent_integral);
+  const double gp = pow(ep / cstate, cfg.exponent_proportional);
+  const double ratio = cfg.safety * gi * gp;
+  const double sf = fmax(cfg.factor_min, fmin(ratio, cfg.factor_max));
+  if (ep >= 1.0) cstate = ep;
+  return sf * dt;
+}
+
+// ---------------------------------------------------------------- outputs
+template <class SH>
+__device__ __forceinline__ void w_write_normal(const WCtx<SH>& c, const double* m, const double* L, double* gm,
+                                               double* gL) {
+  if (gm) wave_copy<SH::ms>(c.l, gm, m);
+  if (gL) wave_copy<SH::nn>(c.l, gL, L);
+}
+
+// Checkpoint k: the filter's marginal, or the smoothers' filtering marginal
+// and (C) the backward conditional that leads to it, an identity with `ident`.
+template <class SH>
+__device__ __forceinline__ void w_write_checkpoint(const WCtx<SH>& c, int k, double t, const double* m,
+                                                   const double* L, double os, double nsteps, const double* C,
+                                                   bool ident) {
+  const pdq_solution& o = c.a->out;
+  const int K = c.a->K;
+  const size_t row = (size_t)c.inst * K + k;
+  if (c.l == 0) {
+    if (o.t) o.t[row] = t;
+    if (o.output_scale && c.a->cfg.solver == PDQ_SOLVER_DYNAMIC) o.output_scale[row] = os;
+    if (o.num_steps && k > 0) o.num_steps[(size_t)c.inst * (K - 1) + k - 1] = (int64_t)nsteps;
+  }
+  if constexpr (!SH::smoother) {
+    w_write_normal(c, m, L, o.mean ? o.mean + row * SH::ms : nullptr, o.chol ? o.chol + row * SH::nn : nullptr);
+  } else {
+    w_write_normal(c, m, L, o.filt_mean ? o.filt_mean + row * SH::ms : nullptr,
+                   o.filt_chol ? o.filt_chol + row * SH::nn : nullptr);
+    if (k == 0 || !C) return;
+    const size_t idx = (size_t)c.inst * (K - 1) + k - 1;
+#pragma unroll
+    for (int e0 = 0; e0 < SH::nn; e0 += 64) {
+      const int e = e0 + c.l;
+      if (e < SH::nn) {
+        o.cond_A[idx * SH::nn + e] = ident ? (e / SH::nc == e % SH::nc ? 1.0 : 0.0) : C[SH::cA + e];
+        o.cond_chol[idx * SH::nn + e] = ident ? 0.0 : C[SH::cL + e];
+      }
+    }
+    if (c.l < SH::ms) o.cond_mean[idx * SH::ms + c.l] = ident ? 0.0 : C[SH::cm + c.l];
+    if (c.l < SH::nc) {
+      o.cond_tl[idx * SH::nc + c.l] = ident ? 1.0 : C[SH::ctl + c.l];
+      o.cond_to[idx * SH::nc + c.l] = ident ? 1.0 : C[SH::cto + c.l];
+    }
+  }
+}
+
+// userfriendly_output + strategy.finalize (solvers.py:439-480, 601-633,
+// 735-767; estimators_and_losses.py:380-391, 437-470).
+template <class SH>
+__device__ __forceinline__ void w_finalize(const WCtx<SH>& c, int sf, const WScal& S) {
+  const pdq_config& cfg = c.a->cfg;
+  const pdq_solution& o = c.a->out;
+  constexpr int cs = SH::nn, ms = SH::ms;
+  const int K = c.a->K, Km1 = K - 1, inst = c.inst;
+  __threadfence_block();
+  wave_sync();
+  double scale = 1.0;
+  const bool mle = cfg.solver == PDQ_SOLVER_MLE;
+  if (mle) {
+    scale = S.mle_run;
+    if (cfg.correct_asymptotic_underconfidence) {
+      const double ns = (double)o.num_steps[(size_t)inst * Km1 + Km1 - 1];
+      scale = scale / sqrt(ns);
+    }
+    if (o.output_scale && c.l == 0)
+      for (int k = 0; k < Km1; ++k) o.output_scale[(size_t)inst * K + k] = scale;
+  } else if (cfg.solver == PDQ_SOLVER && o.output_scale && c.l == 0) {
+    for (int k = 0; k < Km1; ++k) o.output_scale[(size_t)inst * K + k] = 1.0;
+  }
+  if constexpr (!SH::smoother) {
+    if (mle && o.chol)
+      for (int e = c.l; e < K * cs; e += 64)
+        o.chol[(size_t)inst * K * cs + e] = scale * o.chol[(size_t)inst * K * cs + e];
+  } else {
+    double* const X = c.slot(sf);
+    if (mle) {
+      for (int e = c.l; e < K * cs; e += 64)
+        o.filt_chol[(size_t)inst * K * cs + e] = scale * o.filt_chol[(size_t)inst * K * cs + e];
+      for (int e = c.l; e < Km1 * cs; e += 64)
+        o.cond_chol[(size_t)inst * Km1 * cs + e] = scale * o.cond_chol[(size_t)inst * Km1 * cs + e];
+      for (int e = c.l; e < cs; e += 64) {
+        X[SH::sL + e] = scale * X[SH::sL + e];
+        X[SH::sC + SH::cL + e] = scale * X[SH::sC + SH::cL + e];
+      }
+      __threadfence_block();
+      wave_sync();
+    }
+    // rv_at_t1 = posterior1.conditional.marginalise(posterior1.marginal), then
+    // the backward pass x_j = cond_j.marginalise(x_{j+1}), j = K-2 .. 0; the
+    // marginal stays in the terminal slot (j = K - 1: the terminal one itself)
+    double* const C = c.lds + SH::oB;
+    for (int j = Km1; j >= 0; --j) {
+      const bool term = j == Km1;
+      if (!term) {
+        const size_t idx = (size_t)inst * Km1 + j;
+        wave_copy<cs>(c.l, C + SH::cA, o.cond_A + idx * cs);
+        wave_copy<cs>(c.l, C + SH::cL, o.cond_chol + idx * cs);
+        wave_copy<ms>(c.l, C + SH::cm, o.cond_mean + idx * ms);
+        wave_copy<SH::nc>(c.l, C + SH::ctl, o.cond_tl + idx * SH::nc);
+        wave_copy<SH::nc>(c.l, C + SH::cto, o.cond_to + idx * SH::nc);
+        wave_sync();
+      }
+      if (!(term && S.ident))
+        w_marginalise_cond(c, term ? X + SH::sC : C, X + SH::sm, X + SH::sL, X + SH::sm, X + SH::sL);
+      const size_t row = (size_t)inst * K + j;
+      if (term)
+        w_write_normal(c, X + SH::sm, X + SH::sL, o.term_mean ? o.term_mean + (size_t)inst * ms : nullptr,
+                       o.term_chol ? o.term_chol + (size_t)inst * cs : nullptr);
+      w_write_normal(c, X + SH::sm, X + SH::sL, o.mean ? o.mean + row * ms : nullptr,
+                     o.chol ? o.chol + row * cs : nullptr);
+      wave_sync();
+    }
+  }
+}
+
+// ---------------------------------------------------------------- the solve
+enum { WOP_STEP = 0, WOP_BEYOND1 = 1, WOP_BEYOND2 = 2, WOP_AT = 3 };
+
+// One instance: the save_at loop of solvers_via_adaptive_steps.py:46-375 (or
+// the fixed grid, :11-34 of solvers_via_fixed_steps.py) with
+// solver_dynamic.step (solvers.py:549-599), solver.step (:702-733) or
+// solver_mle.step (:395-437), and interpolate_fwd (:205-315).
+template <class SH>
+__device__ __forceinline__ void w_solve_instance(const WCtx<SH>& c) {
+  constexpr int n = SH::nc;
+  const pdq_config& cfg = c.a->cfg;
+  const int K = c.a->K, inst = c.inst, l = c.l;
+  const double* ts = c.a->times + (size_t)inst * K;
+  const bool grid = c.a->mode == MODE_FIXED_GRID;
+  const bool dynamic = cfg.solver == PDQ_SOLVER_DYNAMIC, mle = cfg.solver == PDQ_SOLVER_MLE;
+  const bool fp = SH::smoother && cfg.strategy == PDQ_FIXEDPOINT;
+  const int nord = cfg.error_per_unit_step ? 2 : 1;
+  double* const Um = c.lds + SH::oUm;
+  double* const Pm = c.lds + SH::oPm;
+  double* const PL = c.lds + SH::oPL;
+  double* const B = c.lds + SH::oB;
+  double* const E = c.lds + SH::oE;
+  for (int i = l; i < cfg.n_params; i += 64) c.lds[SH::oPrm + i] = c.a->params[(size_t)inst * cfg.n_params + i];
+  // prior init: mean = tcoeffs, chol = init_std * I (from_mean_and_std)
+  int sf = 0, ifr = 1, pr = 2;
+  {
+    double* const S = c.slot(sf);
+    const double* tc = c.a->tcoeffs + (size_t)inst * SH::N * SH::d;
+    wave_copy<SH::N * SH::d>(l, S + SH::sm, tc);
+#pragma unroll
+    for (int e0 = 0; e0 < SH::ssize - SH::sL; e0 += 64) {
+      const int e = e0 + l;
+      if (e < SH::ssize - SH::sL) {
+        const bool diag = e < SH::nn && e / n == e % n;
+        S[SH::sL + e] = diag ? (cfg.init_std_rows ? cfg.init_std_rows[e / n] : cfg.init_std) : 0.0;
+      }
+    }
+    wave_sync();
+    wave_copy<SH::ssize>(l, c.slot(ifr), S);
+    wave_sync();
+  }
+  WScal F{}, S{}, R{};
+  S.t = wave_bcast(ts[0], 0);
+  S.os = 1.0;
+  S.ident = SH::smoother;
+  F = S;
+  w_write_checkpoint(c, 0, S.t, c.slot(sf) + SH::sm, c.slot(sf) + SH::sL, 1.0, 0.0, nullptr, false);
+  long attempts = 0, accepted = 0;
+  int status = PDQ_STATUS_OK, att = 0, k = 1;
+  bool second = false;
+  double dt = cfg.dt0_per_instance ? wave_bcast(cfg.dt0_per_instance[inst], 0) : cfg.dt0, cstate = 1.0;
+  while (k < K && status == PDQ_STATUS_OK) {
+    const double t1 = wave_bcast(ts[k], 0);
+    int op;
+    if (grid) op = WOP_STEP;
+    else if (second) op = WOP_BEYOND2;
+    else if (S.t + cfg.eps < t1) op = WOP_STEP;
+    else op = S.t > t1 + cfg.eps ? WOP_BEYOND1 : WOP_AT;
+    if (op == WOP_AT) {
+      // interpolate_fwd_at_t1 (solvers.py:271-315)
+      const double* const X = c.slot(sf);
+      w_write_checkpoint(c, k, S.t, X + SH::sm, X + SH::sL, S.os, S.nsteps, X + SH::sC, S.ident);
+      wave_copy<SH::ssize>(l, c.slot(ifr), X);
+      wave_sync();
+      if (fp) S.ident = true;
+      F = S;
+      ++k;
+      continue;
+    }
+    double h;
+    if (op == WOP_STEP) {
+      h = grid ? t1 - wave_bcast(ts[k - 1], 0) : dt;
+      if (!grid && cfg.clip_dt) h = fmin(h, t1 - S.t);
+    } else {
+      h = op == WOP_BEYOND1 ? t1 - F.t : S.t - t1;
+    }
+    const double tn = S.t + h;
+    const double dtn = w_precon(c, h, nord);
+    // the state that is predicted: step_from, interp_from, or the interpolated marginal
+    const double* const Xs = op == WOP_STEP ? c.slot(sf) : c.slot(ifr);
+    const double *const Xm = Xs + SH::sm, *const XL = Xs + SH::sL;
+    WLin<SH> lin;
+    WErr err;
+    double scale = S.os;
+    if (op == WOP_STEP) {
+      scale = 1.0;
+      if (dynamic) {
+        w_apply_flat_mean(c, Xm, Um);
+        w_linearize(c, Um, tn, lin);
+        w_calibrate(c, lin, Um, w_noise_scale(c, h, 1.0), err);
+        scale = wave_bcast(err.sigma, 0);
+      }
+    }
+    const double s = w_noise_scale(c, h, scale);
+    if constexpr (!SH::smoother) {
+      w_marginalise_prior(c, s, Xm, XL, Pm, PL);
+    } else {
+      // the prediction into (Pm, PL) and the conditional into B; in front of it
+      // the fixed-point smoother merges the state's own conditional
+      w_revert_prior(c, s, Xm, XL, Pm, PL, B, c.lds + SH::oTmp);
+      double* const dst = op == WOP_STEP ? c.slot(pr) + SH::sC : (op == WOP_BEYOND1 ? E : c.slot(sf) + SH::sC);
+      if (fp) {
+        w_merge(c, op == WOP_BEYOND2 || (op == WOP_STEP ? S.ident : F.ident),
+                (op == WOP_BEYOND1 ? c.slot(ifr) : c.slot(sf)) + SH::sC, B, dst);
+      } else {
+        wave_copy<SH::csize>(l, dst, B);
+        wave_sync();
+      }
+    }
+    if (op == WOP_STEP) {
+      double* const Y = c.slot(pr);
+      double om[SH::ko * SH::mc], oL[SH::ko * SH::ko];
+      if (!dynamic) w_linearize(c, Pm, tn, lin);
+      w_update(c, lin, Pm, PL, Y + SH::sm, Y + SH::sL, om, oL);
+      R = S;
+      R.t = tn;
+      R.os = dynamic ? scale : (mle ? S.os : 1.0);
+      R.nsteps = S.nsteps + 1.0;
+      R.ident = false;
+      R.mle_run = R.mle_n = 0.0;
+      if (mle) {
+        // bayes_rule_and_residual_whitened_rms_tree: observed = (mo, R_Y^T)
+        const double nt = w_rms_zero<SH>(om, oL);
+        const double nd = S.mle_n;
+        const double x1 = sqrt(nd / (nd + 1)) * S.mle_run;
+        const double x2 = sqrt(1 / (nd + 1)) * nt;
+        R.mle_run = wave_bcast(hypot(x1, x2), 0);
+        R.mle_n = nd + 1;
+      }
+      ++attempts;
+      if (grid) {
+        ++accepted;
+        w_write_checkpoint(c, k, tn, Y + SH::sm, Y + SH::sL, R.os, R.nsteps, Y + SH::sC, false);
+        wave_sync();
+        const int tmp = sf;
+        sf = pr;
+        pr = tmp;
+        S = R;
+        ++k;
+        continue;
+      }
+      if (!dynamic) {
+        w_apply_flat_mean(c, Xm, Um);
+        w_calibrate(c, lin, Um, w_noise_scale(c, h, 1.0), err);
+      }
+      const double ep = wave_bcast(w_error_power(c, err, Xm, Y + SH::sm, dtn, nord), 0);
+      dt = wave_bcast(w_control(cfg, h, cstate, ep), 0);
+      ++att;
+      if (!isfinite(ep) || !isfinite(dt)) {
+        status = PDQ_STATUS_NONFINITE;
+      } else if (ep < 1.0 && (dt == 0.0 || S.t + dt == S.t)) {
+        status = PDQ_STATUS_DT_UNDERFLOW;
+      } else if (ep >= 1.0 && R.t == S.t) {
+        status = PDQ_STATUS_DT_UNDERFLOW;  // accepted without advancing t
+      } else if ((cfg.max_attempts > 0 && att >= cfg.max_attempts && ep < 1.0) || attempts >= kMaxTotalAttempts) {
+        status = PDQ_STATUS_MAX_ATTEMPTS;
+      } else if (ep >= 1.0) {
+        ++accepted;
+        att = 0;
+        // interp_from <- step_from, step_from <- proposed
+        const int old = ifr;
+        ifr = sf;
+        sf = pr;
+        pr = old;
+        F = S;
+        S = R;
+      }
+    } else if (op == WOP_BEYOND1) {
+      // interpolate_fwd (solvers.py:205-269): the marginal at t1 is the new
+      // interp_from's, E the conditional that leads to it
+      double* const X = c.slot(ifr);
+      w_write_checkpoint(c, k, t1, Pm, PL, S.os, S.nsteps, SH::smoother ? E : nullptr, false);
+      wave_copy<SH::ms>(l, X + SH::sm, Pm);
+      wave_copy<SH::nn>(l, X + SH::sL, PL);
+      if (SH::smoother && !fp) wave_copy<SH::csize>(l, X + SH::sC, E);
+      wave_sync();
+      F.t = t1;
+      if (SH::smoother) {
+        F.ident = fp;
+        second = true;
+      } else {
+        ++k;
+      }
+    } else {
+      S.ident = false;
+      second = false;
+      ++k;
+    }
+  }
+  if (status == PDQ_STATUS_OK) w_finalize(c, sf, S);
+  const pdq_solution& o = c.a->out;
+  if (l == 0) {
+    if (o.attempts) o.attempts[inst] = attempts;
+    if (o.accepted) o.accepted[inst] = accepted;
+    if (o.status) o.status[inst] = status;
+  }
+}
+
+// The transition into LDS; lanes of one wavefront.
+template <class SH>
+__device__ __forceinline__ void w_setup(const KArgs& a, double* lds, int l) {
+  wave_copy<SH::nn>(l, lds + SH::oA, a.A);
+  wave_copy<SH::nn>(l, lds + SH::oQ, a.Q);
+  wave_sync();
+}
+
+}  // namespace pdq

@@ -65,6 +65,21 @@ __device__ __forceinline__ double lane_div_nz(double a, double b, double y) {
   return fma(fma(-q, b, a), y, q);
 }
 
+// a / b given y = 1 / b (correctly rounded): q = a y, then one FMA
+// correction step against the exact residual a - b q (Markstein).  For a
+// correctly rounded, normal y and a finite quotient the result is the
+// correctly rounded quotient, as a division gives it, for three instructions
+// once y is known; used where many quotients share one divisor.  Any other
+// case (b = 0, infinities, NaN, y outside the normal range) takes the
+// division itself, so special values behave exactly as IEEE division.
+__device__ __forceinline__ double lane_div(double a, double b, double y) {
+  const double q = a * y;
+  const double r = fma(-q, b, a);
+  const double res = r == 0.0 ? q : fma(r, y, q);  // exact q keeps the sign of a zero quotient
+  if (__builtin_expect(!(__builtin_isnormal(y) && isfinite(res)), 0)) return a / b;
+  return res;
+}
+
 // The inverse N-th root, from a hardware estimate refined by FMA iterations.
 // * lane_root_inv<N>: x^(-1/N) from a single-precision estimate of the
 //   scaled operand (x = xs 2^(N k), xs within single range), then two Newton
@@ -402,17 +417,40 @@ __device__ __forceinline__ double factorial_d(int k) {
 }
 
 // ------------------------------------------------------------- lane groups
+#ifdef PDQ_HOST_EMU
+}  // namespace pdq
+// The CPU build runs a group of more than one lane as threads (tests/emu):
+// these hooks are the harness's barrier and lane exchange.
+void pdq_emu_group_barrier();
+double pdq_emu_shfl_xor(double v, int mask, int width);
+double pdq_emu_shfl(double v, int src, int width);
+namespace pdq {
+#endif
 template <int G>
 struct Grp {
   int l;  // lane index inside the group
   // Orders LDS accesses of the group's lanes (they share one wavefront).
   __device__ __forceinline__ void sync() const {
     if constexpr (G > 1) {
+#ifdef PDQ_HOST_EMU
+      pdq_emu_group_barrier();
+#else
       __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
       __builtin_amdgcn_wave_barrier();
       __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+#endif
     }
   }
+#ifdef PDQ_HOST_EMU
+  double sum(double v) const {
+    for (int m = G / 2; m >= 1; m >>= 1) v += pdq_emu_shfl_xor(v, m, G);
+    return G > 1 ? pdq_emu_shfl(v, 0, G) : v;
+  }
+  double max(double v) const {
+    for (int m = G / 2; m >= 1; m >>= 1) v = fmax(v, pdq_emu_shfl_xor(v, m, G));
+    return v;
+  }
+#else
   // Group sum.  A butterfly leaves each lane with the total in its own
   // association order (lane-dependent rounding), so lane 0's total is
   // broadcast: every lane must take the same accept/reject decisions and
@@ -429,6 +467,7 @@ struct Grp {
     for (int m = G / 2; m >= 1; m >>= 1) v = fmax(v, __shfl_xor(v, m, G));
     return v;
   }
+#endif
   __device__ __forceinline__ int bcast(int v) const {
     if constexpr (G > 1) return __shfl(v, 0, G);
     return v;

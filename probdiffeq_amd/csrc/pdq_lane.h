@@ -37,21 +37,6 @@ namespace pdq {
 #endif
 
 
-// a / b given y = 1 / b (correctly rounded): q = a y, then one FMA
-// correction step against the exact residual a - b q (Markstein).  For a
-// correctly rounded, normal y and a finite quotient the result is the
-// correctly rounded quotient, as a division gives it, for three instructions
-// once y is known; used where many quotients share one divisor.  Any other
-// case (b = 0, infinities, NaN, y outside the normal range) takes the
-// division itself, so special values behave exactly as IEEE division.
-__device__ __forceinline__ double lane_div(double a, double b, double y) {
-  const double q = a * y;
-  const double r = fma(-q, b, a);
-  const double res = r == 0.0 ? q : fma(r, y, q);  // exact q keeps the sign of a zero quotient
-  if (__builtin_expect(!(__builtin_isnormal(y) && isfinite(res)), 0)) return a / b;
-  return res;
-}
-
 // Slot scalars.
 enum { LS_T = 0, LS_OS = 1, LS_NSTEPS = 2, LS_MLE_RUN = 3, LS_MLE_N = 4, LS_IDENT = 5, LS_NSC = 8 };
 

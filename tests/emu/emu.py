@@ -40,8 +40,9 @@ def lib():
 def solve(cfg, params, tcoeffs, times, fixed_grid=False, kernel="coop"):
     """cfg: probdiffeq_amd.capi.Config; numpy inputs; returns numpy outputs.
 
-    kernel: "coop" (the cooperative kernel's code) or "lane" (the
-    lane-per-instance isotropic kernel's code)."""
+    kernel: "coop" (the cooperative kernel's code), "lane" (the
+    lane-per-instance isotropic kernel's code) or "wave" (the fixed-shape
+    cooperative kernel's, 64 threads per instance)."""
     from probdiffeq_amd import capi
 
     params = np.ascontiguousarray(params, dtype=np.float64)
@@ -77,7 +78,7 @@ def solve(cfg, params, tcoeffs, times, fixed_grid=False, kernel="coop"):
         setattr(s, name, a.ctypes.data if a is not None else None)
     c = cfg.c(host=True)
     P = ctypes.c_void_p
-    fn = lib().pdqemu_solve_lane if kernel == "lane" else lib().pdqemu_solve
+    fn = {"lane": lib().pdqemu_solve_lane, "wave": lib().pdqemu_solve_wave, "coop": lib().pdqemu_solve}[kernel]
     rc = fn(ctypes.byref(c), B, P(params.ctypes.data), P(tcoeffs.ctypes.data), P(times.ctypes.data), K, ctypes.byref(s), int(fixed_grid))
     if rc:
         raise RuntimeError(f"emulation rc {rc}")

@@ -10,6 +10,7 @@
 
 #include "../../probdiffeq_amd/csrc/pdq_bd.h"
 #include "../../probdiffeq_amd/csrc/pdq_coop.hip"
+#include "../../probdiffeq_amd/csrc/pdq_coop_wave.h"
 #include "../../probdiffeq_amd/csrc/pdq_iwp.h"
 #include "../../probdiffeq_amd/csrc/pdq_lane.h"
 #include "../../probdiffeq_amd/csrc/pdq_lane_adjoint.h"
@@ -293,6 +294,73 @@ int pdqemu_solve(const pdq_config* cfg, int n_inst, const double* params, const 
   return 0;
 }
 
+}  // extern "C"
+
+// The fixed-shape cooperative kernel on the CPU: one instance's 64 lanes as 64
+// threads with real barriers and lane exchanges.
+namespace {
+template <class SH>
+void wave_emu_instance(const pdq::KArgs& a, int inst) {
+  std::vector<double> lds(SH::fixed_size + a.cfg.n_params, 0.0);
+  std::barrier<> bar(64);
+  g_group_barrier = &bar;
+  std::vector<std::thread> th;
+  th.reserve(64);
+  for (int l = 0; l < 64; ++l)
+    th.emplace_back([&, l] {
+      t_group_lane = l;
+      pdq::WCtx<SH> c;
+      c.a = &a;
+      c.lds = lds.data();
+      c.l = l;
+      c.inst = inst;
+      pdq::w_setup<SH>(a, lds.data(), l);
+      pdq::w_solve_instance(c);
+    });
+  for (auto& t : th) t.join();
+  g_group_barrier = nullptr;
+}
+
+template <int N, bool DENSE>
+void wave_emu(const pdq::KArgs& a, int inst) {
+  if (a.cfg.strategy == PDQ_FILTER) wave_emu_instance<pdq::WShape<N, 2, DENSE, false>>(a, inst);
+  else wave_emu_instance<pdq::WShape<N, 2, DENSE, true>>(a, inst);
+}
+}  // namespace
+
+extern "C" {
+// mode: 0 save_at, 1 fixed grid.  Dense nu = 2..5 or isotropic nu = 2, 5, d = 2.
+int pdqemu_solve_wave(const pdq_config* cfg, int n_inst, const double* params, const double* tcoeffs,
+                      const double* times, int K, const pdq_solution* out, int mode) {
+  if (cfg->ode_dim != 2) return 2;
+  std::vector<double> A, Q;
+  const bool dense = cfg->factorisation == PDQ_DENSE;
+  if (dense) pdq::iwp_dense(cfg->num_derivatives, cfg->ode_dim, cfg->base_output_scale, A, Q);
+  else pdq::iwp_matrices(cfg->num_derivatives, A, Q);
+  pdq::KArgs a{};
+  a.cfg = *cfg;
+  a.lay = pdq::make_layout(*cfg, 0);
+  a.n_inst = n_inst;
+  a.K = K;
+  a.mode = mode;
+  a.params = params;
+  a.tcoeffs = tcoeffs;
+  a.times = times;
+  a.A = A.data();
+  a.Q = Q.data();
+  a.out = *out;
+  for (int i = 0; i < n_inst; ++i) {
+    const int N = cfg->num_derivatives + 1;
+    if (dense && N == 3) wave_emu<3, true>(a, i);
+    else if (dense && N == 4) wave_emu<4, true>(a, i);
+    else if (dense && N == 5) wave_emu<5, true>(a, i);
+    else if (dense && N == 6) wave_emu<6, true>(a, i);
+    else if (!dense && N == 3) wave_emu<3, false>(a, i);
+    else if (!dense && N == 6) wave_emu<6, false>(a, i);
+    else return 2;
+  }
+  return 0;
+}
 
 // LML value and forward-mode gradient (MODE_LML) on the CPU.
 }  // extern "C"
