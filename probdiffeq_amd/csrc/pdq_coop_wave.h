@@ -18,8 +18,14 @@
 // * the solve's scalars (t, dt, output scale, counts) are wave-uniform
 //   registers, and every loop and branch on them is a scalar one.
 // Measured on one MI355X, the same outputs bit for bit: 1024 dense
-// Lotka-Volterra solves (nu = 4, filter, 200 points) 71.3 -> 14.3 ms, one such
-// solve 32.3 -> 5.7 ms, 1024 stiff van der Pol solves (nu = 5, ts1) 20.9 -> 3.2 ms.
+// Lotka-Volterra solves (nu = 4, filter, 200 points) 71.3 -> 10.6 ms, one such
+// solve 32.3 -> 5.6 ms, 1024 stiff van der Pol solves (nu = 5, ts1) 20.9 -> 3.1 ms.
+// Of the 14.3 ms of a first version, 3.7 went with the solve's scalars in
+// vector registers under scalar branches (spilled scalar registers before), no
+// padding in the structs that are copied (padded copies went through scratch
+// memory), the reflectors broadcast by one DPP move per value where the columns
+// fit a row of 16 lanes (two v_readlane before), the next point's time loaded a
+// point ahead, and the outputs' addresses loaded in one batch.
 // Configurations it does not hold (error_state_std, re-linearisation, Monte
 // Carlo Jacobians, the LML) stay with the run-time-shape kernel.
 #pragma once
@@ -56,25 +62,25 @@ struct WShape {
 // The stacks' patterns (WaveQrPlan).
 template <class SH>
 struct WPatStack {  // [dense; upper triangle]
-  static constexpr int nc = SH::nc, M = 2 * nc, NP = nc, MROWS = M;
+  static constexpr int nc = SH::nc, M = 2 * nc, NP = nc, MROWS = M, COLS = nc;
   static constexpr int row(int r) { return r; }
   static constexpr bool nz(int r, int c) { return r < nc || r - nc <= c; }
 };
 template <class SH>
 struct WPatRevert {  // [[upper triangle, 0], [dense, upper triangle]]
-  static constexpr int nc = SH::nc, M = 2 * nc, NP = M, MROWS = M;
+  static constexpr int nc = SH::nc, M = 2 * nc, NP = M, MROWS = M, COLS = M;
   static constexpr int row(int r) { return r; }
   static constexpr bool nz(int r, int c) { return c < nc ? (r >= nc || r <= c) : (r >= nc && r - nc <= c - nc); }
 };
 template <class SH>
 struct WPatUpdate {  // [[diagonal, 0], [(H L)^T, L^T]]: H reads derivatives 0 and 1, the first 2 ko rows of L
-  static constexpr int nc = SH::nc, ko = SH::ko, M = ko + nc, NP = M, MROWS = M;
+  static constexpr int nc = SH::nc, ko = SH::ko, M = ko + nc, NP = M, MROWS = M, COLS = M;
   static constexpr int row(int r) { return r; }
   static constexpr bool nz(int r, int c) { return r < ko ? r == c : (c < ko ? r - ko < 2 * ko : r - ko <= c - ko); }
 };
 template <class SH>
 struct WPatFx {  // [(H L)^T; diagonal], without (H L)^T's zero rows
-  static constexpr int nc = SH::nc, ko = SH::ko, M = 3 * ko, NP = ko, MROWS = nc + ko;
+  static constexpr int nc = SH::nc, ko = SH::ko, M = 3 * ko, NP = ko, MROWS = nc + ko, COLS = ko;
   static constexpr int row(int r) { return r < 2 * ko ? r : nc + r - 2 * ko; }
   static constexpr bool nz(int r, int c) { return r < 2 * ko || r - 2 * ko == c; }
 };
@@ -91,10 +97,11 @@ __device__ __forceinline__ void wave_copy(int l, double* dst, const double* src)
   }
 }
 
-// A solution's scalars.
+// A solution's scalars (the same in every lane).  No padding: copies of a
+// padded struct go through scratch memory.
 struct WScal {
-  double t, os, nsteps, mle_run, mle_n;
-  bool ident;
+  double t, os, mle_run, mle_n;
+  int nsteps, ident;
 };
 
 // The linearisation: the operator's non-zero block J (ko x 2 ko, derivatives 0
@@ -110,18 +117,48 @@ struct WErr {
   double sigma;
 };
 
+// The launch's arguments, in the kernel argument segment.  The solve reads them
+// through a pointer that it renews in every iteration (WCtx::renew): what an
+// iteration needs is then loaded in it (scalar loads, cached) instead of ahead
+// of the loop, where it would take scalar registers throughout and be spilled.
+#ifdef PDQ_HOST_EMU
+using WArgs = const KArgs;
+#else
+using WArgs = const __attribute__((address_space(4))) KArgs;
+#endif
+
+// The configuration an attempt reads, in scalar registers for the whole solve.
+struct WCfg {
+  double rtol, atol, eps, damp, safety, factor_min, factor_max;
+  int ts1, vector_field, error_norm, integral, clip_dt, max_attempts;
+  template <class Cfg>
+  __device__ __forceinline__ explicit WCfg(const Cfg& c)
+      : rtol(c.rtol), atol(c.atol), eps(c.eps), damp(c.damp), safety(c.safety), factor_min(c.factor_min),
+        factor_max(c.factor_max), ts1(c.constraint == PDQ_TS1), vector_field(c.vector_field),
+        error_norm(c.error_norm), integral(c.control == PDQ_CONTROL_INTEGRAL), clip_dt(c.clip_dt),
+        max_attempts(c.max_attempts) {}
+};
+
 template <class SH>
 struct WCtx {
-  const KArgs* a;
+  WArgs* a;
+  WCfg cfg;
   double* lds;
-  int l, inst;
+  int l, inst, K;
+  bool dynamic;  // solver_dynamic
   __device__ __forceinline__ double* P() const { return lds + SH::oP; }
   __device__ __forceinline__ double* PI() const { return lds + SH::oPI; }
   __device__ __forceinline__ const double* A() const { return lds + SH::oA; }
   __device__ __forceinline__ const double* Q() const { return lds + SH::oQ; }
   __device__ __forceinline__ const double* prm() const { return lds + SH::oPrm; }
   __device__ __forceinline__ double* slot(int s) const { return lds + SH::oS + s * SH::ssize; }
-  __device__ __forceinline__ bool ts1() const { return a->cfg.constraint == PDQ_TS1; }
+  __device__ __forceinline__ WCtx(WArgs* args, double* lds_, int lane) : a(args), cfg(args->cfg), lds(lds_), l(lane), inst(0), K(args->K), dynamic(args->cfg.solver == PDQ_SOLVER_DYNAMIC) {}
+  __device__ __forceinline__ bool ts1() const { return cfg.ts1 != 0; }
+  __device__ __forceinline__ void renew() {
+#ifndef PDQ_HOST_EMU
+    asm("" : "+s"(a));
+#endif
+  }
 };
 
 // preconditioner_taylor (utilities.py:74-84) into P and PI, and dt^nord (in
@@ -201,7 +238,7 @@ __device__ __forceinline__ void w_apply_flat_mean(const WCtx<SH>& c, const doubl
 template <class SH>
 __device__ __forceinline__ void w_linearize(const WCtx<SH>& c, const double* Xm, double t, WLin<SH>& lin) {
   constexpr int d = SH::d, ko = SH::ko, K2 = 2 * SH::ko;
-  const int id = c.a->cfg.vector_field;
+  const int id = c.cfg.vector_field;
   double y[d];
 #pragma unroll
   for (int j = 0; j < d; ++j) y[j] = Xm[j];
@@ -290,7 +327,7 @@ __device__ __forceinline__ double w_rms_zero(const double* om, const double* oL)
   }
   double tot = sum[0];
   if constexpr (m == 2) tot = wave_add(sum[0], sum[1]);
-  return sqrt(tot) / sqrt((double)(k * m));
+  return wave_div_root<k * m>(sqrt(tot));
 }
 
 // The error model's observed marginal at the extrapolation Um with output
@@ -300,7 +337,7 @@ __device__ __forceinline__ void w_calibrate(const WCtx<SH>& c, const WLin<SH>& l
                                             WErr& err) {
   constexpr int k = SH::ko, m = SH::mc;
   const int o = c.l < k ? c.l : k - 1;
-  const double damp = c.a->cfg.damp;
+  const double damp = c.cfg.damp;
   double a[3 * k], om[k * m];
 #pragma unroll
   for (int r = 0; r < 2 * k; ++r)
@@ -338,8 +375,9 @@ __device__ __forceinline__ void w_marginalise_prior(const WCtx<SH>& c, double s,
   if (c.l < n) {
 #pragma unroll
     for (int col = 0; col < m; ++col) Ym[i * m + col] = p * (acc[col] + 0.0);
+    const int here = wave_here(i);
 #pragma unroll
-    for (int j = 0; j < n; ++j) YL[i * n + j] = fabs(p) * wave_r(a, j, i);
+    for (int j = 0; j < n; ++j) YL[i * n + j] = fabs(p) * wave_r(a, j, here);
   }
   wave_sync();
 }
@@ -391,16 +429,18 @@ __device__ __forceinline__ void w_revert_prior(const WCtx<SH>& c, double s, cons
       for (int k = 0; k < n; ++k) ac += gn[k] * tmp[k * m + col];
       B[SH::cm + i * m + col] = pi * xm[col] - ac;
     }
+    const int here = wave_here(i);
 #pragma unroll
-    for (int j = 0; j < n; ++j) B[SH::cL + i * n + j] = j <= i ? a[n + j] : 0.0;
+    for (int j = 0; j < n; ++j) B[SH::cL + i * n + j] = j <= here ? a[n + j] : 0.0;
     B[SH::ctl + i] = 1.0 / p;
     B[SH::cto + i] = 1.0 / pi;
   }
   if (!right) {
 #pragma unroll
     for (int col = 0; col < m; ++col) Ym[i * m + col] = p * tmp[i * m + col];
+    const int here = wave_here(i);
 #pragma unroll
-    for (int j = 0; j < n; ++j) YL[i * n + j] = fabs(p) * wave_r(a, j, i);
+    for (int j = 0; j < n; ++j) YL[i * n + j] = fabs(p) * wave_r(a, j, here);
   }
   wave_sync();
 }
@@ -460,8 +500,9 @@ __device__ __forceinline__ void w_merge(const WCtx<SH>& c, bool ident, const dou
   if (c.l < n) {
 #pragma unroll
     for (int col = 0; col < m; ++col) R[SH::cm + i * m + col] = acc[col] + sm[i * m + col];
+    const int here = wave_here(i);
 #pragma unroll
-    for (int j = 0; j < n; ++j) R[SH::cL + i * n + j] = wave_r(a, j, i);
+    for (int j = 0; j < n; ++j) R[SH::cL + i * n + j] = wave_r(a, j, here);
     R[SH::ctl + i] = B[SH::ctl + i];
     R[SH::cto + i] = F[SH::cto + i];
   }
@@ -495,8 +536,9 @@ __device__ __forceinline__ void w_marginalise_cond(const WCtx<SH>& c, const doub
   if (c.l < n) {
 #pragma unroll
     for (int col = 0; col < m; ++col) Ym[i * m + col] = to * (acc[col] + C[SH::cm + i * m + col]);
+    const int here = wave_here(i);
 #pragma unroll
-    for (int j = 0; j < n; ++j) YL[i * n + j] = fabs(to) * wave_r(a, j, i);
+    for (int j = 0; j < n; ++j) YL[i * n + j] = fabs(to) * wave_r(a, j, here);
   }
   wave_sync();
 }
@@ -507,7 +549,7 @@ template <class SH>
 __device__ __forceinline__ void w_update(const WCtx<SH>& c, const WLin<SH>& lin, const double* Pm, const double* PL,
                                          double* Xm, double* XL, double* om, double* oL) {
   constexpr int n = SH::nc, k = SH::ko, m = SH::mc;
-  const double damp = c.a->cfg.damp;
+  const double damp = c.cfg.damp;
   // lanes 0..k-1: the observation's columns, lanes k..k+n-1: the state's (the others repeat the last)
   const bool state = c.l >= k;
   const int o = state ? k - 1 : c.l;
@@ -537,8 +579,9 @@ __device__ __forceinline__ void w_update(const WCtx<SH>& c, const WLin<SH>& lin,
       for (int r = 0; r < k; ++r) acc += gn[r] * om[r * m + col];
       Xm[i * m + col] = Pm[i * m + col] - acc;
     }
+    const int here = wave_here(i);
 #pragma unroll
-    for (int j = 0; j < n; ++j) XL[i * n + j] = j <= i ? a[k + j] : 0.0;
+    for (int j = 0; j < n; ++j) XL[i * n + j] = j <= here ? a[k + j] : 0.0;
   }
 #pragma unroll
   for (int i2 = 0; i2 < k; ++i2)
@@ -553,8 +596,7 @@ template <class SH>
 __device__ __forceinline__ double w_error_power(const WCtx<SH>& c, const WErr& err, const double* prev_m,
                                                 const double* prop_m, double dtn, int nord) {
   constexpr int k = SH::ko, d = SH::d;
-  const pdq_config& cfg = c.a->cfg;
-  const double fact = nord == 1 ? 1.0 : 2.0;
+  const WCfg& cfg = c.cfg;
   const int q = c.l < d ? c.l : d - 1;
   // std of the lane's rescaled observed row: dense per-row qr_r (|beta| of
   // dlarfg), isotropic vector_norm
@@ -576,7 +618,7 @@ __device__ __forceinline__ double w_error_power(const WCtx<SH>& c, const WErr& e
   double std;
   if (SH::dense) std = ss == 0.0 ? fabs(alpha) : fabs(hypot(alpha, sqrt(ss)));
   else std = sqrt(alpha * alpha + ss);
-  const double e = std * dtn / fact;
+  const double e = nord == 1 ? std * dtn : std * dtn * 0.5;  // / n!, exactly
   const double ref = fmax(fabs(prev_m[q]), fabs(prop_m[q]));
   double norm;
   if (cfg.error_norm == PDQ_NORM_SCALE_THEN_RMS) {
@@ -587,7 +629,7 @@ __device__ __forceinline__ double w_error_power(const WCtx<SH>& c, const WErr& e
       const double rx = wave_bcast(rr, x);
       tot = wave_add_square(tot, rx);
     }
-    norm = sqrt(tot) / sqrt((double)d);
+    norm = wave_div_root<d>(sqrt(tot));
   } else {
     double sa = 0.0, sr = 0.0;
 #pragma unroll
@@ -606,13 +648,15 @@ __device__ __forceinline__ double w_error_power(const WCtx<SH>& c, const WErr& e
 }
 
 // controllers.py:66-84 / :24-63
-__device__ __forceinline__ double w_control(const pdq_config& cfg, double dt, double& cstate, double ep) {
-  if (cfg.control == PDQ_CONTROL_INTEGRAL) {
+template <class SH>
+__device__ __forceinline__ double w_control(const WCtx<SH>& c, double dt, double& cstate, double ep) {
+  const WCfg& cfg = c.cfg;
+  if (cfg.integral) {
     const double ratio = cfg.safety * ep;
     return fmax(cfg.factor_min, fmin(ratio, cfg.factor_max)) * dt;
   }
-  const double gi = pow(ep, cfg.exponent_integral);
-  const double gp = pow(ep / cstate, cfg.exponent_proportional);
+  const double gi = pow(ep, c.a->cfg.exponent_integral);
+  const double gp = pow(ep / cstate, c.a->cfg.exponent_proportional);
   const double ratio = cfg.safety * gi * gp;
   const double sf = fmax(cfg.factor_min, fmin(ratio, cfg.factor_max));
   if (ep >= 1.0) cstate = ep;
@@ -631,21 +675,27 @@ __device__ __forceinline__ void w_write_normal(const WCtx<SH>& c, const double* 
 // and (C) the backward conditional that leads to it, an identity with `ident`.
 template <class SH>
 __device__ __forceinline__ void w_write_checkpoint(const WCtx<SH>& c, int k, double t, const double* m,
-                                                   const double* L, double os, double nsteps, const double* C,
+                                                   const double* L, double os, int nsteps, const double* C,
                                                    bool ident) {
-  const pdq_solution& o = c.a->out;
-  const int K = c.a->K;
+  const auto& o = c.a->out;
+  const int K = c.K;
   const size_t row = (size_t)c.inst * K + k;
+  // the outputs' addresses in one batch of scalar loads
+  double *gt = o.t, *gos = c.dynamic ? o.output_scale : nullptr;
+  double *gm = SH::smoother ? o.filt_mean : o.mean, *gL = SH::smoother ? o.filt_chol : o.chol;
+  int64_t* gn = o.num_steps;
+#ifndef PDQ_HOST_EMU
+  asm("" : "+s"(gt), "+s"(gos), "+s"(gm), "+s"(gL), "+s"(gn));
+#endif
   if (c.l == 0) {
-    if (o.t) o.t[row] = t;
-    if (o.output_scale && c.a->cfg.solver == PDQ_SOLVER_DYNAMIC) o.output_scale[row] = os;
-    if (o.num_steps && k > 0) o.num_steps[(size_t)c.inst * (K - 1) + k - 1] = (int64_t)nsteps;
+    if (gt) gt[row] = t;
+    if (gos) gos[row] = os;
+    if (gn && k > 0) gn[(size_t)c.inst * (K - 1) + k - 1] = nsteps;
   }
   if constexpr (!SH::smoother) {
-    w_write_normal(c, m, L, o.mean ? o.mean + row * SH::ms : nullptr, o.chol ? o.chol + row * SH::nn : nullptr);
+    w_write_normal(c, m, L, gm ? gm + row * SH::ms : nullptr, gL ? gL + row * SH::nn : nullptr);
   } else {
-    w_write_normal(c, m, L, o.filt_mean ? o.filt_mean + row * SH::ms : nullptr,
-                   o.filt_chol ? o.filt_chol + row * SH::nn : nullptr);
+    w_write_normal(c, m, L, gm ? gm + row * SH::ms : nullptr, gL ? gL + row * SH::nn : nullptr);
     if (k == 0 || !C) return;
     const size_t idx = (size_t)c.inst * (K - 1) + k - 1;
 #pragma unroll
@@ -668,8 +718,8 @@ __device__ __forceinline__ void w_write_checkpoint(const WCtx<SH>& c, int k, dou
 // 735-767; estimators_and_losses.py:380-391, 437-470).
 template <class SH>
 __device__ __forceinline__ void w_finalize(const WCtx<SH>& c, int sf, const WScal& S) {
-  const pdq_config& cfg = c.a->cfg;
-  const pdq_solution& o = c.a->out;
+  const auto& cfg = c.a->cfg;
+  const auto& o = c.a->out;
   constexpr int cs = SH::nn, ms = SH::ms;
   const int K = c.a->K, Km1 = K - 1, inst = c.inst;
   __threadfence_block();
@@ -741,21 +791,20 @@ enum { WOP_STEP = 0, WOP_BEYOND1 = 1, WOP_BEYOND2 = 2, WOP_AT = 3 };
 // solver_dynamic.step (solvers.py:549-599), solver.step (:702-733) or
 // solver_mle.step (:395-437), and interpolate_fwd (:205-315).
 template <class SH>
-__device__ __forceinline__ void w_solve_instance(const WCtx<SH>& c) {
+__device__ __forceinline__ void w_solve_instance(WCtx<SH> c) {
   constexpr int n = SH::nc;
-  const pdq_config& cfg = c.a->cfg;
-  const int K = c.a->K, inst = c.inst, l = c.l;
+  const int K = c.K, inst = c.inst, l = c.l;
   const double* ts = c.a->times + (size_t)inst * K;
   const bool grid = c.a->mode == MODE_FIXED_GRID;
-  const bool dynamic = cfg.solver == PDQ_SOLVER_DYNAMIC, mle = cfg.solver == PDQ_SOLVER_MLE;
-  const bool fp = SH::smoother && cfg.strategy == PDQ_FIXEDPOINT;
-  const int nord = cfg.error_per_unit_step ? 2 : 1;
+  const bool dynamic = c.dynamic, mle = c.a->cfg.solver == PDQ_SOLVER_MLE;
+  const bool fp = SH::smoother && c.a->cfg.strategy == PDQ_FIXEDPOINT;
+  const int nord = c.a->cfg.error_per_unit_step ? 2 : 1;
   double* const Um = c.lds + SH::oUm;
   double* const Pm = c.lds + SH::oPm;
   double* const PL = c.lds + SH::oPL;
   double* const B = c.lds + SH::oB;
   double* const E = c.lds + SH::oE;
-  for (int i = l; i < cfg.n_params; i += 64) c.lds[SH::oPrm + i] = c.a->params[(size_t)inst * cfg.n_params + i];
+  for (int i = l; i < c.a->cfg.n_params; i += 64) c.lds[SH::oPrm + i] = c.a->params[(size_t)inst * c.a->cfg.n_params + i];
   // prior init: mean = tcoeffs, chol = init_std * I (from_mean_and_std)
   int sf = 0, ifr = 1, pr = 2;
   {
@@ -767,7 +816,7 @@ __device__ __forceinline__ void w_solve_instance(const WCtx<SH>& c) {
       const int e = e0 + l;
       if (e < SH::ssize - SH::sL) {
         const bool diag = e < SH::nn && e / n == e % n;
-        S[SH::sL + e] = diag ? (cfg.init_std_rows ? cfg.init_std_rows[e / n] : cfg.init_std) : 0.0;
+        S[SH::sL + e] = diag ? (c.a->cfg.init_std_rows ? c.a->cfg.init_std_rows[e / n] : c.a->cfg.init_std) : 0.0;
       }
     }
     wave_sync();
@@ -775,22 +824,31 @@ __device__ __forceinline__ void w_solve_instance(const WCtx<SH>& c) {
     wave_sync();
   }
   WScal F{}, S{}, R{};
-  S.t = wave_bcast(ts[0], 0);
-  S.os = 1.0;
+  S.t = wave_rounded(ts[0]);
+  S.os = wave_rounded(1.0);
   S.ident = SH::smoother;
   F = S;
-  w_write_checkpoint(c, 0, S.t, c.slot(sf) + SH::sm, c.slot(sf) + SH::sL, 1.0, 0.0, nullptr, false);
-  long attempts = 0, accepted = 0;
+  w_write_checkpoint(c, 0, S.t, c.slot(sf) + SH::sm, c.slot(sf) + SH::sL, 1.0, 0, nullptr, false);
+  int attempts = 0, accepted = 0;
   int status = PDQ_STATUS_OK, att = 0, k = 1;
   bool second = false;
-  double dt = cfg.dt0_per_instance ? wave_bcast(cfg.dt0_per_instance[inst], 0) : cfg.dt0, cstate = 1.0;
+  double dt = wave_rounded(c.a->cfg.dt0_per_instance ? c.a->cfg.dt0_per_instance[inst] : c.a->cfg.dt0), cstate = 1.0;
+  // the point being solved for, and the one after it (its load is a point ahead of its use)
+  double t1 = wave_rounded(ts[1]), t_prev = S.t, t_ahead = ts[K > 2 ? 2 : 1];
+  auto next_point = [&]() {
+    ++k;
+    t_prev = t1;
+    t1 = wave_rounded(t_ahead);
+    t_ahead = ts[k + 1 < K ? k + 1 : K - 1];
+  };
   while (k < K && status == PDQ_STATUS_OK) {
-    const double t1 = wave_bcast(ts[k], 0);
+    c.renew();
+    const WCfg& cfg = c.cfg;
     int op;
     if (grid) op = WOP_STEP;
     else if (second) op = WOP_BEYOND2;
-    else if (S.t + cfg.eps < t1) op = WOP_STEP;
-    else op = S.t > t1 + cfg.eps ? WOP_BEYOND1 : WOP_AT;
+    else if (wave_true(S.t + cfg.eps < t1)) op = WOP_STEP;
+    else op = wave_true(S.t > t1 + cfg.eps) ? WOP_BEYOND1 : WOP_AT;
     if (op == WOP_AT) {
       // interpolate_fwd_at_t1 (solvers.py:271-315)
       const double* const X = c.slot(sf);
@@ -799,12 +857,12 @@ __device__ __forceinline__ void w_solve_instance(const WCtx<SH>& c) {
       wave_sync();
       if (fp) S.ident = true;
       F = S;
-      ++k;
+      next_point();
       continue;
     }
     double h;
     if (op == WOP_STEP) {
-      h = grid ? t1 - wave_bcast(ts[k - 1], 0) : dt;
+      h = grid ? t1 - t_prev : dt;
       if (!grid && cfg.clip_dt) h = fmin(h, t1 - S.t);
     } else {
       h = op == WOP_BEYOND1 ? t1 - F.t : S.t - t1;
@@ -823,7 +881,7 @@ __device__ __forceinline__ void w_solve_instance(const WCtx<SH>& c) {
         w_apply_flat_mean(c, Xm, Um);
         w_linearize(c, Um, tn, lin);
         w_calibrate(c, lin, Um, w_noise_scale(c, h, 1.0), err);
-        scale = wave_bcast(err.sigma, 0);
+        scale = wave_rounded(err.sigma);
       }
     }
     const double s = w_noise_scale(c, h, scale);
@@ -850,7 +908,7 @@ __device__ __forceinline__ void w_solve_instance(const WCtx<SH>& c) {
       R = S;
       R.t = tn;
       R.os = dynamic ? scale : (mle ? S.os : 1.0);
-      R.nsteps = S.nsteps + 1.0;
+      R.nsteps = S.nsteps + 1;
       R.ident = false;
       R.mle_run = R.mle_n = 0.0;
       if (mle) {
@@ -859,7 +917,7 @@ __device__ __forceinline__ void w_solve_instance(const WCtx<SH>& c) {
         const double nd = S.mle_n;
         const double x1 = sqrt(nd / (nd + 1)) * S.mle_run;
         const double x2 = sqrt(1 / (nd + 1)) * nt;
-        R.mle_run = wave_bcast(hypot(x1, x2), 0);
+        R.mle_run = hypot(x1, x2);
         R.mle_n = nd + 1;
       }
       ++attempts;
@@ -871,25 +929,24 @@ __device__ __forceinline__ void w_solve_instance(const WCtx<SH>& c) {
         sf = pr;
         pr = tmp;
         S = R;
-        ++k;
+        next_point();
         continue;
       }
       if (!dynamic) {
         w_apply_flat_mean(c, Xm, Um);
         w_calibrate(c, lin, Um, w_noise_scale(c, h, 1.0), err);
       }
-      const double ep = wave_bcast(w_error_power(c, err, Xm, Y + SH::sm, dtn, nord), 0);
-      dt = wave_bcast(w_control(cfg, h, cstate, ep), 0);
+      const double ep = wave_rounded(w_error_power(c, err, Xm, Y + SH::sm, dtn, nord));
+      dt = wave_rounded(w_control(c, h, cstate, ep));
       ++att;
-      if (!isfinite(ep) || !isfinite(dt)) {
+      const bool accept = wave_true(ep >= 1.0);
+      if (!wave_true(isfinite(ep) && isfinite(dt))) {
         status = PDQ_STATUS_NONFINITE;
-      } else if (ep < 1.0 && (dt == 0.0 || S.t + dt == S.t)) {
-        status = PDQ_STATUS_DT_UNDERFLOW;
-      } else if (ep >= 1.0 && R.t == S.t) {
-        status = PDQ_STATUS_DT_UNDERFLOW;  // accepted without advancing t
-      } else if ((cfg.max_attempts > 0 && att >= cfg.max_attempts && ep < 1.0) || attempts >= kMaxTotalAttempts) {
+      } else if (wave_true(accept ? R.t == S.t : dt == 0.0 || S.t + dt == S.t)) {
+        status = PDQ_STATUS_DT_UNDERFLOW;  // rejected and dt cannot advance t, or accepted without advancing it
+      } else if ((!accept && cfg.max_attempts > 0 && att >= cfg.max_attempts) || attempts >= kMaxTotalAttempts) {
         status = PDQ_STATUS_MAX_ATTEMPTS;
-      } else if (ep >= 1.0) {
+      } else if (accept) {
         ++accepted;
         att = 0;
         // interp_from <- step_from, step_from <- proposed
@@ -914,16 +971,17 @@ __device__ __forceinline__ void w_solve_instance(const WCtx<SH>& c) {
         F.ident = fp;
         second = true;
       } else {
-        ++k;
+        next_point();
       }
     } else {
       S.ident = false;
       second = false;
-      ++k;
+      next_point();
     }
   }
   if (status == PDQ_STATUS_OK) w_finalize(c, sf, S);
-  const pdq_solution& o = c.a->out;
+  c.renew();
+  const auto& o = c.a->out;
   if (l == 0) {
     if (o.attempts) o.attempts[inst] = attempts;
     if (o.accepted) o.accepted[inst] = accepted;
@@ -933,7 +991,7 @@ __device__ __forceinline__ void w_solve_instance(const WCtx<SH>& c) {
 
 // The transition into LDS; lanes of one wavefront.
 template <class SH>
-__device__ __forceinline__ void w_setup(const KArgs& a, double* lds, int l) {
+__device__ __forceinline__ void w_setup(WArgs& a, double* lds, int l) {
   wave_copy<SH::nn>(l, lds + SH::oA, a.A);
   wave_copy<SH::nn>(l, lds + SH::oQ, a.Q);
   wave_sync();

@@ -10,17 +10,17 @@
 namespace pdq {
 
 template <class SH>
-__global__ void __launch_bounds__(64) solve_wave_kernel(KArgs a) {
+__global__ void __launch_bounds__(64) solve_wave_kernel(KArgs args) {  // read in place (WArgs)
   extern __shared__ double pdq_wave_lds[];
-  WCtx<SH> c;
-  c.a = &a;
-  c.lds = pdq_wave_lds;
-  c.l = threadIdx.x;
+  WCtx<SH> c((WArgs*)__builtin_amdgcn_kernarg_segment_ptr(), pdq_wave_lds, threadIdx.x);
+  const WArgs& a = *c.a;
   w_setup<SH>(a, pdq_wave_lds, c.l);
   for (;;) {
-    int inst = 0;
-    if (c.l == 0) inst = atomicAdd(a.queue, 1);
-    c.inst = __builtin_amdgcn_readfirstlane(inst);
+    // Every lane takes part in the pull (lane 0 adds one, the others nothing).
+    // Under a branch for lane 0 alone, the other lanes' index is a constant of
+    // the loop, and the compiler may split the loop by lane: lane 0 leaves for
+    // the next pull while the others go round with their constant, for ever.
+    c.inst = __builtin_amdgcn_readfirstlane(atomicAdd(a.queue, c.l == 0 ? 1 : 0));
     if (c.inst >= a.n_inst) break;
     w_solve_instance(c);
   }

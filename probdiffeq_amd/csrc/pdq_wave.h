@@ -29,6 +29,28 @@ __device__ __forceinline__ double wave_bcast(double v, int src) {
 #endif
 }
 
+// The value that lane I of each row of 16 lanes holds, in that row's lanes: one
+// instruction where wave_bcast takes two.
+template <int I>
+__device__ __forceinline__ double wave_bcast_row(double v) {
+  static_assert(I < 16, "a lane of a row");
+#ifdef PDQ_HOST_EMU
+  return pdq_emu_shfl(v, I, 16);
+#else
+  return __builtin_amdgcn_update_dpp(0.0, v, 0x150 + I, 0xf, 0xf, true);  // row_newbcast
+#endif
+}
+
+// The lane index as a value of its own: comparisons with it are made where
+// they stand (one instruction) instead of ahead of the solve's loop, where
+// their masks would take scalar registers throughout and be spilled.
+__device__ __forceinline__ int wave_here(int lane) {
+#ifndef PDQ_HOST_EMU
+  asm("" : "+v"(lane));
+#endif
+  return lane;
+}
+
 // Whether v != 0 (or NaN) in lane src: a wave-uniform condition.
 __device__ __forceinline__ bool wave_nonzero(double v, int src) {
 #ifdef PDQ_HOST_EMU
@@ -39,6 +61,7 @@ __device__ __forceinline__ bool wave_nonzero(double v, int src) {
 }
 
 // A matrix pattern Pat gives
+//   COLS             columns (lanes that hold one)
 //   M                rows held (a lane's registers)
 //   NP               columns to triangularise (pivots 0..NP-1)
 //   MROWS            rows of the whole matrix
@@ -112,6 +135,13 @@ struct WaveQr {
     return t[0];
   }
 
+  // A reflector's value in every lane that holds a column.
+  template <int I>
+  static __device__ __forceinline__ double bcast(double v) {
+    if constexpr (Pat::COLS <= 16) return wave_bcast_row<I>(v);
+    else return wave_bcast(v, I);
+  }
+
   // Reflector I and the ones after it.
   template <int I>
   static __device__ __forceinline__ void from(double (&a)[Pat::M], int lane) {
@@ -122,18 +152,18 @@ struct WaveQr {
         if (wave_nonzero(ss, I)) {
           const double alpha = a[p];
           const double beta = -copysign(lane_sqrt_pos(fma(alpha, alpha, ss)), alpha);
-          const double tau = wave_bcast(lane_div_nz(beta - alpha, beta, lane_rcp_nz(beta)), I);
+          const double tau = bcast<I>(lane_div_nz(beta - alpha, beta, lane_rcp_nz(beta)));
           const double scal = lane_rcp_nz(alpha - beta);
           double v[Pat::M];
 #pragma unroll
           for (int r = 0; r < Pat::M; ++r)
-            if (plan.act[I][r]) v[r] = wave_bcast(a[r] * scal, I);
+            if (plan.act[I][r]) v[r] = bcast<I>(a[r] * scal);
           double w = alpha;
 #pragma unroll
           for (int r = 0; r < Pat::M; ++r)
             if (plan.act[I][r]) w += v[r] * a[r];
           w *= tau;
-          a[p] = lane == I ? beta : alpha - w;
+          a[p] = wave_here(lane) == I ? beta : alpha - w;
 #pragma unroll
           for (int r = 0; r < Pat::M; ++r)
             if (plan.act[I][r]) a[r] -= v[r] * w;
@@ -167,6 +197,17 @@ __device__ __forceinline__ double wave_rounded(double x) {
   return x;
 }
 
+// Whether c holds (the same in every lane), as a scalar condition: the branches
+// on it are scalar ones, while the values it compares stay in vector registers
+// (scalar registers are the scarce ones here).
+__device__ __forceinline__ bool wave_true(bool c) {
+#ifdef PDQ_HOST_EMU
+  return c;
+#else
+  return __builtin_amdgcn_ballot_w64(c) != 0;
+#endif
+}
+
 // acc + x x as one fused operation, also from acc = 0 (an addition of zero that
 // is folded away would leave two products to choose from).
 __device__ __forceinline__ double wave_add_square(double acc, double x) {
@@ -185,6 +226,15 @@ __device__ __forceinline__ double wave_add(double x, double y) {
   return x + y;
 }
 
+// x / sqrt(n) for n = 1, 2: the division's quotient, from the constant's
+// correctly rounded reciprocal (lane_div).
+template <int n>
+__device__ __forceinline__ double wave_div_root(double x) {
+  static_assert(n == 1 || n == 2, "the roots of 1 and 2");
+  constexpr double root = 1.4142135623730951, inverse = 0.7071067811865475;  // 1 / root, rounded to nearest
+  return n == 1 ? x : lane_div(x, root, inverse);
+}
+
 // Back substitution with the K x K leading triangle of R (lane c holds its
 // column c): x = R^-1 a[0..K-1] for the lane's own column.  The quotients are
 // those of the division: the diagonal's reciprocals are taken by their lanes
@@ -192,6 +242,7 @@ __device__ __forceinline__ double wave_add(double x, double y) {
 template <int K, int M>
 __device__ __forceinline__ void wave_backsolve(const double (&a)[M], int lane, double (&x)[K]) {
   double dg = a[0];
+  lane = wave_here(lane);
 #pragma unroll
   for (int i = 1; i < K; ++i) dg = lane == i ? a[i] : dg;
   const double y = 1.0 / dg;

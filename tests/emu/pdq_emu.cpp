@@ -309,10 +309,7 @@ void wave_emu_instance(const pdq::KArgs& a, int inst) {
   for (int l = 0; l < 64; ++l)
     th.emplace_back([&, l] {
       t_group_lane = l;
-      pdq::WCtx<SH> c;
-      c.a = &a;
-      c.lds = lds.data();
-      c.l = l;
+      pdq::WCtx<SH> c(&a, lds.data(), l);
       c.inst = inst;
       pdq::w_setup<SH>(a, lds.data(), l);
       pdq::w_solve_instance(c);
