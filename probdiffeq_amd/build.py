@@ -20,6 +20,7 @@ UNITS = [
     "pdq_coop.hip",
     "pdq_coop_wave_filter.hip",
     "pdq_coop_wave_smoother.hip",
+    "pdq_coop_wave_expo.hip",
     "pdq_lane.hip",
     "pdq_lane_filter.hip",
     "pdq_lane_fixedpoint.hip",

@@ -66,6 +66,7 @@ void launch_zero_queue(int* queue, hipStream_t st);
 // The same for fixed shapes at 64 lanes per instance (pdq_coop_wave_*.hip).
 int launch_coop_wave_filter(KArgs& a, hipStream_t st);
 int launch_coop_wave_smoother(KArgs& a, hipStream_t st);
+int launch_coop_wave_exponential(KArgs& a, hipStream_t st);
 // Lane-per-instance isotropic kernel (pdq_lane.hip): shapes (N = nu + 1, d)
 // it is instantiated for and its launcher.
 bool lane_supported(int N, int D);

@@ -12,6 +12,7 @@
 // (ssm_impl_dense.py:15-363, ssm_impl_isotropic.py:72-403).
 #include "pdq_args.h"
 #include "pdq_device.h"
+#include "pdq_pade.h"
 
 namespace pdq {
 
@@ -280,27 +281,6 @@ __device__ void g_lu_solve(const Grp<G>& g, double* M, int n, double* X1, int m1
     }
   }
   g.sync();
-}
-
-// pade_and_legendre_9 (util/gram_util.py:261-331): Pade coefficients and the
-// Legendre coefficient matrix.
-__device__ __forceinline__ double pade9(int i) {
-  constexpr double c[10] = {17643225600.0, 8821612800.0, 2075673600.0, 302702400.0, 30270240.0,
-                            2162160.0,     110880.0,     3960.0,       90.0,        1.0};
-  return c[i];
-}
-__device__ __forceinline__ double legendre9(int i, int j) {
-  constexpr double c[10][10] = {{17643225600.0, 0, 605404800.0, 0, 4324320.0, 0, 7920.0, 0, 2.0, 0},
-                                {0, 8821612800.0, 0, 155675520.0, 0, 617760.0, 0, 528.0, 0, 0},
-                                {0, 0, 1470268800.0, 0, 15444000.0, 0, 34320.0, 0, 10.0, 0},
-                                {0, 0, 0, 147026880.0, 0, 960960.0, 0, 1092.0, 0, 0},
-                                {0, 0, 0, 0, 10501920.0, 0, 42120.0, 0, 18.0, 0},
-                                {0, 0, 0, 0, 0, 583440.0, 0, 1320.0, 0, 0},
-                                {0, 0, 0, 0, 0, 0, 26520.0, 0, 26.0, 0},
-                                {0, 0, 0, 0, 0, 0, 0, 1020.0, 0, 0},
-                                {0, 0, 0, 0, 0, 0, 0, 0, 34.0, 0},
-                                {0, 0, 0, 0, 0, 0, 0, 0, 0, 1.0}};
-  return c[i][j];
 }
 
 // DenseExponential.transition (ssm_impl_dense.py:405-423) for the step dt,
@@ -1989,7 +1969,8 @@ int launch_offgrid_coop(OffgridCoopArgs& o, int G, hipStream_t st) {
 // show in the results.
 static bool coop_wave_supported(const KArgs& a) {
   const pdq_config& c = a.cfg;
-  if (a.mode == MODE_LML || a.lay.d != 2 || a.lay.expo) return false;
+  if (a.mode == MODE_LML || a.lay.d != 2) return false;
+  if (a.lay.expo && c.strategy != PDQ_FILTER) return false;
   if (c.error_estimator != PDQ_ERROR_RESIDUAL_STD || c.error_re_linearize || c.re_linearize_after_calibration)
     return false;
   if (c.factorisation == PDQ_DENSE) return a.lay.N >= 3 && a.lay.N <= 6;
@@ -1999,7 +1980,8 @@ static bool coop_wave_supported(const KArgs& a) {
 
 int launch_coop(KArgs& a, int G, hipStream_t st) {
   if (G == 64 && coop_wave_supported(a))
-    return a.cfg.strategy == PDQ_FILTER ? launch_coop_wave_filter(a, st) : launch_coop_wave_smoother(a, st);
+    return a.lay.expo ? launch_coop_wave_exponential(a, st)
+           : a.cfg.strategy == PDQ_FILTER ? launch_coop_wave_filter(a, st) : launch_coop_wave_smoother(a, st);
   switch (G) {
     case 4: return launch_coop_g<4>(a, st);
     case 8: return launch_coop_g<8>(a, st);

@@ -31,17 +31,19 @@
 #pragma once
 
 #include "pdq_args.h"
+#include "pdq_pade.h"
 #include "pdq_wave.h"
 
 namespace pdq {
 
-// A fixed shape: N = nu + 1, d, dense or isotropic, smoother or filter.
-template <int N_, int D_, bool DENSE_, bool SMOOTHER_>
+// A fixed shape: N = nu + 1, d, dense or isotropic, smoother or filter, IWP or
+// exponential prior.
+template <int N_, int D_, bool DENSE_, bool SMOOTHER_, bool EXPO_ = false>
 struct WShape {
   static constexpr int N = N_, d = D_;
-  static constexpr bool dense = DENSE_, smoother = SMOOTHER_;
+  static constexpr bool dense = DENSE_, smoother = SMOOTHER_, expo = EXPO_;
   static constexpr int nc = dense ? N * d : N, mc = dense ? 1 : d, ko = dense ? d : 1;
-  static constexpr int st = dense ? d : 1;  // stride of the IWP transition's non-zeros
+  static constexpr int st = dense && !expo ? d : 1;  // stride of the transition's non-zeros
   static constexpr int nn = nc * nc, ms = nc * mc;
   // LDS (doubles): the transition, then the instance
   static constexpr int oA = 0, oQ = oA + nn;
@@ -53,10 +55,16 @@ struct WShape {
   // three solution slots: mean, factor, conditional
   static constexpr int sm = 0, sL = sm + ms, sC = sL + nn, ssize = sC + (smoother ? csize : 0);
   static constexpr int oS = oE + (smoother ? csize : 0);
-  static constexpr int oPrm = oS + 3 * ssize;
+  // the exponential prior's drift rows and the scratch of its transition
+  static constexpr int m10 = 10 * d;  // columns of the Legendre terms
+  static constexpr int xD = oS + 3 * ssize, xp = xD + (expo ? d * nc : 0), xB = xp + nn, x2 = xB + nc * d, x4 = x2 + nn,
+                       x6 = x4 + nn, x8 = x6 + nn, xT = x8 + nn, xV = xT + nn, xW = xV + nn, xPB = xW + nn,
+                       xR = xPB + nc * d, xend = xR + nc * m10;
+  static constexpr int oPrm = expo ? xend : xD;
   static constexpr int fixed_size = oPrm;  // + n_params
   static_assert(2 * nc <= 32, "a column of the revert block per lane, a power per half wavefront");
   static_assert(N >= 2 && d <= 2, "the observation's rows and the columns' sums");
+  static_assert(!expo || (dense && 2 * nc + m10 <= 64), "a column of the linear system per lane");
 };
 
 // The stacks' patterns (WaveQrPlan).
@@ -77,6 +85,18 @@ struct WPatUpdate {  // [[diagonal, 0], [(H L)^T, L^T]]: H reads derivatives 0 a
   static constexpr int nc = SH::nc, ko = SH::ko, M = ko + nc, NP = M, MROWS = M, COLS = M;
   static constexpr int row(int r) { return r; }
   static constexpr bool nz(int r, int c) { return r < ko ? r == c : (c < ko ? r - ko < 2 * ko : r - ko <= c - ko); }
+};
+template <class SH>
+struct WPatTall {  // the Legendre terms: dense
+  static constexpr int nc = SH::nc, M = SH::m10, NP = nc, MROWS = M, COLS = nc;
+  static constexpr int row(int r) { return r; }
+  static constexpr bool nz(int, int) { return true; }
+};
+template <class SH>
+struct WPatDouble {  // [upper triangle; dense]
+  static constexpr int nc = SH::nc, M = 2 * nc, NP = nc, MROWS = M, COLS = nc;
+  static constexpr int row(int r) { return r; }
+  static constexpr bool nz(int r, int c) { return r >= nc || r <= c; }
 };
 template <class SH>
 struct WPatFx {  // [(H L)^T; diagonal], without (H L)^T's zero rows
@@ -139,6 +159,27 @@ struct WCfg {
         max_attempts(c.max_attempts) {}
 };
 
+// The exponential prior's constants of a lane: rhs lane 2 nc + q of the linear
+// system holds column q of the Legendre terms (block q / d), with the block's
+// coefficients and the root of 2 block + 1.
+struct WLegendre {
+  double c[5], den, rden;
+  __device__ __forceinline__ WLegendre(int col, int d) {
+    int blk = col < 0 ? 0 : col / d;
+    blk = blk < 10 ? blk : 9;
+#pragma unroll
+    for (int kk = 0; kk < 5; ++kk) {
+      // row `blk` of the table by selection: the index differs between lanes
+      double v = 0.0;
+#pragma unroll
+      for (int b = 0; b < 10; ++b) v = blk == b ? legendre9(b, 2 * kk + (b & 1)) : v;
+      c[kk] = v;
+    }
+    den = sqrt((double)(2 * blk + 1));
+    rden = 1.0 / den;
+  }
+};
+
 template <class SH>
 struct WCtx {
   WArgs* a;
@@ -146,13 +187,16 @@ struct WCtx {
   double* lds;
   int l, inst, K;
   bool dynamic;  // solver_dynamic
+  double base_scale;
+  WLegendre lg;
   __device__ __forceinline__ double* P() const { return lds + SH::oP; }
   __device__ __forceinline__ double* PI() const { return lds + SH::oPI; }
   __device__ __forceinline__ const double* A() const { return lds + SH::oA; }
   __device__ __forceinline__ const double* Q() const { return lds + SH::oQ; }
   __device__ __forceinline__ const double* prm() const { return lds + SH::oPrm; }
   __device__ __forceinline__ double* slot(int s) const { return lds + SH::oS + s * SH::ssize; }
-  __device__ __forceinline__ WCtx(WArgs* args, double* lds_, int lane) : a(args), cfg(args->cfg), lds(lds_), l(lane), inst(0), K(args->K), dynamic(args->cfg.solver == PDQ_SOLVER_DYNAMIC) {}
+  __device__ __forceinline__ WCtx(WArgs* args, double* lds_, int lane) : a(args), cfg(args->cfg), lds(lds_), l(lane), inst(0), K(args->K), dynamic(args->cfg.solver == PDQ_SOLVER_DYNAMIC),
+        base_scale(args->cfg.base_output_scale), lg(SH::expo ? lane - 2 * SH::nc : 0, SH::d) {}
   __device__ __forceinline__ bool ts1() const { return cfg.ts1 != 0; }
   __device__ __forceinline__ void renew() {
 #ifndef PDQ_HOST_EMU
@@ -174,16 +218,221 @@ __device__ __forceinline__ double w_precon(const WCtx<SH>& c, double dt, int nor
   return wave_bcast(p, 31);
 }
 
-template <class SH>
-__device__ __forceinline__ double w_noise_scale(const WCtx<SH>& c, double dt, double s) {
-  if (SH::dense) return sqrt(fabs(dt)) * s;
-  return sqrt(fabs(dt)) * c.a->cfg.base_output_scale * s;
-}
-
 // Row i's lane: lane i < nc (the others repeat row nc - 1 and write nothing).
 template <class SH>
 __device__ __forceinline__ int w_row(const WCtx<SH>& c) {
   return c.l < SH::nc ? c.l : SH::nc - 1;
+}
+
+// Z = X Y for n x n matrices in LDS (Z another one), each product's sum in
+// ascending order: a lane takes W consecutive entries of one row.
+template <int n>
+__device__ __forceinline__ void w_gemm(int l, const double* X, const double* Y, double* Z) {
+  constexpr int W = n * n <= 64 ? 1 : (n * n <= 128 ? 2 : 3);
+  static_assert(n % W == 0 && n * (n / W) <= 64, "one lane per W entries");
+  constexpr int per = n / W, lanes = n * per;
+  const int t = l < lanes ? l : lanes - 1, i = t / per, j = (t % per) * W;
+  double acc[W] = {};
+#pragma unroll
+  for (int q = 0; q < n; ++q) {
+    const double x = X[i * n + q];
+#pragma unroll
+    for (int w = 0; w < W; ++w) acc[w] += x * Y[q * n + j + w];
+  }
+  if (l < lanes)
+#pragma unroll
+    for (int w = 0; w < W; ++w) Z[i * n + j + w] = acc[w];
+  wave_sync();
+}
+
+// Z = X B for an n x n matrix X and n x d columns B.
+template <int n, int d>
+__device__ __forceinline__ void w_gemm_cols(int l, const double* X, const double* B, double* Z) {
+  static_assert(n * d <= 64, "a lane per entry");
+  const int t = l < n * d ? l : n * d - 1, i = t / d, k = t % d;
+  double acc = 0.0;
+#pragma unroll
+  for (int q = 0; q < n; ++q) acc += X[i * n + q] * B[q * d + k];
+  if (l < n * d) Z[t] = acc;
+  wave_sync();
+}
+
+// DenseExponential.transition (ssm_impl_dense.py:405-423) for the step dt:
+// e^{A_p} into A and the lower-triangular Gramian factor U into Q, as
+// exp_transition (pdq_coop.hip) forms them: A_p = dt p^-1 A p, B_p = sqrt|dt|
+// |p^-1| B, scaling by 2^-s, the degree-9 Pade / Legendre approximation, s
+// doublings, non-negative diagonal (exp_gram_cholesky, util/gram_util.py:
+// 17-77).  The linear system's columns (the denominator's, the numerator's,
+// the Legendre terms') are held one per lane: its LU with partial pivoting
+// eliminates all of them at once, and the back substitution runs on the
+// right-hand sides' lanes.  Its time is the instructions of one wavefront, a
+// few thousand in sequence; the run-time-shape form waited for LDS operands.
+// 200 Matern solves (nu = 4, d = 2, 20 points): 142 -> 23.5 ms, the same bits.
+template <class SH>
+__device__ __forceinline__ void w_exp_transition(const WCtx<SH>& c, double dt) {
+  constexpr int n = SH::nc, d = SH::d, N = SH::N, nn = SH::nn, m10 = SH::m10;
+  const int l = c.l;
+  double* const lds = c.lds;
+  double *const eA = lds + SH::oA, *const U = lds + SH::oQ, *const Ap = lds + SH::xp, *const Bp = lds + SH::xB;
+  double *const A2 = lds + SH::x2, *const A4 = lds + SH::x4, *const A6 = lds + SH::x6, *const A8 = lds + SH::x8;
+  double *const T = lds + SH::xT, *const V = lds + SH::xV, *const W = lds + SH::xW, *const PB = lds + SH::xPB;
+  double* const rhs = lds + SH::xR;
+  const double base = c.base_scale;
+#pragma unroll
+  for (int e0 = 0; e0 < nn; e0 += 64) {
+    const int e = e0 + l < nn ? e0 + l : nn - 1, i = e / n, j = e % n;
+    const double drift = lds[SH::xD + (i < n - d ? j : (i - (n - d)) * n + j)];
+    const double a = i < n - d ? (j == i + d ? 1.0 : 0.0) : drift;
+    const double v = ((dt * c.PI()[i]) * a) * c.P()[j];
+    if (e0 + l < nn) Ap[e] = v;
+  }
+  if (l < n * d) {
+    const int i = l / d, k = l % d;
+    Bp[l] = (sqrt(fabs(dt)) * fabs(c.PI()[i])) * (i == (N - 1) * d + k ? base : 0.0);
+  }
+  wave_sync();
+  // _exp_gram_cholesky_init: the number of doublings from the 1-norm
+  double a_l1;
+  {
+    const int j = w_row(c);
+    double s = 0.0;
+#pragma unroll
+    for (int i = 0; i < n; ++i) s += fabs(Ap[i * n + j]);
+    s = fmax(0.0, s);
+    a_l1 = 0.0;
+#pragma unroll
+    for (int q = 0; q < n; ++q) a_l1 = fmax(a_l1, wave_bcast(s, q));
+  }
+  const double s1 = log2(a_l1 / 0.41098379928173995), s2 = log2((double)(n - 1) / 9.0);
+  // at most 64 doublings (a 1-norm up to 0.41 2^64): a larger or non-finite
+  // norm gives a non-finite transition either way, and the loop stays bounded
+  double num = fmax(0.0, ceil(fmax(s1, s2)));
+  if (!(num <= 64.0)) num = 64.0;
+  const int nd = wave_int((int)num);
+  const double two = ldexp(1.0, nd), sq = sqrt(two);
+#pragma unroll
+  for (int e0 = 0; e0 < nn; e0 += 64)
+    if (e0 + l < nn) Ap[e0 + l] = (1.0 / two) * Ap[e0 + l];
+  if (l < n * d) Bp[l] = Bp[l] / sq;
+  wave_sync();
+  w_gemm<n>(l, Ap, Ap, A2);
+  w_gemm<n>(l, A2, A2, A4);
+  w_gemm<n>(l, A4, A2, A6);
+  w_gemm<n>(l, A6, A2, A8);
+#pragma unroll
+  for (int e0 = 0; e0 < nn; e0 += 64) {
+    const int e = e0 + l < nn ? e0 + l : nn - 1;
+    const double id = (e / n == e % n) ? 1.0 : 0.0, a2 = A2[e], a4 = A4[e], a6 = A6[e], a8 = A8[e];
+    const double t = (((pade9(9) * a8 + pade9(7) * a6) + pade9(5) * a4) + pade9(3) * a2) + pade9(1) * id;
+    const double v = (((pade9(8) * a8 + pade9(6) * a6) + pade9(4) * a4) + pade9(2) * a2) + pade9(0) * id;
+    if (e0 + l < nn) {
+      T[e] = t;
+      V[e] = v;
+      W[e] = a2;
+    }
+  }
+  wave_sync();
+  w_gemm<n>(l, Ap, T, A4);  // the odd part of the Pade approximant
+  w_gemm_cols<n, d>(l, A2, Bp, PB);
+  // the lane's column of the system
+  const bool den = l < n, num_l = l >= n && l < 2 * n;
+  const int mc = den ? l : (num_l ? l - n : n - 1);
+  const int rc = l >= 2 * n ? (l - 2 * n < m10 ? l - 2 * n : m10 - 1) : 0, rk = rc % d;
+  double x[n];
+#pragma unroll
+  for (int r = 0; r < n; ++r) x[r] = c.lg.c[1] * PB[r * d + rk] + c.lg.c[0] * Bp[r * d + rk];
+  // the Legendre terms: blocks 2i (even) and 2i + 1 (odd)
+#pragma unroll
+  for (int kk = 2; kk <= 4; ++kk) {
+    double* const to = kk % 2 == 0 ? T : W;
+    w_gemm<n>(l, A2, kk % 2 == 0 ? W : T, to);
+    w_gemm_cols<n, d>(l, to, Bp, PB);
+#pragma unroll
+    for (int r = 0; r < n; ++r) x[r] = x[r] + c.lg.c[kk] * PB[r * d + rk];
+  }
+  // L_odd = A L_odd, then every block / sqrt(2 b + 1)
+  {
+    const bool odd = (rc / d) % 2 == 1;
+    double y[n];
+#pragma unroll
+    for (int r = 0; r < n; ++r) {
+      double acc = 0.0;
+#pragma unroll
+      for (int q = 0; q < n; ++q) acc += Ap[r * n + q] * x[q];
+      y[r] = acc;
+    }
+#pragma unroll
+    for (int r = 0; r < n; ++r) {
+      const double v = lane_div(odd ? y[r] : x[r], c.lg.den, c.lg.rden);
+      const double vv = V[r * n + mc], pw = A4[r * n + mc], m = den ? vv - pw : vv + pw;
+      x[r] = l < 2 * n ? m : v;
+    }
+  }
+  wave_lu<n>(x, l);
+  double sol[n];
+  wave_backsolve<n>(x, l, sol);
+  if (num_l)
+#pragma unroll
+    for (int i = 0; i < n; ++i) eA[i * n + mc] = sol[i];
+  if (l >= 2 * n && l < 2 * n + m10)
+#pragma unroll
+    for (int i = 0; i < n; ++i) rhs[i * m10 + rc] = sol[i];
+  wave_sync();
+  const int row = w_row(c);
+  {
+    // qr_r(L^T)^T: the Gramian factor of the scaled problem
+    double a[m10];
+#pragma unroll
+    for (int r = 0; r < m10; ++r) a[r] = rhs[row * m10 + r];
+    wave_qr<WPatTall<SH>>(a, l);
+    const int here = wave_here(row);
+    if (l < n)
+#pragma unroll
+      for (int i = 0; i < n; ++i) U[row * n + i] = wave_r(a, i, here);
+    wave_sync();
+  }
+  // _exp_gram_cholesky_double
+  for (int it = 0; it < nd; ++it) {
+    double a[2 * n];
+#pragma unroll
+    for (int r = 0; r < n; ++r) {
+      a[r] = U[row * n + r];
+      a[n + r] = 0.0;
+    }
+#pragma unroll
+    for (int k = 0; k < n; ++k) {
+      const double g = eA[row * n + k];
+#pragma unroll
+      for (int r = 0; r <= k; ++r) a[n + r] += g * U[k * n + r];
+    }
+    w_gemm<n>(l, eA, eA, T);
+    wave_qr<WPatDouble<SH>>(a, l);
+    const int here = wave_here(row);
+    if (l < n)
+#pragma unroll
+      for (int i = 0; i < n; ++i) U[row * n + i] = wave_r(a, i, here);
+    wave_copy<nn>(l, eA, T);
+    wave_sync();
+  }
+  // non-negative diagonal (column signs)
+  double sgn[n], u[n];
+#pragma unroll
+  for (int j = 0; j < n; ++j) {
+    sgn[j] = U[j * n + j] < 0.0 ? -1.0 : 1.0;
+    u[j] = U[row * n + j];
+  }
+  wave_sync();
+  if (l < n)
+#pragma unroll
+    for (int j = 0; j < n; ++j) U[row * n + j] = u[j] * sgn[j];
+  wave_sync();
+}
+
+template <class SH>
+__device__ __forceinline__ double w_noise_scale(const WCtx<SH>& c, double dt, double s) {
+  if (SH::expo) return s;  // the factor holds sqrt|dt| and the base scale
+  if (SH::dense) return sqrt(fabs(dt)) * s;
+  return sqrt(fabs(dt)) * c.a->cfg.base_output_scale * s;
 }
 
 // The entries A[i][k] of row i of the transition in ascending k: f(A[i][k], k).
@@ -191,7 +440,7 @@ template <class SH, class F>
 __device__ __forceinline__ void w_prior_terms(const WCtx<SH>& c, int i, F f) {
   const int k0 = SH::st == 1 ? 0 : i % SH::st;
 #pragma unroll
-  for (int q = 0; q < SH::N; ++q) {
+  for (int q = 0; q < SH::nc / SH::st; ++q) {
     const int k = q * SH::st + k0;
     f(c.A()[i * SH::nc + k], k);
   }
@@ -205,7 +454,7 @@ __device__ __forceinline__ void w_prior_column(const WCtx<SH>& c, int i, const d
 #pragma unroll
   for (int r = 0; r < SH::nc; ++r) a[r] = 0.0;
 #pragma unroll
-  for (int q = 0; q < SH::N; ++q) {
+  for (int q = 0; q < SH::nc / SH::st; ++q) {
     const int k = q * SH::st + k0;
     const double ak = c.A()[i * SH::nc + k], p = c.PI()[k], pk = abs_p ? fabs(p) : p;
 #pragma unroll
@@ -869,6 +1118,7 @@ __device__ __forceinline__ void w_solve_instance(WCtx<SH> c) {
     }
     const double tn = S.t + h;
     const double dtn = w_precon(c, h, nord);
+    if constexpr (SH::expo) w_exp_transition(c, h);
     // the state that is predicted: step_from, interp_from, or the interpolated marginal
     const double* const Xs = op == WOP_STEP ? c.slot(sf) : c.slot(ifr);
     const double *const Xm = Xs + SH::sm, *const XL = Xs + SH::sL;
@@ -992,8 +1242,12 @@ __device__ __forceinline__ void w_solve_instance(WCtx<SH> c) {
 // The transition into LDS; lanes of one wavefront.
 template <class SH>
 __device__ __forceinline__ void w_setup(WArgs& a, double* lds, int l) {
-  wave_copy<SH::nn>(l, lds + SH::oA, a.A);
-  wave_copy<SH::nn>(l, lds + SH::oQ, a.Q);
+  if constexpr (SH::expo) {
+    wave_copy<SH::d * SH::nc>(l, lds + SH::xD, a.cfg.prior_drift);
+  } else {
+    wave_copy<SH::nn>(l, lds + SH::oA, a.A);
+    wave_copy<SH::nn>(l, lds + SH::oQ, a.Q);
+  }
   wave_sync();
 }
 

@@ -41,6 +41,17 @@ int launch_wave(KArgs& a, hipStream_t st) {
   return PDQ_OK;
 }
 
+// The exponential prior: the filter.
+inline int launch_coop_wave_expo(KArgs& a, hipStream_t st) {
+  switch (a.lay.N) {
+    case 3: return launch_wave<WShape<3, 2, true, false, true>>(a, st);
+    case 4: return launch_wave<WShape<4, 2, true, false, true>>(a, st);
+    case 5: return launch_wave<WShape<5, 2, true, false, true>>(a, st);
+    case 6: return launch_wave<WShape<6, 2, true, false, true>>(a, st);
+  }
+  return host_error(PDQ_ERR_UNSUPPORTED, "no fixed-shape kernel for num_derivatives = %d", a.lay.N - 1);
+}
+
 template <bool SMOOTHER>
 int launch_coop_wave_s(KArgs& a, hipStream_t st) {
   if (a.cfg.factorisation == PDQ_ISOTROPIC)

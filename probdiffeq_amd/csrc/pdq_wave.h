@@ -29,6 +29,15 @@ __device__ __forceinline__ double wave_bcast(double v, int src) {
 #endif
 }
 
+// The whole number that lane `src` holds, as a scalar.
+__device__ __forceinline__ int wave_pick(int v, int src) {
+#ifdef PDQ_HOST_EMU
+  return (int)pdq_emu_shfl((double)v, src, 64);
+#else
+  return __builtin_amdgcn_readlane(v, src);
+#endif
+}
+
 // The value that lane I of each row of 16 lanes holds, in that row's lanes: one
 // instruction where wave_bcast takes two.
 template <int I>
@@ -233,6 +242,50 @@ __device__ __forceinline__ double wave_div_root(double x) {
   static_assert(n == 1 || n == 2, "the roots of 1 and 2");
   constexpr double root = 1.4142135623730951, inverse = 0.7071067811865475;  // 1 / root, rounded to nearest
   return n == 1 ? x : lane_div(x, root, inverse);
+}
+
+// A whole number that every lane holds alike, as a scalar.
+__device__ __forceinline__ int wave_int(int v) {
+#ifdef PDQ_HOST_EMU
+  return v;
+#else
+  return __builtin_amdgcn_readfirstlane(v);
+#endif
+}
+
+// LU with partial pivoting (the first largest |entry| of each column pivots, as
+// LAPACK's idamax) of the K x K matrix whose columns lanes 0..K-1 hold, with
+// the row swaps and the forward substitution applied to the columns of all the
+// other lanes: on return lane c < K holds U's column c in the rows up to c, the
+// others their right-hand side, ready for wave_backsolve.
+template <int K>
+__device__ __forceinline__ void wave_lu(double (&a)[K], int lane) {
+#pragma unroll
+  for (int k = 0; k < K; ++k) {
+    double best = -1.0;
+    int bi = k;
+#pragma unroll
+    for (int r = k; r < K; ++r) {
+      const double v = fabs(a[r]);
+      if (v > best) {
+        best = v;
+        bi = r;
+      }
+    }
+    const int piv = wave_pick(bi, k);
+    if (piv != k) {
+#pragma unroll
+      for (int r = k + 1; r < K; ++r)
+        if (piv == r) {
+          const double t = a[k];
+          a[k] = a[r];
+          a[r] = t;
+        }
+    }
+    const double inv = 1.0 / a[k];
+#pragma unroll
+    for (int r = k + 1; r < K; ++r) a[r] -= wave_bcast(a[r] * inv, k) * a[k];
+  }
 }
 
 // Back substitution with the K x K leading triangle of R (lane c holds its

@@ -320,7 +320,8 @@ void wave_emu_instance(const pdq::KArgs& a, int inst) {
 
 template <int N, bool DENSE>
 void wave_emu(const pdq::KArgs& a, int inst) {
-  if (a.cfg.strategy == PDQ_FILTER) wave_emu_instance<pdq::WShape<N, 2, DENSE, false>>(a, inst);
+  if (DENSE && a.cfg.prior == PDQ_PRIOR_EXPONENTIAL) wave_emu_instance<pdq::WShape<N, 2, true, false, true>>(a, inst);
+  else if (a.cfg.strategy == PDQ_FILTER) wave_emu_instance<pdq::WShape<N, 2, DENSE, false>>(a, inst);
   else wave_emu_instance<pdq::WShape<N, 2, DENSE, true>>(a, inst);
 }
 }  // namespace
