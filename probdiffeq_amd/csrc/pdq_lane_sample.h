@@ -82,6 +82,7 @@ struct SampleStep {
 // loaded into a second set of registers before step k is computed, and two
 // doubles move per instruction (a wavefront's lanes are 64 rows apart in the
 // draws and samples: each access costs a cache line per lane).
+// 4096 instances x 16 samples x 200 points, nu = 4: 1.49 -> 1.03 ms (2.0 GB).
 template <int N, int D>
 __device__ __forceinline__ void lane_sample(const SampleArgs& a, size_t gid) {
   const int K = a.K;
