@@ -34,6 +34,7 @@ UNITS = [
     "pdq_lane_sample.hip",
     "pdq_bd.hip",
     "pdq_bd_filter.hip",
+    "pdq_bd_filter_opts.hip",
     "pdq_bd_fixedpoint.hip",
     "pdq_bd_fixedinterval.hip",
 ]

@@ -30,12 +30,22 @@
 // uniform.  Lanes beyond d pad the group: they take part in every
 // synchronisation and contribute exact zeros to the sums, and write nothing.
 //
+// What bounds it.  Instruction issue: at d = 512 two wavefronts share each
+// SIMD, and an attempt is about 900 instructions of each (nu = 2, filter), of
+// which only the controller's part is taken by one wavefront for all.  256
+// instances with d = 512 (25 600 attempts each): 117.1 ms with every option read
+// at run time, sums by LDS exchanges and the controller in every wavefront,
+// 86.6 ms (8 100 cycles per attempt) with the filter's default options folded
+// in, sums by register moves and the controller in one wavefront; d = 64: 1.38
+// and 0.99 ms, d = 200: 6.9 and 5.1 ms.
+//
 // The loops follow _ivpsolve/solvers_via_adaptive_steps.py:46-375 and
 // solvers.py:205-767 in the order of the lane-per-instance kernel
 // (pdq_lane.h) and the oracle, with the same status exits.
 #pragma once
 
 #include "pdq_lane.h"
+#include "pdq_wave.h"
 
 #ifdef PDQ_HOST_EMU
 // The CPU build runs a group as G threads (tests/emu): these hooks are the
@@ -51,6 +61,7 @@ namespace pdq {
 // instance).
 constexpr int kBdMaxDim = 512;
 constexpr int kBdRedStride = kBdMaxDim / 64;  // one group sum buffer: a partial per wavefront
+constexpr int kBdRedSize = 2 * kBdRedStride + 2;  // two such buffers, then the controller's results
 
 // Arguments of the block-diagonal kernel.
 struct BdArgs {
@@ -70,7 +81,7 @@ struct BdGroup {
   int lane;    // = block index
   bool multi;  // the group is the whole (multi-wavefront) workgroup
   double* y;   // 2 G doubles of LDS: the published zeroth coefficients, two buffers
-  double* red; // multi: one partial sum per wavefront, two buffers of kBdRedStride
+  double* red; // multi: kBdRedSize doubles: a partial sum per wavefront, two buffers; the controller's results
   // The buffer each of the next linearisation and group sum uses.  They
   // alternate, so a write never meets a read of the same buffer from the
   // previous call: between the two calls that share a buffer lies the other
@@ -105,26 +116,73 @@ struct BdGroup {
     return __shfl(v, src, w);
 #endif
   }
-  // Group sum; every lane returns the bitwise same total.  One wavefront: a
-  // butterfly, then lane 0's total.  Several: each wavefront's butterfly
-  // total, then the wavefronts' totals added in wavefront order.
+  // Whether this lane's wavefront takes the step's scalar decisions (sum).
+  __device__ __forceinline__ bool first_wave() const { return !multi || lane < 64; }
+  __device__ __forceinline__ double* ctl() const { return red + 2 * kBdRedStride; }
+  // Group sum: a butterfly per wavefront, whose total is the bitwise same in
+  // every lane (each stage adds the same two values in both lanes), then the
+  // wavefronts' totals added in wavefront order.  With several wavefronts only
+  // the first one's lanes get the total.
   __device__ __forceinline__ double sum(double v) const {
-    if (!multi) {
-      for (int m = G / 2; m >= 1; m >>= 1) v += shfl_xor(v, m, G);
-      return shfl(v, 0, G);
-    }
-#pragma unroll
-    for (int m = 32; m >= 1; m >>= 1) v += shfl_xor(v, m, 64);
-    v = shfl(v, 0, 64);
+    if (!multi) return wave_total(v, G);
+    v = wave_total(v, 64);
     const int w = lane / 64, nw = G / 64;
     double* const r = red + rbuf * kBdRedStride;
     rbuf ^= 1;
     if ((lane & 63) == 0) r[w] = v;
     sync();
-    double s = 0.0;
-    for (int i = 0; i < nw; ++i) s += r[i];
+    if (!first_wave()) return 0.0;
+    // all reads at once; the entries beyond nw stay 0
+    double p[kBdRedStride], s = 0.0;
+#pragma unroll
+    for (int i = 0; i < kBdRedStride; ++i) p[i] = r[i];
+#pragma unroll
+    for (int i = 0; i < kBdRedStride; ++i) s += p[i];
     return s;
   }
+  // The butterfly total over groups of w lanes.
+  __device__ __forceinline__ double wave_total(double v, int w) const {
+#ifdef PDQ_HOST_EMU
+    for (int m = w / 2; m >= 1; m >>= 1) v += shfl_xor(v, m, w);
+#else
+    if (w >= 16) {
+      // The same sums by register moves.  After the stage of distance m the
+      // values repeat with period m, so that within a row of 16 lanes a
+      // rotation by m fetches what an exchange would.
+      if (w >= 64) v = swap_sum<32>(v);
+      if (w >= 32) v = swap_sum<16>(v);
+      v += row_ror<8>(v);
+      v += row_ror<4>(v);
+      v += row_ror<2>(v);
+      v += row_ror<1>(v);
+    } else {
+      for (int m = w / 2; m >= 1; m >>= 1) v += shfl_xor(v, m, w);
+    }
+#endif
+    return v;
+  }
+#ifndef PDQ_HOST_EMU
+  template <int M>
+  static __device__ __forceinline__ double row_ror(double v) {
+    const uint64_t u = __builtin_bit_cast(uint64_t, v);
+    const uint32_t lo = __builtin_amdgcn_update_dpp(0, (int)(uint32_t)u, 0x120 + M, 0xf, 0xf, true);
+    const uint32_t hi = __builtin_amdgcn_update_dpp(0, (int)(uint32_t)(u >> 32), 0x120 + M, 0xf, 0xf, true);
+    return __builtin_bit_cast(double, ((uint64_t)hi << 32) | lo);
+  }
+  // v[l] + v[l ^ M], M = 16 or 32: the swap instruction leaves the lower M
+  // lanes' values (of each 2 M) in one register and the upper ones' in the other.
+  template <int M>
+  static __device__ __forceinline__ double swap_sum(double v) {
+    const uint64_t u = __builtin_bit_cast(uint64_t, v);
+    const uint32_t a = (uint32_t)u, b = (uint32_t)(u >> 32);
+    const auto lo = M == 32 ? __builtin_amdgcn_permlane32_swap(a, a, false, false)
+                            : __builtin_amdgcn_permlane16_swap(a, a, false, false);
+    const auto hi = M == 32 ? __builtin_amdgcn_permlane32_swap(b, b, false, false)
+                            : __builtin_amdgcn_permlane16_swap(b, b, false, false);
+    return __builtin_bit_cast(double, ((uint64_t)hi[0] << 32) | lo[0]) +
+           __builtin_bit_cast(double, ((uint64_t)hi[1] << 32) | lo[1]);
+  }
+#endif
 };
 
 // One block's solution slot: mean, lower factor (full N x N with structural
@@ -168,6 +226,15 @@ struct BdScal {
   double mle_n;
   bool ident;  // smoothers: the conditional is the identity
 };
+
+// Values rounded where they stand: not fused into a later sum.  (In the
+// kernels with OPTS the options' branches end the regions in which products
+// are fused; without the branches these marks keep the results the same bits.)
+template <int n>
+__device__ __forceinline__ void bd_rounded(double (&x)[n]) {
+#pragma unroll
+  for (int i = 0; i < n; ++i) x[i] = wave_rounded(x[i]);
+}
 
 template <int N, int STRATEGY>
 struct BdCtx {
@@ -234,7 +301,8 @@ __device__ __forceinline__ void bd_linearize(const BdCtx<N, STRATEGY>& c, const 
 // the previous and proposed means), as error_residual_std / error_state_std
 // produce them (solvers.py:925-996, 1041-1098); then the error power of the
 // whole instance from group sums (error_norm_scale_then_rms /
-// _rms_then_scale, solvers.py:770-811, over d errors and d references).
+// _rms_then_scale, solvers.py:770-811, over d errors and d references): in the
+// group's first wavefront, 0 in the others (bd_control).
 template <int N, int STRATEGY>
 __device__ __forceinline__ double bd_error_power(const BdCtx<N, STRATEGY>& c, double err, int row, const double* prev_m,
                                                  const double* prop_m, double dt, int nord) {
@@ -249,13 +317,35 @@ __device__ __forceinline__ double bd_error_power(const BdCtx<N, STRATEGY>& c, do
   if (cfg.error_norm == PDQ_NORM_SCALE_THEN_RMS) {
     const double rr = e / (cfg.atol + cfg.rtol * fabs(ref));
     const double tot = c.g.sum(c.act ? rr * rr : 0.0);
+    if (!c.g.first_wave()) return 0.0;
     norm = lane_div(sqrt(tot), c.sqd, c.rsqd);  // sqrt(tot) / sqrt(d)
   } else {
     const double sa = c.g.sum(c.act ? e * e : 0.0);
     const double sr = c.g.sum(c.act ? ref * ref : 0.0);
+    if (!c.g.first_wave()) return 0.0;
     norm = (sqrt(sa) / sqrt(d)) / (cfg.atol + cfg.rtol * (sqrt(sr) / sqrt(d)));
   }
   return lane_root_inv<N>(norm);  // pow(norm, -1/N), as the lane kernel's error power takes it
+}
+
+// The controller on the error power.  With several wavefronts the first one
+// takes the roots and powers for all (they would run one after another on the
+// SIMDs that hold two of them) and hands ep and the new dt over in LDS.
+template <int N, int STRATEGY>
+__device__ __forceinline__ double bd_control(const BdCtx<N, STRATEGY>& c, double h, double& cstate, double& ep) {
+  const pdq_config& cfg = c.a->cfg;
+  if (!c.g.multi) return lane_control(cfg, h, cstate, ep);
+  double* const r = c.g.ctl();
+  if (c.g.first_wave()) {
+    const double dt = lane_control(cfg, h, cstate, ep);
+    if (c.g.lane == 0) {
+      r[0] = ep;
+      r[1] = dt;
+    }
+  }
+  c.g.sync();
+  ep = r[0];
+  return r[1];
 }
 
 // The transition's marginalise with the block-diagonal |to_latent| on the
@@ -428,7 +518,10 @@ __device__ __forceinline__ double bd_step(const BdCtx<N, STRATEGY>& c, const BdS
     for (int i = 0; i < N; ++i)
 #pragma unroll
       for (int j = 0; j < N; ++j) UL[i * N + j] = fabs(P[i]) * (s1 * lane_iwp_q<N>(Q, i, j));
+    bd_rounded(Um);
+    bd_rounded(UL);
     bd_linearize<N, STRATEGY>(c, Um, tn, b, h0);
+    b = wave_rounded(b);
     double om, oL;
     lane_marginalise_fx<N, 1>(cfg, &b, h0, Um, UL, &om, oL);
     sigma = lane_rms_zero<1>(&om, oL);
@@ -446,6 +539,9 @@ __device__ __forceinline__ double bd_step(const BdCtx<N, STRATEGY>& c, const BdS
     PDQ_PHASE_BOUNDARY();
     if (STRATEGY == PDQ_FIXEDPOINT) lane_merge<N, 1>(zs.ident, sf.c, cv<N>(pr.c), cv<N>(pr.c));
   }
+  Pm[0] = wave_rounded(Pm[0]);  // the rows that the linearisation reads; the others' products are the update's
+  Pm[1] = wave_rounded(Pm[1]);
+  bd_rounded(PL);
   PDQ_PHASE_BOUNDARY();
   // (3) the update, the MLE running scale and the error estimate
   double Rm[N], RL[N * N], mo, oLu;
@@ -491,6 +587,10 @@ __device__ __forceinline__ double bd_step(const BdCtx<N, STRATEGY>& c, const BdS
       sigma = 1.0;
     }
   }
+  sigma = wave_rounded(sigma);
+  err = wave_rounded(err);
+
+
   double ep = 0.0;
   if (estimate) {
     const int err_row = state_std ? cfg.error_derivative_idx : 0;
@@ -707,8 +807,8 @@ __device__ __forceinline__ void bd_solve_instance(const BdArgs& a, const BdGroup
         double h = dt;
         if (cfg.clip_dt) h = fmin(h, t1 - zs.t);
         c.lin_set = pdq_lin_set(cfg, accepted);
-        const double ep = bd_step<N, STRATEGY>(c, sf, zs, pr, zp, h, true);
-        dt = lane_control(cfg, h, cstate, ep);
+        double ep = bd_step<N, STRATEGY>(c, sf, zs, pr, zp, h, true);
+        dt = bd_control(c, h, cstate, ep);
         ++att;
         ++attempts;
         if (!isfinite(ep) || !isfinite(dt)) {
@@ -752,15 +852,44 @@ __device__ __forceinline__ void bd_solve_instance(const BdArgs& a, const BdGroup
   }
 }
 
+// Whether the filter's kernels without OPTS take a solve: the options that
+// they fold in.  The kernels for every option hold five times the code
+// (burgers, d = 512: 13 900 instructions against 2 800) and keep twice as many
+// scalars as there are scalar registers.  The smoothers have no such kernels:
+// their slots' conditionals fill the vector registers either way.
+inline bool bd_default_options(const pdq_config& c, int mode) {
+  return c.strategy == PDQ_FILTER && mode == LMODE_SAVE_AT && c.solver == PDQ_SOLVER_DYNAMIC &&
+         c.constraint == PDQ_TS0 && c.error_estimator == PDQ_ERROR_RESIDUAL_STD &&
+         c.error_norm == PDQ_NORM_SCALE_THEN_RMS && !c.error_re_linearize && !c.error_per_unit_step &&
+         !c.re_linearize_after_calibration;
+}
+
+// The kernel's arguments with what an instantiation knows at compile time.
+template <bool OPTS>
+__device__ __forceinline__ BdArgs bd_args(const BdArgs& args, int strategy) {
+  BdArgs a = args;
+  a.cfg.strategy = strategy;
+  if (!OPTS) {
+    a.mode = LMODE_SAVE_AT;
+    a.cfg.solver = PDQ_SOLVER_DYNAMIC;
+    a.cfg.constraint = PDQ_TS0;
+    a.cfg.error_estimator = PDQ_ERROR_RESIDUAL_STD;
+    a.cfg.error_norm = PDQ_NORM_SCALE_THEN_RMS;
+    a.cfg.error_re_linearize = 0;
+    a.cfg.error_per_unit_step = 0;
+    a.cfg.re_linearize_after_calibration = 0;
+  }
+  return a;
+}
+
 #ifndef PDQ_HOST_EMU
 // Groups of G <= 64 lanes, 64 / G instances per wavefront, grid-stride over
 // instances.  A group's instances and its exits depend only on values the
 // whole group shares, so each group leaves the loop as a unit.
-template <int N, int STRATEGY>
+template <int N, int STRATEGY, bool OPTS>
 __global__ void __launch_bounds__(64) bd_wave_kernel(BdArgs args) {
   __shared__ double y[2 * 64];
-  BdArgs a = args;
-  a.cfg.strategy = STRATEGY;
+  const BdArgs a = bd_args<OPTS>(args, STRATEGY);
   const int G = a.G;
   const int gpw = 64 / G;
   BdGroup g;
@@ -776,12 +905,14 @@ __global__ void __launch_bounds__(64) bd_wave_kernel(BdArgs args) {
 
 // One workgroup of G = 64 * ceil(d / 64) <= 512 lanes per instance, grid-
 // stride over instances (uniform across the workgroup).
-template <int N, int STRATEGY>
+template <int N, int STRATEGY, bool OPTS>
 __global__ void __launch_bounds__(512) bd_block_kernel(BdArgs args) {
   __shared__ double y[2 * kBdMaxDim];
-  __shared__ double red[2 * kBdRedStride];
-  BdArgs a = args;
-  a.cfg.strategy = STRATEGY;
+  __shared__ double red[kBdRedSize];
+  const BdArgs a = bd_args<OPTS>(args, STRATEGY);
+  // zero: the partial sums of wavefronts that the workgroup does not have
+  if (threadIdx.x < kBdRedSize) red[threadIdx.x] = 0.0;
+  __syncthreads();
   BdGroup g;
   g.G = a.G;
   g.lane = threadIdx.x;

@@ -1,5 +1,6 @@
 // Dispatch of the block-diagonal kernel to its instantiations (compiled in
-// pdq_bd_<strategy>.hip).
+// pdq_bd_<strategy>.hip; the filter's for the default options in
+// pdq_bd_filter.hip, for every option in pdq_bd_filter_opts.hip).
 #include "pdq_bd_launch.h"
 
 namespace pdq {
@@ -9,9 +10,11 @@ namespace {
 template <int N>
 int launch_bd_n(BdArgs& a, hipStream_t st) {
   switch (a.cfg.strategy) {
-    case PDQ_FILTER: return launch_bd_ns<N, PDQ_FILTER>(a, st);
-    case PDQ_FIXEDPOINT: return launch_bd_ns<N, PDQ_FIXEDPOINT>(a, st);
-    case PDQ_FIXEDINTERVAL: return launch_bd_ns<N, PDQ_FIXEDINTERVAL>(a, st);
+    case PDQ_FILTER:
+      return bd_default_options(a.cfg, a.mode) ? launch_bd_ns<N, PDQ_FILTER, false>(a, st)
+                                               : launch_bd_ns<N, PDQ_FILTER, true>(a, st);
+    case PDQ_FIXEDPOINT: return launch_bd_ns<N, PDQ_FIXEDPOINT, true>(a, st);
+    case PDQ_FIXEDINTERVAL: return launch_bd_ns<N, PDQ_FIXEDINTERVAL, true>(a, st);
     default: return host_error(PDQ_ERR_INVALID, "unknown strategy %d", a.cfg.strategy);
   }
 }

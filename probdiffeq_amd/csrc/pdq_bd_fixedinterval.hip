@@ -3,5 +3,5 @@
 #include "pdq_bd_launch.h"
 
 namespace pdq {
-PDQ_BD_INSTANTIATE(PDQ_FIXEDINTERVAL)
+PDQ_BD_INSTANTIATE(PDQ_FIXEDINTERVAL, true)
 }  // namespace pdq

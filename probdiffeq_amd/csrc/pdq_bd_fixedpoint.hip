@@ -3,5 +3,5 @@
 #include "pdq_bd_launch.h"
 
 namespace pdq {
-PDQ_BD_INSTANTIATE(PDQ_FIXEDPOINT)
+PDQ_BD_INSTANTIATE(PDQ_FIXEDPOINT, true)
 }  // namespace pdq
