@@ -29,6 +29,8 @@ UNITS = [
     "pdq_lane_fixedpoint_opts.hip",
     "pdq_lane_fixedinterval_opts.hip",
     "pdq_lane_lml.hip",
+    "pdq_lane_lml_shared_nu3.hip",
+    "pdq_lane_lml_shared_nu4.hip",
     "pdq_lane_offgrid.hip",
     "pdq_post.hip",
     "pdq_lane_sample.hip",

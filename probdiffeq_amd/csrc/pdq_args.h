@@ -86,6 +86,7 @@ struct LmlArgs {
   double* value;    // n_inst, or null
   double* grad;     // n_inst x n_tan, or null
   double* scratch;  // (Kobs - 1) x CondLayout<N, MC>::size x (n_inst G)
+  double* shared;   // the batch's factors (pdq_lane_lml_shared.h), or null
 };
 
 int lane_lml_tangents_per_lane(int n_tan);
@@ -96,6 +97,13 @@ int launch_lane_lml(LmlArgs& a, int N, int D, int tpl, hipStream_t st);
 // scratch buffer holds lane_adj_scratch_doubles(...) doubles.
 size_t lane_adj_scratch_doubles(int N, int D, int K, int every, int n_inst);
 int launch_lane_adj(LmlArgs& a, int N, int D, hipStream_t st);
+// The same with the factors computed once for the batch (pdq_lane_lml_shared.h):
+// whether a solve takes that form, the doubles of the shared buffer and of the
+// lanes' scratch, the launch.
+bool lml_shared_takes(const pdq_config& c, int N, int D, int K, bool reverse);
+size_t lml_shared_doubles(int N, int K, int every);
+size_t lml_shared_scratch(int N, int D, int tpl, int K, int every, int n_inst, int G, bool reverse);
+int launch_lml_shared(LmlArgs& a, int N, int D, int tpl, bool reverse, hipStream_t st);
 // Off-grid marginals (pdq_lane_offgrid.hip), isotropic shapes of the lane
 // kernel, filter and fixed-interval smoother.
 struct OffgridArgs {

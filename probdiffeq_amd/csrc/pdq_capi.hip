@@ -604,7 +604,12 @@ int32_t pdq_lml_value_and_grad(const pdq_config* cfg, int32_t n_inst, const doub
     double* tinit = nullptr;
     double* adj_buf = nullptr;  // conditionals, node data, checkpoints and one segment per lane
     HIP_TRY(bufs.alloc(&tinit, sizeof(double) * (size_t)n_inst * N * d * (1 + n_tan)));
-    HIP_TRY(bufs.alloc(&adj_buf, sizeof(double) * pdq::lane_adj_scratch_doubles(N, d, K_grid, every, n_inst)));
+    const bool shared = pdq::lml_shared_takes(*cfg, N, d, K_grid, true);
+    double* shared_buf = nullptr;
+    if (shared) HIP_TRY(bufs.alloc(&shared_buf, sizeof(double) * pdq::lml_shared_doubles(N, K_grid, every)));
+    HIP_TRY(bufs.alloc(&adj_buf,
+                       sizeof(double) * (shared ? pdq::lml_shared_scratch(N, d, 0, K_grid, every, n_inst, 1, true)
+                                                : pdq::lane_adj_scratch_doubles(N, d, K_grid, every, n_inst))));
     rc = pdq::launch_taylor_tangents(cfg->vector_field, d, cfg->n_params, n_inst, cfg->num_derivatives, n_tan, params,
                                      y0, grid, tinit, st);
     if (rc) return rc;
@@ -625,7 +630,8 @@ int32_t pdq_lml_value_and_grad(const pdq_config* cfg, int32_t n_inst, const doub
     la.value = value;
     la.grad = grad;
     la.scratch = adj_buf;
-    return pdq::launch_lane_adj(la, N, d, st);
+    la.shared = shared_buf;
+    return shared ? pdq::launch_lml_shared(la, N, d, 0, true, st) : pdq::launch_lane_adj(la, N, d, st);
   }
   if (lane_ok && cfg->lanes_per_instance <= 1) {
     // lane-per-instance LML: G lanes per instance, `tpl` tangent columns each
@@ -640,7 +646,12 @@ int32_t pdq_lml_value_and_grad(const pdq_config* cfg, int32_t n_inst, const doub
     double* tinit = nullptr;
     double* cond_buf = nullptr;  // backward conditionals between observation nodes
     HIP_TRY(bufs.alloc(&tinit, sizeof(double) * (size_t)n_inst * N * d * (1 + n_tan)));
-    HIP_TRY(bufs.alloc(&cond_buf, sizeof(double) * csz * (size_t)std::max(1, Kobs - 1) * n_lanes));
+    const bool shared = pdq::lml_shared_takes(*cfg, N, d, K_grid, false);
+    double* shared_buf = nullptr;
+    if (shared) HIP_TRY(bufs.alloc(&shared_buf, sizeof(double) * pdq::lml_shared_doubles(N, K_grid, every)));
+    HIP_TRY(bufs.alloc(&cond_buf,
+                       sizeof(double) * (shared ? pdq::lml_shared_scratch(N, d, tpl, K_grid, every, n_inst, G, false)
+                                                : csz * (size_t)std::max(1, Kobs - 1) * n_lanes)));
     rc = pdq::launch_taylor_tangents(cfg->vector_field, d, cfg->n_params, n_inst, cfg->num_derivatives, n_tan, params,
                                      y0, grid, tinit, st);
     if (rc) return rc;
@@ -661,7 +672,8 @@ int32_t pdq_lml_value_and_grad(const pdq_config* cfg, int32_t n_inst, const doub
     la.value = value;
     la.grad = grad;
     la.scratch = cond_buf;
-    return pdq::launch_lane_lml(la, N, d, tpl, st);
+    la.shared = shared_buf;
+    return shared ? pdq::launch_lml_shared(la, N, d, tpl, false, st) : pdq::launch_lane_lml(la, N, d, tpl, st);
   }
   pdq::Layout L = pdq::make_layout(*cfg, n_tan);
   if (L.nc > 32) return set_err(PDQ_ERR_UNSUPPORTED, "dense state dimension %d exceeds 32", L.nc);

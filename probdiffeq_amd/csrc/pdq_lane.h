@@ -805,7 +805,8 @@ __device__ __forceinline__ double lane_rms_zero(const double* om, double oL) {
 // fx.revert(pred) + apply_flat(0) (ssm_impl_api.py:112-132): the update.
 template <int N, int D>
 __device__ __forceinline__ void lane_update(const pdq_config& cfg, const double* b, double h0, const double* Pm,
-                                            const double* PL, double* Xm, double* XL, double* mo, double& oL_out) {
+                                            const double* PL, double* Xm, double* XL, double* mo, double& oL_out,
+                                            double* gain_out = nullptr) {
   constexpr int n2 = N + 1;
   double big[n2 * n2];
 #pragma unroll
@@ -824,6 +825,9 @@ __device__ __forceinline__ void lane_update(const pdq_config& cfg, const double*
   const double r0 = lane_rcp_nz(big[0]);
 #pragma unroll
   for (int j = 0; j < N; ++j) gain[j] = lane_div(big[1 + j], big[0], r0);
+  if (gain_out)
+#pragma unroll
+    for (int j = 0; j < N; ++j) gain_out[j] = gain[j];
 #pragma unroll
   for (int i = 0; i < N; ++i)
 #pragma unroll

@@ -191,6 +191,230 @@ __device__ __forceinline__ void adj_recompute_step(const LaneCtx<N, D>& c, int f
   for (int j = 0; j < N; ++j) s.gain[j] = lane_div(big[1 + j], big[0], r0);
 }
 
+// The reverse scan (evaluate_lml) from the terminal marginal (Xm, XL) over the
+// intervals' conditionals cond(j): returns the value and stores each node's
+// gain, factor and residuals at node(j) (stride n_lanes).
+template <int N, int D, class C, class F>
+__device__ __forceinline__ double adj_scan(const LmlArgs& a, int inst, double* Xm, double* XL, size_t n_lanes, C&& cond,
+                                           F&& node) {
+  const int Kobs = (a.K - 1) / a.every + 1;
+  double lp = 0.0, num = 0.0;
+  const double c2pi = log(M_PI * 2.0);
+  constexpr int n2 = N + 1;
+  for (int j = Kobs - 1; j >= 0; --j) {
+    if (j < Kobs - 1) {
+      double Ym[N * D], YL[N * N];
+      lane_marginalise_cond<N, D>(cond(j), Xm, XL, Ym, YL);
+#pragma unroll
+      for (int e = 0; e < N * D; ++e) Xm[e] = Ym[e];
+#pragma unroll
+      for (int e = 0; e < N * N; ++e) XL[e] = YL[e];
+    }
+    PDQ_PHASE_BOUNDARY();
+    const double* y = a.data + ((size_t)inst * Kobs + j) * D;
+    const double sd = a.stds[(size_t)inst * Kobs + j];
+    double big[n2 * n2], mo[D];
+#pragma unroll
+    for (int r = 0; r < n2; ++r)
+#pragma unroll
+      for (int col = 0; col < n2; ++col) {
+        double v;
+        if (r < 1) v = col < 1 ? sd : 0.0;
+        else v = col < 1 ? XL[0 * N + (r - 1)] : XL[(col - 1) * N + (r - 1)];
+        big[r * n2 + col] = v;
+      }
+#pragma unroll
+    for (int col = 0; col < D; ++col) mo[col] = Xm[0 * D + col] + 0.0;
+    lane_qr<n2, n2, ObsRows0>(big);
+    const double r00 = big[0], rinv = 1.0 / r00;
+    double gain[N];
+#pragma unroll
+    for (int i = 0; i < N; ++i) gain[i] = lane_div(big[1 + i], r00, rinv);
+    double lpb = 0.0, wv[D];
+    const double slogdet = log(fabs(r00));
+#pragma unroll
+    for (int col = 0; col < D; ++col) {
+      wv[col] = lane_div(y[col] - mo[col], r00, rinv);
+      const double sq = 0.0 + wv[col] * wv[col];
+      lpb += -0.5 * (2.0 * slogdet + sq + 1.0 * c2pi);
+    }
+    if (num == 0.0) lp = lpb;
+    else if (a.average_pdfs) lp = (lp * num + lpb) / (num + 1);
+    else lp = lp + lpb;
+    num += 1.0;
+    double* nd = node(j);
+#pragma unroll
+    for (int i = 0; i < N; ++i) nd[(size_t)i * n_lanes] = gain[i];
+    nd[(size_t)N * n_lanes] = r00;
+#pragma unroll
+    for (int col = 0; col < D; ++col) nd[(size_t)(N + 1 + col) * n_lanes] = wv[col];
+    // updated = reverted.apply_flat(data)
+    double Ym[N * D], YL[N * N];
+#pragma unroll
+    for (int i = 0; i < N; ++i)
+#pragma unroll
+      for (int col = 0; col < D; ++col) {
+        const double gy = 0.0 + gain[i] * y[col];
+        const double gm = 0.0 + gain[i] * mo[col];
+        Ym[i * D + col] = gy + (Xm[i * D + col] - gm);
+      }
+#pragma unroll
+    for (int i = 0; i < N; ++i)
+#pragma unroll
+      for (int k = 0; k < N; ++k) YL[i * N + k] = big[(1 + k) * n2 + 1 + i];
+#pragma unroll
+    for (int e = 0; e < N * D; ++e) Xm[e] = Ym[e];
+#pragma unroll
+    for (int e = 0; e < N * N; ++e) XL[e] = YL[e];
+  }
+  return lp;
+}
+
+// The scan's adjoint, forward over the nodes: the adjoint of every interval
+// conditional's noise mean (at xibar(j)) and of the terminal marginal's mean.
+template <int N, int D, class C, class F, class X>
+__device__ __forceinline__ void adj_scan_adjoint(const LmlArgs& a, size_t n_lanes, C&& cond, F&& node, X&& xibar,
+                                                 double* xterm_bar) {
+  const int Kobs = (a.K - 1) / a.every + 1;
+  const double cw = a.average_pdfs ? 1.0 / (double)Kobs : 1.0;  // d lml / d logpdf_j
+  double corr_bar[N * D];
+#pragma unroll
+  for (int e = 0; e < N * D; ++e) corr_bar[e] = 0.0;
+  for (int j = 0; j < Kobs; ++j) {
+    const double* nd = node(j);
+    double gain[N], wv[D];
+#pragma unroll
+    for (int i = 0; i < N; ++i) gain[i] = nd[(size_t)i * n_lanes];
+    const double r00 = nd[(size_t)N * n_lanes];
+#pragma unroll
+    for (int col = 0; col < D; ++col) wv[col] = nd[(size_t)(N + 1 + col) * n_lanes];
+    // corrected_j = pred_j + gain (y - pred_j[0]); logpdf_j = -1/2 |(y - pred_j[0]) / r00|^2 + ...
+    double pred_bar[N * D];
+#pragma unroll
+    for (int col = 0; col < D; ++col) {
+      double mo_bar = cw * wv[col] / r00;
+#pragma unroll
+      for (int i = 0; i < N; ++i) mo_bar -= gain[i] * corr_bar[i * D + col];
+#pragma unroll
+      for (int i = 0; i < N; ++i) pred_bar[i * D + col] = corr_bar[i * D + col] + (i == 0 ? mo_bar : 0.0);
+    }
+    if (j == Kobs - 1) {
+#pragma unroll
+      for (int e = 0; e < N * D; ++e) xterm_bar[e] = pred_bar[e];
+      break;
+    }
+    // pred_j = to o (A (tl o corrected_{j+1}) + xi_j)  (marginalise of conditional j)
+    const auto cj = cond(j);
+    double* xb = xibar(j);
+    double tp[N * D];
+#pragma unroll
+    for (int i = 0; i < N; ++i)
+#pragma unroll
+      for (int col = 0; col < D; ++col) {
+        tp[i * D + col] = cj.to(i) * pred_bar[i * D + col];
+        xb[(size_t)(i * D + col) * n_lanes] = tp[i * D + col];
+      }
+#pragma unroll
+    for (int k = 0; k < N; ++k)
+#pragma unroll
+      for (int col = 0; col < D; ++col) {
+        double acc = 0.0;
+#pragma unroll
+        for (int i = 0; i < N; ++i) acc += cj.A(i, k) * tp[i * D + col];
+        corr_bar[k * D + col] = cj.tl(k) * acc;
+      }
+  }
+}
+
+// The adjoint of one forward step: from those of its results, the mean (mbar)
+// and the running conditional's noise mean (cbar), to those of its inputs, and
+// the parameters' share (tbar).  `ident`: the running conditional before the
+// step is the identity, else self (its A and to_latent scales).
+template <int N, int D, class C>
+__device__ __forceinline__ void adj_back_step(const pdq_config& cfg, const double* prm, int np, const double* P,
+                                              const double* PI, const double* Gb, const double* tob, const double* gain,
+                                              const double* Pm, bool ident, const C& self, double* mbar, double* cbar,
+                                              double* tbar) {
+  // update: m_{k+1} = Pm - gain (Pm[1] + b), b = -f(Pm[0])
+  double Pbar[N * D], bbar[D];
+#pragma unroll
+  for (int col = 0; col < D; ++col) {
+    double mo_bar = 0.0;
+#pragma unroll
+    for (int i = 0; i < N; ++i) mo_bar -= gain[i] * mbar[i * D + col];
+    bbar[col] = mo_bar;
+#pragma unroll
+    for (int i = 0; i < N; ++i) Pbar[i * D + col] = mbar[i * D + col] + (i == 1 ? mo_bar : 0.0);
+  }
+  // linearisation: d(-f)/dy and d(-f)/dtheta at y = Pm[0]
+  {
+    double yv[D];
+#pragma unroll
+    for (int jj = 0; jj < D; ++jj) yv[jj] = Pm[jj];
+#pragma unroll
+    for (int jj = 0; jj < D; ++jj) {
+      double acc = 0.0;
+#pragma unroll
+      for (int jf = 0; jf < D; ++jf) acc += bbar[jf] * vf_jac(cfg.vector_field, D, yv, prm, jf, jj);
+      Pbar[jj] -= acc;
+    }
+#pragma unroll
+    for (int q = 0; q < 8; ++q)
+      if (q < np) {
+        double acc = 0.0;
+#pragma unroll
+        for (int jf = 0; jf < D; ++jf) acc += bbar[jf] * vf_jac_param(cfg.vector_field, D, yv, prm, jf, q);
+        tbar[q] -= acc;
+      }
+  }
+  // merge(self = running conditional, other = bw): xi' = A_self (T o xi_bw) + xi_self,
+  // or to_bw o xi_bw behind an identity
+  double mbbar[N * D];
+  if (ident) {
+#pragma unroll
+    for (int i = 0; i < N; ++i)
+#pragma unroll
+      for (int col = 0; col < D; ++col) mbbar[i * D + col] = tob[i] * cbar[i * D + col];
+#pragma unroll
+    for (int e = 0; e < N * D; ++e) cbar[e] = 0.0;
+  } else {
+#pragma unroll
+    for (int k2 = 0; k2 < N; ++k2) {
+      const double T = self.tl(k2) * tob[k2];
+#pragma unroll
+      for (int col = 0; col < D; ++col) {
+        double acc = 0.0;
+#pragma unroll
+        for (int i = 0; i < N; ++i) acc += self.A(i, k2) * cbar[i * D + col];
+        mbbar[k2 * D + col] = T * acc;
+      }
+    }
+  }
+  // revert: tmp = A (PI o m); Pm = P o tmp; xi_bw = PI o m - G_b tmp
+  double tbarv[N * D];
+#pragma unroll
+  for (int i = 0; i < N; ++i)
+#pragma unroll
+    for (int col = 0; col < D; ++col) {
+      double acc = P[i] * Pbar[i * D + col];
+#pragma unroll
+      for (int r = 0; r < N; ++r) acc -= Gb[r * N + i] * mbbar[r * D + col];
+      tbarv[i * D + col] = acc;
+    }
+#pragma unroll
+  for (int k2 = 0; k2 < N; ++k2)
+#pragma unroll
+    for (int col = 0; col < D; ++col) {
+      double acc = 0.0;
+#pragma unroll
+      for (int i = 0; i < N; ++i) {
+        const double av = lane_iwp_a<N>(i, k2);
+        if (av != 0.0) acc += av * tbarv[i * D + col];
+      }
+      mbar[k2 * D + col] = PI[k2] * (mbbar[k2 * D + col] + acc);
+    }
+}
+
 // One lane: the forward pass with checkpoints, the reverse scan (value), the
 // scan's adjoint, and the backward sweep over the checkpoint segments.  With
 // SPLIT this is wavefront 0's part (lane_adj_recompute_role is wavefront 1's),
@@ -211,7 +435,7 @@ __device__ __forceinline__ void lane_adj_instance(const LArgs& la, const LmlArgs
   c.w.base = slots;
   c.lin_set = 0;
   const LaneWs<N, D>& w = c.w;
-  const int K = a.K, every = a.every, Kobs = (K - 1) / every + 1, ntan = a.n_tan;
+  const int K = a.K, every = a.every, ntan = a.n_tan;
   const AdjLayout<N, D> lay(K, every);
   double* const base = a.scratch + lane;
   auto at = [&](size_t off) -> double* { return base + off * n_lanes; };
@@ -289,127 +513,14 @@ __device__ __forceinline__ void lane_adj_instance(const LArgs& la, const LmlArgs
     sf = 0;
   }
   // ---- reverse scan (evaluate_lml): value, and each node's gain, factor, residuals
-  double lp = 0.0, num = 0.0;
-  const double c2pi = log(M_PI * 2.0);
-  constexpr int n2 = N + 1;
-  for (int j = Kobs - 1; j >= 0; --j) {
-    if (j < Kobs - 1) {
-      const CondStrided<N, D> src{at(lay.conds + (size_t)j * CL::size), n_lanes};
-      double Ym[N * D], YL[N * N];
-      lane_marginalise_cond<N, D>(src, Xm, XL, Ym, YL);
-#pragma unroll
-      for (int e = 0; e < N * D; ++e) Xm[e] = Ym[e];
-#pragma unroll
-      for (int e = 0; e < N * N; ++e) XL[e] = YL[e];
-    }
-    PDQ_PHASE_BOUNDARY();
-    const double* y = a.data + ((size_t)inst * Kobs + j) * D;
-    const double sd = a.stds[(size_t)inst * Kobs + j];
-    double big[n2 * n2], mo[D];
-#pragma unroll
-    for (int r = 0; r < n2; ++r)
-#pragma unroll
-      for (int col = 0; col < n2; ++col) {
-        double v;
-        if (r < 1) v = col < 1 ? sd : 0.0;
-        else v = col < 1 ? XL[0 * N + (r - 1)] : XL[(col - 1) * N + (r - 1)];
-        big[r * n2 + col] = v;
-      }
-#pragma unroll
-    for (int col = 0; col < D; ++col) mo[col] = Xm[0 * D + col] + 0.0;
-    lane_qr<n2, n2, ObsRows0>(big);
-    const double r00 = big[0], rinv = 1.0 / r00;
-    double gain[N];
-#pragma unroll
-    for (int i = 0; i < N; ++i) gain[i] = lane_div(big[1 + i], r00, rinv);
-    double lpb = 0.0, wv[D];
-    const double slogdet = log(fabs(r00));
-#pragma unroll
-    for (int col = 0; col < D; ++col) {
-      wv[col] = lane_div(y[col] - mo[col], r00, rinv);
-      const double sq = 0.0 + wv[col] * wv[col];
-      lpb += -0.5 * (2.0 * slogdet + sq + 1.0 * c2pi);
-    }
-    if (num == 0.0) lp = lpb;
-    else if (a.average_pdfs) lp = (lp * num + lpb) / (num + 1);
-    else lp = lp + lpb;
-    num += 1.0;
-    double* nd = at(lay.nodes + (size_t)j * AdjLayout<N, D>::node);
-#pragma unroll
-    for (int i = 0; i < N; ++i) nd[(size_t)i * n_lanes] = gain[i];
-    nd[(size_t)N * n_lanes] = r00;
-#pragma unroll
-    for (int col = 0; col < D; ++col) nd[(size_t)(N + 1 + col) * n_lanes] = wv[col];
-    // updated = reverted.apply_flat(data)
-    double Ym[N * D], YL[N * N];
-#pragma unroll
-    for (int i = 0; i < N; ++i)
-#pragma unroll
-      for (int col = 0; col < D; ++col) {
-        const double gy = 0.0 + gain[i] * y[col];
-        const double gm = 0.0 + gain[i] * mo[col];
-        Ym[i * D + col] = gy + (Xm[i * D + col] - gm);
-      }
-#pragma unroll
-    for (int i = 0; i < N; ++i)
-#pragma unroll
-      for (int k = 0; k < N; ++k) YL[i * N + k] = big[(1 + k) * n2 + 1 + i];
-#pragma unroll
-    for (int e = 0; e < N * D; ++e) Xm[e] = Ym[e];
-#pragma unroll
-    for (int e = 0; e < N * N; ++e) XL[e] = YL[e];
-  }
+  auto cond = [&](int j) { return CondStrided<N, D>{at(lay.conds + (size_t)j * CL::size), n_lanes}; };
+  auto node = [&](int j) { return at(lay.nodes + (size_t)j * AdjLayout<N, D>::node); };
+  const double lp = adj_scan<N, D>(a, inst, Xm, XL, n_lanes, cond, node);
   if (a.value && active) a.value[inst] = lp;
   if (!a.grad) return;
   // ---- adjoint of the scan, forward over the nodes
-  const double cw = a.average_pdfs ? 1.0 / (double)Kobs : 1.0;  // d lml / d logpdf_j
-  double corr_bar[N * D], xterm_bar[N * D];
-#pragma unroll
-  for (int e = 0; e < N * D; ++e) corr_bar[e] = 0.0;
-  for (int j = 0; j < Kobs; ++j) {
-    const double* nd = at(lay.nodes + (size_t)j * AdjLayout<N, D>::node);
-    double gain[N], wv[D];
-#pragma unroll
-    for (int i = 0; i < N; ++i) gain[i] = nd[(size_t)i * n_lanes];
-    const double r00 = nd[(size_t)N * n_lanes];
-#pragma unroll
-    for (int col = 0; col < D; ++col) wv[col] = nd[(size_t)(N + 1 + col) * n_lanes];
-    // corrected_j = pred_j + gain (y - pred_j[0]); logpdf_j = -1/2 |(y - pred_j[0]) / r00|^2 + ...
-    double pred_bar[N * D];
-#pragma unroll
-    for (int col = 0; col < D; ++col) {
-      double mo_bar = cw * wv[col] / r00;
-#pragma unroll
-      for (int i = 0; i < N; ++i) mo_bar -= gain[i] * corr_bar[i * D + col];
-#pragma unroll
-      for (int i = 0; i < N; ++i) pred_bar[i * D + col] = corr_bar[i * D + col] + (i == 0 ? mo_bar : 0.0);
-    }
-    if (j == Kobs - 1) {
-#pragma unroll
-      for (int e = 0; e < N * D; ++e) xterm_bar[e] = pred_bar[e];
-      break;
-    }
-    // pred_j = to o (A (tl o corrected_{j+1}) + xi_j)  (marginalise of conditional j)
-    const CondStrided<N, D> cj{at(lay.conds + (size_t)j * CL::size), n_lanes};
-    double* xb = at(lay.xibar + (size_t)j * N * D);
-    double tp[N * D];
-#pragma unroll
-    for (int i = 0; i < N; ++i)
-#pragma unroll
-      for (int col = 0; col < D; ++col) {
-        tp[i * D + col] = cj.to(i) * pred_bar[i * D + col];
-        xb[(size_t)(i * D + col) * n_lanes] = tp[i * D + col];
-      }
-#pragma unroll
-    for (int k = 0; k < N; ++k)
-#pragma unroll
-      for (int col = 0; col < D; ++col) {
-        double acc = 0.0;
-#pragma unroll
-        for (int i = 0; i < N; ++i) acc += cj.A(i, k) * tp[i * D + col];
-        corr_bar[k * D + col] = cj.tl(k) * acc;
-      }
-  }
+  double xterm_bar[N * D];
+  adj_scan_adjoint<N, D>(a, n_lanes, cond, node, [&](int j) { return at(lay.xibar + (size_t)j * N * D); }, xterm_bar);
   // ---- backward sweep over the forward steps
   double mbar[N * D], cbar[N * D], tbar[kMaxParams > 8 ? 8 : kMaxParams];
   const int np = cfg.n_params < 8 ? cfg.n_params : 8;
@@ -457,83 +568,7 @@ __device__ __forceinline__ void lane_adj_instance(const LArgs& la, const LmlArgs
       AdjStep<N, D> s;
       adj_recompute_step<N, D>(c, sf, a.times[k + 1] - a.times[k], s);
       const bool ident = w.at(sf, LS_IDENT) != 0.0;
-      // update: m_{k+1} = Pm - gain (Pm[1] + b), b = -f(Pm[0])
-      double Pbar[N * D], bbar[D];
-#pragma unroll
-      for (int col = 0; col < D; ++col) {
-        double mo_bar = 0.0;
-#pragma unroll
-        for (int i = 0; i < N; ++i) mo_bar -= s.gain[i] * mbar[i * D + col];
-        bbar[col] = mo_bar;
-#pragma unroll
-        for (int i = 0; i < N; ++i) Pbar[i * D + col] = mbar[i * D + col] + (i == 1 ? mo_bar : 0.0);
-      }
-      // linearisation: d(-f)/dy and d(-f)/dtheta at y = Pm[0]
-      {
-        double yv[D];
-#pragma unroll
-        for (int jj = 0; jj < D; ++jj) yv[jj] = s.Pm[jj];
-#pragma unroll
-        for (int jj = 0; jj < D; ++jj) {
-          double acc = 0.0;
-#pragma unroll
-          for (int jf = 0; jf < D; ++jf) acc += bbar[jf] * vf_jac(cfg.vector_field, D, yv, c.prm, jf, jj);
-          Pbar[jj] -= acc;
-        }
-        for (int q = 0; q < np; ++q) {
-          double acc = 0.0;
-#pragma unroll
-          for (int jf = 0; jf < D; ++jf) acc += bbar[jf] * vf_jac_param(cfg.vector_field, D, yv, c.prm, jf, q);
-          tbar[q] -= acc;
-        }
-      }
-      // merge(self = running conditional, other = bw): xi' = A_self (T o xi_bw) + xi_self,
-      // or to_bw o xi_bw behind an identity
-      double mbbar[N * D];
-      if (ident) {
-#pragma unroll
-        for (int i = 0; i < N; ++i)
-#pragma unroll
-          for (int col = 0; col < D; ++col) mbbar[i * D + col] = s.tob[i] * cbar[i * D + col];
-#pragma unroll
-        for (int e = 0; e < N * D; ++e) cbar[e] = 0.0;
-      } else {
-        const CondRef<N, D> self = w.cond(sf);
-#pragma unroll
-        for (int k2 = 0; k2 < N; ++k2) {
-          const double T = self.tl(k2) * s.tob[k2];
-#pragma unroll
-          for (int col = 0; col < D; ++col) {
-            double acc = 0.0;
-#pragma unroll
-            for (int i = 0; i < N; ++i) acc += self.A(i, k2) * cbar[i * D + col];
-            mbbar[k2 * D + col] = T * acc;
-          }
-        }
-      }
-      // revert: tmp = A (PI o m); Pm = P o tmp; xi_bw = PI o m - G_b tmp
-      double tbarv[N * D];
-#pragma unroll
-      for (int i = 0; i < N; ++i)
-#pragma unroll
-        for (int col = 0; col < D; ++col) {
-          double acc = s.P[i] * Pbar[i * D + col];
-#pragma unroll
-          for (int r = 0; r < N; ++r) acc -= s.Gb[r * N + i] * mbbar[r * D + col];
-          tbarv[i * D + col] = acc;
-        }
-#pragma unroll
-      for (int k2 = 0; k2 < N; ++k2)
-#pragma unroll
-        for (int col = 0; col < D; ++col) {
-          double acc = 0.0;
-#pragma unroll
-          for (int i = 0; i < N; ++i) {
-            const double av = lane_iwp_a<N>(i, k2);
-            if (av != 0.0) acc += av * tbarv[i * D + col];
-          }
-          mbar[k2 * D + col] = s.PI[k2] * (mbbar[k2 * D + col] + acc);
-        }
+      adj_back_step<N, D>(cfg, c.prm, np, s.P, s.PI, s.Gb, s.tob, s.gain, s.Pm, ident, w.cond(sf), mbar, cbar, tbar);
     }
   }
   // the initial mean's adjoint against the Taylor coefficients' sensitivities

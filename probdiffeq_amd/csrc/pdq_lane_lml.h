@@ -264,87 +264,13 @@ __device__ __forceinline__ int lane_lml_forward_split(const LaneCtx<N, D * (1 + 
 }
 #endif
 
-// Lane g of instance `inst`: the forward pass, the reverse scan, and its
-// share of the outputs.  `slots` is the lane's LDS column (stride 64);
-// `glane` / `n_lanes` index the lane in the HBM scratch buffer.  With SPLIT
-// the forward pass runs on two wavefronts (lane_lml_forward_split); `active`
-// tells whether the lane has work (every lane of both wavefronts calls this,
-// the merging wavefront's lanes only for the forward pass), `lds_req` is the
-// workgroup's request array.
-template <int N, int D, int TPL, bool SPLIT = false>
-__device__ __forceinline__ void lane_lml_instance(const LArgs& la, const LmlArgs& a, int inst, int g, double* slots,
-                                                  size_t glane, size_t n_lanes, bool active = true,
-                                                  int* lds_req = nullptr) {
+// The reverse scan (MarkovSequence.evaluate_lml, estimators_and_losses.py:180-218)
+// from the terminal marginal (Xm, XL) over the intervals' conditionals cond(j),
+// and this tangent group's share of the outputs.
+template <int N, int D, int TPL, class F>
+__device__ __forceinline__ void lane_lml_scan(const LmlArgs& a, int inst, int g, double* Xm, double* XL, F&& cond) {
   constexpr int MC = D * (1 + TPL);
-  using CL = CondLayout<N, MC>;
-  const pdq_config& cfg = a.cfg;
-  LaneCtx<N, MC> c;
-  c.a = &la;
-  c.inst = inst;
-  c.prm = a.params + (size_t)inst * cfg.n_params;
-  c.w.base = slots;
-  c.lin_set = 0;
-  const LaneWs<N, MC>& w = c.w;
-  const int ntan = a.n_tan, q0 = g * TPL;
-  const int K = a.K, every = a.every, Kobs = (K - 1) / every + 1;
-  int sf = 0, pr = 1;
-  if (active && !(SPLIT && threadIdx.x >= kLaneBlock)) {
-    // prior: mean = Taylor coefficients (with tangents), chol = init_std I
-    const double* tc = a.tcoeffs + (size_t)inst * N * D * (1 + ntan);
-    double m[N * MC], L[N * N];
-#pragma unroll
-    for (int i = 0; i < N; ++i)
-#pragma unroll
-      for (int k = 0; k < D; ++k) {
-        m[i * MC + k] = tc[(i * D + k) * (1 + ntan)];
-#pragma unroll
-        for (int tt = 0; tt < TPL; ++tt) m[i * MC + (1 + tt) * D + k] = tc[(i * D + k) * (1 + ntan) + 1 + q0 + tt];
-      }
-#pragma unroll
-    for (int i = 0; i < N; ++i)
-#pragma unroll
-      for (int j = 0; j < N; ++j) L[i * N + j] = i == j ? (cfg.init_std_rows ? cfg.init_std_rows[i] : cfg.init_std) : 0.0;
-#pragma unroll
-    for (int e = 0; e < SlotLayout<N, MC>::size; ++e) w.at(sf, e) = 0.0;
-    w.store_mL(sf, m, L);
-    w.at(sf, LS_T) = a.times[0];
-    w.at(sf, LS_OS) = 1.0;
-    w.at(sf, LS_IDENT) = 1.0;
-  }
-  if constexpr (SPLIT) {
-#ifndef PDQ_HOST_EMU
-    sf = lane_lml_forward_split<N, D, TPL>(c, a, q0, glane, n_lanes, active, lds_req);
-    if (threadIdx.x >= kLaneBlock) return;  // the merging wavefront's part ends here
-#endif
-  } else {
-    for (int k = 1; k < K; ++k) {
-      lane_lml_step<N, D, TPL>(c, q0, sf, pr, a.times[k] - a.times[k - 1]);
-      const int tmp = sf;
-      sf = pr;
-      pr = tmp;
-      if (k % every == 0) {
-        // the reset: store the interval's conditional, restart behind an identity
-        const CondStrided<N, MC> dst{a.scratch + (size_t)(k / every - 1) * CL::size * n_lanes + glane, n_lanes};
-        cond_copy<N, MC>(dst, w.cond(sf));
-        w.at(sf, LS_IDENT) = 1.0;
-      }
-    }
-  }
-  if (!active) return;
-  // terminal marginal: posterior1.conditional.marginalise(posterior1.marginal)
-  double Xm[N * MC], XL[N * N];
-  {
-    double Sm[N * MC], SLf[N * N];
-    w.load_mL(sf, Sm, SLf);
-    if (w.at(sf, LS_IDENT) != 0.0) {
-#pragma unroll
-      for (int e = 0; e < N * MC; ++e) Xm[e] = Sm[e];
-#pragma unroll
-      for (int e = 0; e < N * N; ++e) XL[e] = SLf[e];
-    } else {
-      lane_marginalise_cond<N, MC>(w.cond(sf), Sm, SLf, Xm, XL);
-    }
-  }
+  const int ntan = a.n_tan, q0 = g * TPL, Kobs = (a.K - 1) / a.every + 1;
   double lp[1 + TPL];
 #pragma unroll
   for (int q = 0; q <= TPL; ++q) lp[q] = 0.0;
@@ -353,9 +279,8 @@ __device__ __forceinline__ void lane_lml_instance(const LArgs& la, const LmlArgs
   constexpr int n2 = N + 1;
   for (int j = Kobs - 1; j >= 0; --j) {
     if (j < Kobs - 1) {
-      const CondStrided<N, MC> src{a.scratch + (size_t)j * CL::size * n_lanes + glane, n_lanes};
       double Ym[N * MC], YL[N * N];
-      lane_marginalise_cond<N, MC>(src, Xm, XL, Ym, YL);
+      lane_marginalise_cond<N, MC>(cond(j), Xm, XL, Ym, YL);
 #pragma unroll
       for (int e = 0; e < N * MC; ++e) Xm[e] = Ym[e];
 #pragma unroll
@@ -431,6 +356,92 @@ __device__ __forceinline__ void lane_lml_instance(const LArgs& la, const LmlArgs
   if (a.grad)
 #pragma unroll
     for (int tt = 0; tt < TPL; ++tt) a.grad[(size_t)inst * ntan + q0 + tt] = lp[1 + tt];
+}
+
+// Lane g of instance `inst`: the forward pass, the reverse scan, and its
+// share of the outputs.  `slots` is the lane's LDS column (stride 64);
+// `glane` / `n_lanes` index the lane in the HBM scratch buffer.  With SPLIT
+// the forward pass runs on two wavefronts (lane_lml_forward_split); `active`
+// tells whether the lane has work (every lane of both wavefronts calls this,
+// the merging wavefront's lanes only for the forward pass), `lds_req` is the
+// workgroup's request array.
+template <int N, int D, int TPL, bool SPLIT = false>
+__device__ __forceinline__ void lane_lml_instance(const LArgs& la, const LmlArgs& a, int inst, int g, double* slots,
+                                                  size_t glane, size_t n_lanes, bool active = true,
+                                                  int* lds_req = nullptr) {
+  constexpr int MC = D * (1 + TPL);
+  using CL = CondLayout<N, MC>;
+  const pdq_config& cfg = a.cfg;
+  LaneCtx<N, MC> c;
+  c.a = &la;
+  c.inst = inst;
+  c.prm = a.params + (size_t)inst * cfg.n_params;
+  c.w.base = slots;
+  c.lin_set = 0;
+  const LaneWs<N, MC>& w = c.w;
+  const int ntan = a.n_tan, q0 = g * TPL;
+  const int K = a.K, every = a.every;
+  int sf = 0, pr = 1;
+  if (active && !(SPLIT && threadIdx.x >= kLaneBlock)) {
+    // prior: mean = Taylor coefficients (with tangents), chol = init_std I
+    const double* tc = a.tcoeffs + (size_t)inst * N * D * (1 + ntan);
+    double m[N * MC], L[N * N];
+#pragma unroll
+    for (int i = 0; i < N; ++i)
+#pragma unroll
+      for (int k = 0; k < D; ++k) {
+        m[i * MC + k] = tc[(i * D + k) * (1 + ntan)];
+#pragma unroll
+        for (int tt = 0; tt < TPL; ++tt) m[i * MC + (1 + tt) * D + k] = tc[(i * D + k) * (1 + ntan) + 1 + q0 + tt];
+      }
+#pragma unroll
+    for (int i = 0; i < N; ++i)
+#pragma unroll
+      for (int j = 0; j < N; ++j) L[i * N + j] = i == j ? (cfg.init_std_rows ? cfg.init_std_rows[i] : cfg.init_std) : 0.0;
+#pragma unroll
+    for (int e = 0; e < SlotLayout<N, MC>::size; ++e) w.at(sf, e) = 0.0;
+    w.store_mL(sf, m, L);
+    w.at(sf, LS_T) = a.times[0];
+    w.at(sf, LS_OS) = 1.0;
+    w.at(sf, LS_IDENT) = 1.0;
+  }
+  if constexpr (SPLIT) {
+#ifndef PDQ_HOST_EMU
+    sf = lane_lml_forward_split<N, D, TPL>(c, a, q0, glane, n_lanes, active, lds_req);
+    if (threadIdx.x >= kLaneBlock) return;  // the merging wavefront's part ends here
+#endif
+  } else {
+    for (int k = 1; k < K; ++k) {
+      lane_lml_step<N, D, TPL>(c, q0, sf, pr, a.times[k] - a.times[k - 1]);
+      const int tmp = sf;
+      sf = pr;
+      pr = tmp;
+      if (k % every == 0) {
+        // the reset: store the interval's conditional, restart behind an identity
+        const CondStrided<N, MC> dst{a.scratch + (size_t)(k / every - 1) * CL::size * n_lanes + glane, n_lanes};
+        cond_copy<N, MC>(dst, w.cond(sf));
+        w.at(sf, LS_IDENT) = 1.0;
+      }
+    }
+  }
+  if (!active) return;
+  // terminal marginal: posterior1.conditional.marginalise(posterior1.marginal)
+  double Xm[N * MC], XL[N * N];
+  {
+    double Sm[N * MC], SLf[N * N];
+    w.load_mL(sf, Sm, SLf);
+    if (w.at(sf, LS_IDENT) != 0.0) {
+#pragma unroll
+      for (int e = 0; e < N * MC; ++e) Xm[e] = Sm[e];
+#pragma unroll
+      for (int e = 0; e < N * N; ++e) XL[e] = SLf[e];
+    } else {
+      lane_marginalise_cond<N, MC>(w.cond(sf), Sm, SLf, Xm, XL);
+    }
+  }
+  lane_lml_scan<N, D, TPL>(a, inst, g, Xm, XL, [&](int j) {
+    return CondStrided<N, MC>{a.scratch + (size_t)j * CL::size * n_lanes + glane, n_lanes};
+  });
 }
 
 // LDS bytes of one workgroup: two slots per lane, or with the merging

@@ -89,10 +89,10 @@ size_t lane_adj_scratch_doubles(int N, int D, int K, int every, int n_inst) {
 }
 
 int launch_lane_adj(LmlArgs& a, int N, int D, hipStream_t st) {
-  if (D == 2 && (N == 4 || N == 5)) {
-    const bool dyn = a.cfg.solver == PDQ_SOLVER_DYNAMIC;
-    if (N == 4) return dyn ? launch_adj_nd<4, 2, PDQ_SOLVER_DYNAMIC>(a, st) : launch_adj_nd<4, 2, PDQ_SOLVER>(a, st);
-    return dyn ? launch_adj_nd<5, 2, PDQ_SOLVER_DYNAMIC>(a, st) : launch_adj_nd<5, 2, PDQ_SOLVER>(a, st);
+  // (PDQ_SOLVER's factors are the batch's: pdq_lane_lml_shared.h)
+  if (D == 2 && a.cfg.solver == PDQ_SOLVER_DYNAMIC) {
+    if (N == 4) return launch_adj_nd<4, 2, PDQ_SOLVER_DYNAMIC>(a, st);
+    if (N == 5) return launch_adj_nd<5, 2, PDQ_SOLVER_DYNAMIC>(a, st);
   }
   return host_error(PDQ_ERR_UNSUPPORTED, "no adjoint LML kernel for nu + 1 = %d, d = %d", N, D);
 }

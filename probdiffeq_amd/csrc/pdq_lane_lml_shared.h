@@ -1,0 +1,616 @@
+// The LML and its reverse adjoint with the square-root factors computed once
+// for the whole batch (isotropic, ts0, PDQ_SOLVER).
+//
+// With ts0, the integrated Wiener prior and a constant output scale every
+// factor of the fixed-point smoother's forward pass is a function of the grid
+// and the prior alone (solver.step, solvers.py:702-733; the QRs never see a
+// mean), and the grid is one for all instances.  The lane kernels
+// (pdq_lane_lml.h, pdq_lane_adjoint.h) compute them in every lane of every
+// instance and tangent, in one serial chain of 9 400 cycles per grid step, and
+// the adjoint once more on its way back.  Here
+//  1. lml_chain_kernel: one wavefront runs the factors' own chain, the
+//     prediction's R_Y and the update (2 400 cycles per step; its lanes take 64
+//     steps' preconditioners at once), and leaves each step's factor and gain;
+//  2. lml_revert_kernel: one lane per step, the backward conditional's gain
+//     and factor;
+//  3. lml_merge_kernel: one lane per observation interval, the fixed-point
+//     merges (estimators_and_losses.py:473-591) of its steps;
+//  4. lml_means_kernel / lml_adjoint_kernel: one lane per instance (and tangent
+//     group), the means' recursion through those factors, the reverse scan
+//     (whose factors depend on the instance's observation stds) and the
+//     adjoint, which recomputes a segment's means from a checkpoint.
+// What the means' pass reads of a step is the same for every lane: a tile of
+// steps is staged in LDS by the wavefront, the next tile's loads under way.
+// The order of operations is the lane kernels'; against 64-bit arithmetic in
+// another order both gradients' errors are 3e-14 on average (nu = 3, 4; 64 to
+// 2000 steps).
+//
+// 1024 instances, nu = 3, 2000 steps, 101 observations: value 7.29 -> 3.31 ms,
+// with the gradient by tangents 7.82 -> 4.46 ms (chain 2.03, means 2.27), by the
+// adjoint 18.2 -> 5.28 ms (chain 2.03, means and adjoint 3.1); 300 instances,
+// nu = 4, 500 steps: 4.63 -> 1.68 and 10.95 -> 2.13 ms.  The chain and the
+// means' pass are bound by one wavefront's instruction issue.
+#pragma once
+
+#include "pdq_lane_adjoint.h"
+#include "pdq_lane_lml.h"
+#include "pdq_wave.h"
+
+namespace pdq {
+
+constexpr int kLmlTile = 16;  // grid steps staged at once, and per checkpoint of the adjoint
+
+// What a step's mean recursion needs of the factors (doubles): P, PI, the
+// update's gain, the merge's T = tl_self o to_b (behind an identity: to_b), the
+// revert's gain G, the running conditional's A before the step, and the time after it.
+template <int N>
+struct LmlRec {
+  static constexpr int P = 0, PI = N, gain = 2 * N, T = 3 * N, G = 4 * N, A = G + N * N, t = A + N * N,
+                       size = t + 1;
+};
+
+// The shared buffer: the records of the K - 1 steps; per step (and for the
+// final state) the factor before it and the backward conditional's; the
+// intervals' conditionals without their means.
+template <int N>
+struct LmlShared {
+  static constexpr int tri = N * (N + 1) / 2, fac = 2 * tri;
+  static constexpr int cA = 0, cL = N * N, ctl = cL + tri, cto = ctl + N, cond = cto + N;
+  size_t oF, oC, size;
+  __host__ __device__ LmlShared(int K, int every) {
+    oF = (size_t)(K - 1) * LmlRec<N>::size;
+    oC = oF + (size_t)K * fac;
+    size = oC + (size_t)((K - 1) / every) * cond;
+  }
+};
+
+// Interval j's conditional: the shared part and a lane's means (stride).
+template <int N, int D>
+struct LmlCond {
+  using SH = LmlShared<N>;
+  const double* __restrict__ f;
+  const double* mp;
+  size_t stride;
+  __device__ __forceinline__ double A(int i, int j) const { return f[SH::cA + i * N + j]; }
+  __device__ __forceinline__ double L(int i, int j) const { return j <= i ? f[SH::cL + tri(i, j)] : 0.0; }
+  __device__ __forceinline__ double tl(int i) const { return f[SH::ctl + i]; }
+  __device__ __forceinline__ double to(int i) const { return f[SH::cto + i]; }
+  __device__ __forceinline__ double m(int i, int c) const { return mp[(size_t)(i * D + c) * stride]; }
+};
+
+// The left columns of the revert block: rows N..2N-1 are dense, rows 0..N-1
+// upper triangular.
+template <int N>
+struct RevertLeftRows {
+  static constexpr bool nz(int, int r) { return r >= N; }
+};
+
+// One step of the factors' chain: L -> the update's gain and the next L.
+template <int N>
+__device__ __forceinline__ void lml_chain_step(const pdq_config& cfg, const double* Q, const double* P,
+                                               const double* PI, double s, double* L, double* gain) {
+  double big[2 * N * N], PL[N * N];
+#pragma unroll
+  for (int r = 0; r < N; ++r)
+#pragma unroll
+    for (int col = 0; col < N; ++col) {
+      big[r * N + col] = s * lane_iwp_q<N>(Q, col, r);
+      double acc = 0.0;
+#pragma unroll
+      for (int k = 0; k < N; ++k) {
+        const double a = lane_iwp_a<N>(col, k);
+        if (a != 0.0 && r <= k) acc += a * (fabs(PI[k]) * L[k * N + r]);
+      }
+      big[(N + r) * N + col] = acc;
+    }
+  lane_qr<2 * N, N, RevertLeftRows<N>>(big);
+#pragma unroll
+  for (int i = 0; i < N; ++i)
+#pragma unroll
+    for (int j = 0; j < N; ++j) PL[i * N + j] = j <= i ? fabs(P[i]) * big[j * N + i] : 0.0;
+  double none[N], Xm[N], mo, oL;
+  const double b = 0.0;
+#pragma unroll
+  for (int i = 0; i < N; ++i) none[i] = i == 1 ? 1.0 : 0.0;
+  lane_update<N, 1>(cfg, &b, 0.0, none, PL, Xm, L, &mo, oL, gain);
+}
+
+#ifndef PDQ_HOST_EMU
+template <int N>
+__global__ void __launch_bounds__(64) lml_chain_kernel(LmlArgs a) {
+  constexpr int ps = 2 * N + 2;
+  using R = LmlRec<N>;
+  using SH = LmlShared<N>;
+  __shared__ double pre[64 * ps];
+  pdq_config cfg = a.cfg;
+  cfg.constraint = PDQ_TS0;
+  const SH lay(a.K, a.every);
+  double* const rec = a.shared;
+  double* const fac = a.shared + lay.oF;
+  double L[N * N], Q[N * N], t = a.times[0];
+#pragma unroll
+  for (int e = 0; e < N * N; ++e) {
+    const int i = e / N;
+    L[e] = i == e % N ? (cfg.init_std_rows ? cfg.init_std_rows[i] : cfg.init_std) : 0.0;
+    Q[e] = a.Q[e];
+  }
+  auto put = [&](int s) {
+    if (threadIdx.x == 0) {
+#pragma unroll
+      for (int i = 0; i < N; ++i)
+#pragma unroll
+        for (int j = 0; j <= i; ++j) fac[(size_t)s * SH::fac + tri(i, j)] = L[i * N + j];
+    }
+  };
+  for (int c0 = 0; c0 < a.K - 1; c0 += 64) {
+    const int s = c0 + threadIdx.x;
+    if (s < a.K - 1) {
+      double P[N], PI[N];
+      const double h = a.times[s + 1] - a.times[s];
+      lane_precon<N>(h, P, PI);
+#pragma unroll
+      for (int i = 0; i < N; ++i) {
+        pre[threadIdx.x * ps + i] = P[i];
+        pre[threadIdx.x * ps + N + i] = PI[i];
+        rec[(size_t)s * R::size + R::P + i] = P[i];
+        rec[(size_t)s * R::size + R::PI + i] = PI[i];
+      }
+      pre[threadIdx.x * ps + 2 * N] = lane_noise_scale(cfg, h, 1.0);
+      pre[threadIdx.x * ps + 2 * N + 1] = h;
+    }
+    Grp<64>{}.sync();
+    const int n = a.K - 1 - c0 < 64 ? a.K - 1 - c0 : 64;
+    auto step = [&](int i, const double* now, double* next) {
+      double gain[N];
+#pragma unroll
+      for (int e = 0; e < ps; ++e) next[e] = pre[(i + 1 < n ? i + 1 : i) * ps + e];
+      PDQ_PHASE_BOUNDARY();
+      put(c0 + i);
+      t += now[2 * N + 1];
+      lml_chain_step<N>(cfg, Q, now, now + N, now[2 * N], L, gain);
+      if (threadIdx.x == 0) {
+        double* const r = rec + (size_t)(c0 + i) * R::size;
+#pragma unroll
+        for (int e = 0; e < N; ++e) r[R::gain + e] = gain[e];
+        r[R::t] = t;
+      }
+    };
+    double x[ps], y[ps];
+#pragma unroll
+    for (int e = 0; e < ps; ++e) x[e] = pre[e];
+    for (int i = 0; i < n; i += 2) {
+      step(i, x, y);
+      if (i + 1 < n) step(i + 1, y, x);
+    }
+    Grp<64>{}.sync();
+  }
+  put(a.K - 1);
+}
+
+// Step s's backward conditional from its factor.
+template <int N>
+__global__ void __launch_bounds__(64) lml_revert_kernel(LmlArgs a) {
+  using R = LmlRec<N>;
+  using SH = LmlShared<N>;
+  const SH lay(a.K, a.every);
+  const int s = blockIdx.x * 64 + threadIdx.x;
+  if (s >= a.K - 1) return;
+  double* const rec = a.shared + (size_t)s * R::size;
+  double* const fac = a.shared + lay.oF + (size_t)s * SH::fac;
+  double P[N], PI[N], Xm[N], XL[N * N], Ym[N], YL[N * N];
+#pragma unroll
+  for (int i = 0; i < N; ++i) {
+    P[i] = rec[R::P + i];
+    PI[i] = rec[R::PI + i];
+    Xm[i] = 0.0;
+#pragma unroll
+    for (int j = 0; j < N; ++j) XL[i * N + j] = j <= i ? fac[tri(i, j)] : 0.0;
+  }
+  LCond<N, 1> bw;
+  lane_revert_prior<N, 1>(a.Q, P, PI, lane_noise_scale(a.cfg, a.times[s + 1] - a.times[s], 1.0), Xm, XL, Ym, YL,
+                          LCondViewD<N, 1>{&bw});
+#pragma unroll
+  for (int e = 0; e < N * N; ++e) rec[R::G + e] = bw.v[CondLayout<N, 1>::A + e];
+#pragma unroll
+  for (int i = 0; i < N; ++i)
+#pragma unroll
+    for (int j = 0; j <= i; ++j) fac[SH::tri + tri(i, j)] = bw.L(i, j);
+}
+
+// Interval j's merges, in the order of its steps.
+template <int N>
+__global__ void __launch_bounds__(64) lml_merge_kernel(LmlArgs a) {
+  using R = LmlRec<N>;
+  using SH = LmlShared<N>;
+  const SH lay(a.K, a.every);
+  const int j = blockIdx.x * 64 + threadIdx.x;
+  if (j >= (a.K - 1) / a.every) return;
+  LCond<N, 1> self, bw;
+#pragma unroll
+  for (int e = 0; e < CondLayout<N, 1>::size; ++e) self.v[e] = bw.v[e] = 0.0;
+  for (int e0 = 0; e0 < a.every; ++e0) {
+    const size_t s = (size_t)j * a.every + e0;
+    double* const rec = a.shared + s * R::size;
+    const double* const fac = a.shared + lay.oF + s * SH::fac;
+#pragma unroll
+    for (int i = 0; i < N; ++i) {
+#pragma unroll
+      for (int k = 0; k < N; ++k) {
+        bw.A(i, k) = rec[R::G + i * N + k];
+        bw.setL(i, k, k <= i ? fac[SH::tri + tri(i, k)] : 0.0);
+      }
+      bw.tl(i) = lane_rcp_nz(rec[R::P + i]);
+      bw.to(i) = lane_rcp_nz(rec[R::PI + i]);
+      bw.m(i, 0) = 0.0;
+      rec[R::T + i] = e0 == 0 ? bw.to(i) : self.tl(i) * bw.to(i);
+    }
+#pragma unroll
+    for (int e = 0; e < N * N; ++e) rec[R::A + e] = self.v[CondLayout<N, 1>::A + e];
+    LCond<N, 1> res;
+    lane_merge<N, 1>(e0 == 0, LCondViewD<N, 1>{&self}, LCondViewD<N, 1>{&bw}, LCondViewD<N, 1>{&res});
+    self = res;
+  }
+  double* const c = a.shared + lay.oC + (size_t)j * SH::cond;
+#pragma unroll
+  for (int i = 0; i < N; ++i) {
+#pragma unroll
+    for (int k = 0; k < N; ++k) {
+      c[SH::cA + i * N + k] = self.A(i, k);
+      if (k <= i) c[SH::cL + tri(i, k)] = self.L(i, k);
+    }
+    c[SH::ctl + i] = self.tl(i);
+    c[SH::cto + i] = self.to(i);
+  }
+}
+#endif
+
+// One step of the means: m and the running conditional's noise mean r, from
+// the step's record.
+template <int N, int D, int TPL>
+__device__ __forceinline__ void lml_mean_step(const pdq_config& cfg, const double* prm, int q0, const double* rec,
+                                              bool ident, double* m, double* r) {
+  constexpr int MC = D * (1 + TPL);
+  using R = LmlRec<N>;
+  double tmp[N * MC], Pm[N * MC], b[MC], mv[N * MC];
+#pragma unroll
+  for (int i = 0; i < N; ++i)
+#pragma unroll
+    for (int c = 0; c < MC; ++c) {
+      double acc = 0.0;
+#pragma unroll
+      for (int k = 0; k < N; ++k) {
+        const double av = lane_iwp_a<N>(i, k);
+        if (av != 0.0) acc += av * (rec[R::PI + k] * m[k * MC + c]);
+      }
+      tmp[i * MC + c] = acc + 0.0;
+      // rounded here: the value alone and the value with a gradient fuse alike
+      Pm[i * MC + c] = wave_rounded(rec[R::P + i] * tmp[i * MC + c]);
+    }
+  lane_lml_linearize<N, D, TPL>(cfg, prm, q0, Pm, rec[R::t], b);
+#pragma unroll
+  for (int i = 0; i < N; ++i)
+#pragma unroll
+    for (int c = 0; c < MC; ++c) {
+      double acc = 0.0;
+#pragma unroll
+      for (int k = 0; k < N; ++k) acc += rec[R::G + i * N + k] * tmp[k * MC + c];
+      mv[i * MC + c] = rec[R::T + i] * fma(rec[R::PI + i], m[i * MC + c], -acc);
+    }
+  if (ident) {
+#pragma unroll
+    for (int e = 0; e < N * MC; ++e) r[e] = mv[e];
+  } else {
+#pragma unroll
+    for (int i = 0; i < N; ++i)
+#pragma unroll
+      for (int c = 0; c < MC; ++c) {
+        double acc = 0.0;
+#pragma unroll
+        for (int k = 0; k < N; ++k) acc += rec[R::A + i * N + k] * mv[k * MC + c];
+        r[i * MC + c] = acc + r[i * MC + c];
+      }
+  }
+#pragma unroll
+  for (int c = 0; c < MC; ++c) {
+    const double mo = Pm[1 * MC + c] + b[c];
+#pragma unroll
+    for (int i = 0; i < N; ++i) m[i * MC + c] = Pm[i * MC + c] - rec[R::gain + i] * mo;
+  }
+}
+
+// A step's record in registers, read a step ahead of its use.
+template <int N>
+struct LmlRegs {
+  double v[LmlRec<N>::size];
+  __device__ __forceinline__ void load(const double* rec) {
+#pragma unroll
+    for (int e = 0; e < LmlRec<N>::size; ++e) v[e] = rec[e];
+  }
+};
+
+// A vector field's parameters in registers (no field of two components reads
+// more than four).
+struct LmlParams {
+  double v[8];
+  __device__ __forceinline__ LmlParams(const double* p, int n) {
+#pragma unroll
+    for (int q = 0; q < 8; ++q) v[q] = q < n ? p[q] : 0.0;
+  }
+};
+
+#ifndef PDQ_HOST_EMU
+// A tile of records on its way to LDS.
+template <int N>
+struct LmlStage {
+  static constexpr int n = kLmlTile * LmlRec<N>::size, per = (n + 63) / 64;
+  double v[per];
+  __device__ __forceinline__ void load(const double* __restrict__ shared, int s0, int K) {
+    const int count = (K - 1 - s0 < kLmlTile ? K - 1 - s0 : kLmlTile) * LmlRec<N>::size;
+#pragma unroll
+    for (int q = 0; q < per; ++q) {
+      const int e = q * 64 + (int)threadIdx.x;
+      if (e < count) v[q] = shared[(size_t)s0 * LmlRec<N>::size + e];
+    }
+  }
+  __device__ __forceinline__ void store(double* lds) const {
+#pragma unroll
+    for (int q = 0; q < per; ++q) {
+      const int e = q * 64 + (int)threadIdx.x;
+      if (e < n) lds[e] = v[q];
+    }
+  }
+};
+
+// The forward pass of a lane's means: `at_step(s, m)` before every step s,
+// `at_node(j, r)` with interval j's noise mean after its last step.
+template <int N, int D, int TPL, class S, class F>
+__device__ __forceinline__ void lml_means_pass(const LmlArgs& a, const pdq_config& cfg, const double* prm, int q0,
+                                               double* lds, double* m, S&& at_step, F&& at_node) {
+  constexpr int MC = D * (1 + TPL);
+  const int K = a.K, every = a.every;
+  double r[N * MC];
+#pragma unroll
+  for (int e = 0; e < N * MC; ++e) r[e] = 0.0;
+  int in = 0, j = 0;  // the step's place in its interval; the interval
+  LmlStage<N> st;
+  st.load(a.shared, 0, K);
+  for (int s0 = 0; s0 < K - 1; s0 += kLmlTile) {
+    Grp<64>{}.sync();
+    st.store(lds);
+    Grp<64>{}.sync();
+    if (s0 + kLmlTile < K - 1) st.load(a.shared, s0 + kLmlTile, K);
+    const int n = K - 1 - s0 < kLmlTile ? K - 1 - s0 : kLmlTile;
+    auto step = [&](int i, const LmlRegs<N>& now, LmlRegs<N>& next) {
+      next.load(lds + (i + 1 < n ? i + 1 : i) * LmlRec<N>::size);
+      PDQ_PHASE_BOUNDARY();
+      at_step(s0 + i, m);
+      lml_mean_step<N, D, TPL>(cfg, prm, q0, now.v, in == 0, m, r);
+      if (++in == every) {
+        at_node(j, r);
+        in = 0;
+        ++j;
+      }
+    };
+    LmlRegs<N> ra, rb;
+    ra.load(lds);
+    for (int i = 0; i < n; i += 2) {
+      step(i, ra, rb);
+      if (i + 1 < n) step(i + 1, rb, ra);
+    }
+  }
+}
+
+// The arguments with what an instantiation knows: the vector field is one of
+// them, so that a step does not choose among the fields for every component.
+__device__ __forceinline__ LmlArgs lml_shared_args(const LmlArgs& args, int field) {
+  LmlArgs a = args;
+  a.cfg.strategy = PDQ_FIXEDPOINT;
+  a.cfg.solver = PDQ_SOLVER;
+  a.cfg.constraint = PDQ_TS0;
+  a.cfg.re_linearize_after_calibration = 0;
+  a.cfg.vector_field = field;
+  return a;
+}
+
+// A lane per (instance, tangent group): means, reverse scan, outputs.  A lane
+// beyond the last one computes it again and writes nothing.
+template <int N, int D, int TPL, int FIELD>
+__global__ void __launch_bounds__(64) lml_means_kernel(LmlArgs args) {
+  constexpr int MC = D * (1 + TPL);
+  using SH = LmlShared<N>;
+  __shared__ double lds[LmlStage<N>::n];
+  LmlArgs a = lml_shared_args(args, FIELD);
+  const size_t n_lanes = (size_t)a.n_inst * a.G, gl = (size_t)blockIdx.x * 64 + threadIdx.x;
+  const bool active = gl < n_lanes;
+  const size_t lane = active ? gl : n_lanes - 1;
+  const int inst = (int)(lane / a.G), g = (int)(lane % a.G), q0 = g * TPL, ntan = a.n_tan;
+  const LmlParams params(a.params + (size_t)inst * a.cfg.n_params, a.cfg.n_params);
+  const double* const prm = params.v;
+  const double* const tc = a.tcoeffs + (size_t)inst * N * D * (1 + ntan);
+  double m[N * MC];
+#pragma unroll
+  for (int i = 0; i < N; ++i)
+#pragma unroll
+    for (int k = 0; k < D; ++k) {
+      m[i * MC + k] = tc[(i * D + k) * (1 + ntan)];
+#pragma unroll
+      for (int tt = 0; tt < TPL; ++tt) m[i * MC + (1 + tt) * D + k] = tc[(i * D + k) * (1 + ntan) + 1 + q0 + tt];
+    }
+  lml_means_pass<N, D, TPL>(
+      a, a.cfg, prm, q0, lds, m, [](int, const double*) {},
+      [&](int j, const double* r) {
+        if (active)
+#pragma unroll
+          for (int e = 0; e < N * MC; ++e) a.scratch[((size_t)j * N * MC + e) * n_lanes + lane] = r[e];
+      });
+  if (!active) return;
+  const SH lay(a.K, a.every);
+  double XL[N * N];
+  const double* const fin = a.shared + lay.oF + (size_t)(a.K - 1) * SH::fac;
+#pragma unroll
+  for (int e = 0; e < N * N; ++e) XL[e] = e % N <= e / N ? fin[tri(e / N, e % N)] : 0.0;
+  lane_lml_scan<N, D, TPL>(a, inst, g, m, XL, [&](int j) {
+    return LmlCond<N, MC>{a.shared + lay.oC + (size_t)j * SH::cond, a.scratch + (size_t)j * N * MC * n_lanes + lane,
+                          n_lanes};
+  });
+}
+#endif
+
+// The adjoint's storage per lane (doubles): interval means, node data,
+// adjoints of the interval means, checkpoints of the mean.
+template <int N, int D>
+struct LmlAdjShared {
+  static constexpr int node = N + 1 + D;
+  size_t means, nodes, xibar, ckpt, size;
+  __host__ __device__ LmlAdjShared(int K, int every) {
+    const size_t kobs = (size_t)(K - 1) / every + 1;
+    means = 0;
+    nodes = means + (kobs - 1) * N * D;
+    xibar = nodes + kobs * node;
+    ckpt = xibar + (kobs - 1) * N * D;
+    size = ckpt + ((size_t)(K - 2) / kLmlTile + 1) * N * D;
+  }
+};
+
+#ifndef PDQ_HOST_EMU
+// A lane per instance: means with a checkpoint per tile, reverse scan, its
+// adjoint, and the tiles backwards (a tile's means from its checkpoint into
+// the lane's column of LDS, then its steps' adjoints).
+template <int N, int D, int FIELD>
+__global__ void __launch_bounds__(64) lml_adjoint_kernel(LmlArgs args) {
+  using R = LmlRec<N>;
+  using SH = LmlShared<N>;
+  constexpr int ND = N * D;
+  __shared__ double lds[LmlStage<N>::n];
+  __shared__ double means[kLmlTile * ND * 64];
+  LmlArgs a = lml_shared_args(args, FIELD);
+  const int K = a.K, every = a.every, ntan = a.n_tan;
+  const size_t n_lanes = (size_t)gridDim.x * 64, lane = (size_t)blockIdx.x * 64 + threadIdx.x;
+  const bool active = lane < (size_t)a.n_inst;
+  const int inst = active ? (int)lane : a.n_inst - 1;
+  const LmlParams params(a.params + (size_t)inst * a.cfg.n_params, a.cfg.n_params);
+  const double* const prm = params.v;
+  const double* const tc = a.tcoeffs + (size_t)inst * ND * (1 + ntan);
+  const SH lay(K, every);
+  const LmlAdjShared<N, D> own(K, every);
+  auto at = [&](size_t off) -> double* { return a.scratch + off * n_lanes + lane; };
+  double m[ND];
+#pragma unroll
+  for (int e = 0; e < ND; ++e) m[e] = tc[e * (1 + ntan)];
+  lml_means_pass<N, D, 0>(
+      a, a.cfg, prm, 0, lds, m,
+      [&](int s, const double* x) {
+        if (s % kLmlTile == 0) {
+          double* const c = at(own.ckpt + (size_t)(s / kLmlTile) * ND);
+#pragma unroll
+          for (int e = 0; e < ND; ++e) c[(size_t)e * n_lanes] = x[e];
+        }
+      },
+      [&](int j, const double* r) {
+        double* const c = at(own.means + (size_t)j * ND);
+#pragma unroll
+        for (int e = 0; e < ND; ++e) c[(size_t)e * n_lanes] = r[e];
+      });
+  double XL[N * N];
+  const double* const fin = a.shared + lay.oF + (size_t)(K - 1) * SH::fac;
+#pragma unroll
+  for (int e = 0; e < N * N; ++e) XL[e] = e % N <= e / N ? fin[tri(e / N, e % N)] : 0.0;
+  auto cond = [&](int j) {
+    return LmlCond<N, D>{a.shared + lay.oC + (size_t)j * SH::cond, at(own.means + (size_t)j * ND), n_lanes};
+  };
+  auto node = [&](int j) { return at(own.nodes + (size_t)j * LmlAdjShared<N, D>::node); };
+  const double lp = adj_scan<N, D>(a, inst, m, XL, n_lanes, cond, node);
+  if (a.value && active) a.value[inst] = lp;
+  if (!a.grad) return;
+  double mbar[ND], cbar[ND], tbar[8];
+  adj_scan_adjoint<N, D>(a, n_lanes, cond, node, [&](int j) { return at(own.xibar + (size_t)j * ND); }, mbar);
+  // (every divides the grid's steps: the terminal marginal stands behind an identity)
+#pragma unroll
+  for (int e = 0; e < ND; ++e) cbar[e] = 0.0;
+#pragma unroll
+  for (int q = 0; q < 8; ++q) tbar[q] = 0.0;
+  const int np = a.cfg.n_params < 8 ? a.cfg.n_params : 8;
+  struct Self {
+    const double* rec;
+    __device__ double tl(int) const { return 1.0; }  // (T holds both scales)
+    __device__ double A(int i, int k) const { return rec[R::A + i * N + k]; }
+  };
+  double* const mine = means + threadIdx.x;
+  LmlStage<N> st;
+  double ck[ND];
+  auto fetch = [&](int s0) {
+    st.load(a.shared, s0, K);
+    const double* const c = at(own.ckpt + (size_t)(s0 / kLmlTile) * ND);
+#pragma unroll
+    for (int e = 0; e < ND; ++e) ck[e] = c[(size_t)e * n_lanes];
+  };
+  int in = 0, j = (K - 1) / every;  // the place of the step after the current one in its interval, that interval
+  const int last = (K - 2) / kLmlTile * kLmlTile;
+  fetch(last);
+  for (int s0 = last; s0 >= 0; s0 -= kLmlTile) {
+    Grp<64>{}.sync();
+    st.store(lds);
+    Grp<64>{}.sync();
+#pragma unroll
+    for (int e = 0; e < ND; ++e) m[e] = ck[e];
+    if (s0 > 0) fetch(s0 - kLmlTile);
+    const int n = K - 1 - s0 < kLmlTile ? K - 1 - s0 : kLmlTile;
+    double r[ND];
+#pragma unroll
+    for (int e = 0; e < ND; ++e) r[e] = 0.0;
+    LmlRegs<N> ra, rb;
+    auto again = [&](int i, const LmlRegs<N>& now, LmlRegs<N>& next) {
+      next.load(lds + (i + 1 < n ? i + 1 : i) * R::size);
+      PDQ_PHASE_BOUNDARY();
+#pragma unroll
+      for (int e = 0; e < ND; ++e) mine[(i * ND + e) * 64] = m[e];
+      lml_mean_step<N, D, 0>(a.cfg, prm, 0, now.v, true, m, r);  // (r is not used)
+    };
+    ra.load(lds);
+    for (int i = 0; i < n; i += 2) {  // (the last step's result is not used)
+      again(i, ra, rb);
+      if (i + 1 < n) again(i + 1, rb, ra);
+    }
+    auto back = [&](int i, const LmlRegs<N>& now, LmlRegs<N>& next) {
+      const double* const rec = now.v;
+      next.load(lds + (i > 0 ? i - 1 : 0) * R::size);
+      PDQ_PHASE_BOUNDARY();
+      if (in == 0) {
+        // after this step a reset stored the running conditional as interval
+        // j - 1's: its adjoint comes from the scan
+        --j;
+        in = every;
+        const double* const xb = at(own.xibar + (size_t)j * ND);
+#pragma unroll
+        for (int e = 0; e < ND; ++e) cbar[e] = xb[(size_t)e * n_lanes];
+      }
+      --in;
+      double Pm[D];
+#pragma unroll
+      for (int c = 0; c < D; ++c) {
+        double acc = 0.0;
+#pragma unroll
+        for (int k = 0; k < N; ++k) acc += lane_iwp_a<N>(0, k) * (rec[R::PI + k] * mine[(i * ND + k * D + c) * 64]);
+        Pm[c] = rec[R::P] * (acc + 0.0);
+      }
+      adj_back_step<N, D>(a.cfg, prm, np, rec + R::P, rec + R::PI, rec + R::G, rec + R::T, rec + R::gain, Pm, in == 0,
+                          Self{rec}, mbar, cbar, tbar);
+    };
+    ra.load(lds + (n - 1) * R::size);
+    for (int i = n - 1; i >= 0; i -= 2) {
+      back(i, ra, rb);
+      if (i > 0) back(i - 1, rb, ra);
+    }
+  }
+  for (int q = 0; q < ntan; ++q) {
+    double g = 0.0;
+#pragma unroll
+    for (int e = 0; e < 8; ++e) g = e == q && q < np ? tbar[e] : g;
+#pragma unroll
+    for (int e = 0; e < ND; ++e) g += mbar[e] * tc[(size_t)e * (1 + ntan) + 1 + q];
+    if (active) a.grad[(size_t)inst * ntan + q] = g;
+  }
+}
+#endif
+
+}  // namespace pdq
