@@ -8,28 +8,30 @@
 // (pdq_lane_lml.h, pdq_lane_adjoint.h) compute them in every lane of every
 // instance and tangent, in one serial chain of 9 400 cycles per grid step, and
 // the adjoint once more on its way back.  Here
-//  1. lml_chain_kernel: one wavefront runs the factors' own chain, the
-//     prediction's R_Y and the update (2 400 cycles per step; its lanes take 64
-//     steps' preconditioners at once), and leaves each step's factor and gain;
-//  2. lml_revert_kernel: one lane per step, the backward conditional's gain
-//     and factor;
-//  3. lml_merge_kernel: one lane per observation interval, the fixed-point
-//     merges (estimators_and_losses.py:473-591) of its steps;
-//  4. lml_means_kernel / lml_adjoint_kernel: one lane per instance (and tangent
-//     group), the means' recursion through those factors, the reverse scan
-//     (whose factors depend on the instance's observation stds) and the
-//     adjoint, which recomputes a segment's means from a checkpoint.
+//  1. lml_chain: one wavefront runs the factors' own chain, the prediction's R_Y
+//     and the update (2 400 cycles per step; its lanes take 64 steps'
+//     preconditioners at once), and leaves each step's factor and gain;
+//  2. lml_revert: one lane per step, the backward conditional's gain and factor;
+//  3. lml_merge: one lane per observation interval, the fixed-point merges
+//     (estimators_and_losses.py:473-591) of its steps;
+//  4. lml_means_part: one lane per instance (and tangent group), the means'
+//     recursion through those factors, then the reverse scan (whose factors
+//     depend on the instance's observation stds); lml_adjoint_kernel: the scan
+//     and the adjoint, which recomputes a tile's means from a checkpoint.
+// The grid is cut into chunks of whole intervals, and a launch runs the four
+// parts on four successive chunks (lml_parts_kernel): the chain, which leaves
+// the chip idle, runs beside the lanes' means.
 // What the means' pass reads of a step is the same for every lane: a tile of
 // steps is staged in LDS by the wavefront, the next tile's loads under way.
 // The order of operations is the lane kernels'; against 64-bit arithmetic in
 // another order both gradients' errors are 3e-14 on average (nu = 3, 4; 64 to
 // 2000 steps).
 //
-// 1024 instances, nu = 3, 2000 steps, 101 observations: value 7.29 -> 3.31 ms,
-// with the gradient by tangents 7.82 -> 4.46 ms (chain 2.03, means 2.27), by the
-// adjoint 18.2 -> 5.28 ms (chain 2.03, means and adjoint 3.1); 300 instances,
-// nu = 4, 500 steps: 4.63 -> 1.68 and 10.95 -> 2.13 ms.  The chain and the
-// means' pass are bound by one wavefront's instruction issue.
+// 1024 instances, nu = 3, 2000 steps, 101 observations: value 7.29 -> 2.51 ms,
+// with the gradient by tangents 7.82 -> 2.78 ms (4.46 with the chain, 2.03, before
+// the means, 2.27), by the adjoint 18.2 -> 4.49 ms (5.28); 300 instances, nu = 4,
+// 500 steps: 4.63 -> 1.53 and 10.97 -> 1.87 ms.  The chain and the means' pass are
+// bound by one wavefront's instruction issue.
 #pragma once
 
 #include "pdq_lane_adjoint.h"
@@ -116,24 +118,25 @@ __device__ __forceinline__ void lml_chain_step(const pdq_config& cfg, const doub
 }
 
 #ifndef PDQ_HOST_EMU
+// The factors' chain from step b to step e (one wavefront; the factor before a
+// later step than the first is where the previous call left it).
 template <int N>
-__global__ void __launch_bounds__(64) lml_chain_kernel(LmlArgs a) {
+__device__ __forceinline__ void lml_chain(const LmlArgs& a, const pdq_config& cfg, int b, int e, double* pre) {
   constexpr int ps = 2 * N + 2;
   using R = LmlRec<N>;
   using SH = LmlShared<N>;
-  __shared__ double pre[64 * ps];
-  pdq_config cfg = a.cfg;
-  cfg.constraint = PDQ_TS0;
   const SH lay(a.K, a.every);
   double* const rec = a.shared;
   double* const fac = a.shared + lay.oF;
-  double L[N * N], Q[N * N], t = a.times[0];
+  double L[N * N], Q[N * N], t = b == 0 ? a.times[0] : rec[(size_t)(b - 1) * R::size + R::t];
 #pragma unroll
-  for (int e = 0; e < N * N; ++e) {
-    const int i = e / N;
-    L[e] = i == e % N ? (cfg.init_std_rows ? cfg.init_std_rows[i] : cfg.init_std) : 0.0;
-    Q[e] = a.Q[e];
-  }
+  for (int i = 0; i < N; ++i)
+#pragma unroll
+    for (int j = 0; j < N; ++j) {
+      if (b == 0) L[i * N + j] = i == j ? (cfg.init_std_rows ? cfg.init_std_rows[i] : cfg.init_std) : 0.0;
+      else L[i * N + j] = j <= i ? fac[(size_t)b * SH::fac + tri(i, j)] : 0.0;
+      Q[i * N + j] = a.Q[i * N + j];
+    }
   auto put = [&](int s) {
     if (threadIdx.x == 0) {
 #pragma unroll
@@ -142,9 +145,9 @@ __global__ void __launch_bounds__(64) lml_chain_kernel(LmlArgs a) {
         for (int j = 0; j <= i; ++j) fac[(size_t)s * SH::fac + tri(i, j)] = L[i * N + j];
     }
   };
-  for (int c0 = 0; c0 < a.K - 1; c0 += 64) {
+  for (int c0 = b; c0 < e; c0 += 64) {
     const int s = c0 + threadIdx.x;
-    if (s < a.K - 1) {
+    if (s < e) {
       double P[N], PI[N];
       const double h = a.times[s + 1] - a.times[s];
       lane_precon<N>(h, P, PI);
@@ -159,11 +162,11 @@ __global__ void __launch_bounds__(64) lml_chain_kernel(LmlArgs a) {
       pre[threadIdx.x * ps + 2 * N + 1] = h;
     }
     Grp<64>{}.sync();
-    const int n = a.K - 1 - c0 < 64 ? a.K - 1 - c0 : 64;
+    const int n = e - c0 < 64 ? e - c0 : 64;
     auto step = [&](int i, const double* now, double* next) {
       double gain[N];
 #pragma unroll
-      for (int e = 0; e < ps; ++e) next[e] = pre[(i + 1 < n ? i + 1 : i) * ps + e];
+      for (int q = 0; q < ps; ++q) next[q] = pre[(i + 1 < n ? i + 1 : i) * ps + q];
       PDQ_PHASE_BOUNDARY();
       put(c0 + i);
       t += now[2 * N + 1];
@@ -171,30 +174,28 @@ __global__ void __launch_bounds__(64) lml_chain_kernel(LmlArgs a) {
       if (threadIdx.x == 0) {
         double* const r = rec + (size_t)(c0 + i) * R::size;
 #pragma unroll
-        for (int e = 0; e < N; ++e) r[R::gain + e] = gain[e];
+        for (int q = 0; q < N; ++q) r[R::gain + q] = gain[q];
         r[R::t] = t;
       }
     };
     double x[ps], y[ps];
 #pragma unroll
-    for (int e = 0; e < ps; ++e) x[e] = pre[e];
+    for (int q = 0; q < ps; ++q) x[q] = pre[q];
     for (int i = 0; i < n; i += 2) {
       step(i, x, y);
       if (i + 1 < n) step(i + 1, y, x);
     }
     Grp<64>{}.sync();
   }
-  put(a.K - 1);
+  put(e);
 }
 
 // Step s's backward conditional from its factor.
 template <int N>
-__global__ void __launch_bounds__(64) lml_revert_kernel(LmlArgs a) {
+__device__ __forceinline__ void lml_revert(const LmlArgs& a, int s) {
   using R = LmlRec<N>;
   using SH = LmlShared<N>;
   const SH lay(a.K, a.every);
-  const int s = blockIdx.x * 64 + threadIdx.x;
-  if (s >= a.K - 1) return;
   double* const rec = a.shared + (size_t)s * R::size;
   double* const fac = a.shared + lay.oF + (size_t)s * SH::fac;
   double P[N], PI[N], Xm[N], XL[N * N], Ym[N], YL[N * N];
@@ -219,12 +220,10 @@ __global__ void __launch_bounds__(64) lml_revert_kernel(LmlArgs a) {
 
 // Interval j's merges, in the order of its steps.
 template <int N>
-__global__ void __launch_bounds__(64) lml_merge_kernel(LmlArgs a) {
+__device__ __forceinline__ void lml_merge(const LmlArgs& a, int j) {
   using R = LmlRec<N>;
   using SH = LmlShared<N>;
   const SH lay(a.K, a.every);
-  const int j = blockIdx.x * 64 + threadIdx.x;
-  if (j >= (a.K - 1) / a.every) return;
   LCond<N, 1> self, bw;
 #pragma unroll
   for (int e = 0; e < CondLayout<N, 1>::size; ++e) self.v[e] = bw.v[e] = 0.0;
@@ -344,8 +343,9 @@ template <int N>
 struct LmlStage {
   static constexpr int n = kLmlTile * LmlRec<N>::size, per = (n + 63) / 64;
   double v[per];
-  __device__ __forceinline__ void load(const double* __restrict__ shared, int s0, int K) {
-    const int count = (K - 1 - s0 < kLmlTile ? K - 1 - s0 : kLmlTile) * LmlRec<N>::size;
+  // the records of steps s0 .. end - 1, at most a tile
+  __device__ __forceinline__ void load(const double* __restrict__ shared, int s0, int end) {
+    const int count = (end - s0 < kLmlTile ? end - s0 : kLmlTile) * LmlRec<N>::size;
 #pragma unroll
     for (int q = 0; q < per; ++q) {
       const int e = q * 64 + (int)threadIdx.x;
@@ -361,25 +361,22 @@ struct LmlStage {
   }
 };
 
-// The forward pass of a lane's means: `at_step(s, m)` before every step s,
+// The means' pass of a lane from step b (an interval's first) to step e: m and
+// the running conditional's noise mean r; `at_step(s, m)` before every step s,
 // `at_node(j, r)` with interval j's noise mean after its last step.
 template <int N, int D, int TPL, class S, class F>
-__device__ __forceinline__ void lml_means_pass(const LmlArgs& a, const pdq_config& cfg, const double* prm, int q0,
-                                               double* lds, double* m, S&& at_step, F&& at_node) {
-  constexpr int MC = D * (1 + TPL);
-  const int K = a.K, every = a.every;
-  double r[N * MC];
-#pragma unroll
-  for (int e = 0; e < N * MC; ++e) r[e] = 0.0;
-  int in = 0, j = 0;  // the step's place in its interval; the interval
+__device__ __forceinline__ void lml_means_pass(const LmlArgs& a, const pdq_config& cfg, const double* prm, int q0, int b,
+                                               int e, double* lds, double* m, double* r, S&& at_step, F&& at_node) {
+  const int every = a.every;
+  int in = 0, j = b / every;  // the step's place in its interval; the interval
   LmlStage<N> st;
-  st.load(a.shared, 0, K);
-  for (int s0 = 0; s0 < K - 1; s0 += kLmlTile) {
+  st.load(a.shared, b, e);
+  for (int s0 = b; s0 < e; s0 += kLmlTile) {
     Grp<64>{}.sync();
     st.store(lds);
     Grp<64>{}.sync();
-    if (s0 + kLmlTile < K - 1) st.load(a.shared, s0 + kLmlTile, K);
-    const int n = K - 1 - s0 < kLmlTile ? K - 1 - s0 : kLmlTile;
+    if (s0 + kLmlTile < e) st.load(a.shared, s0 + kLmlTile, e);
+    const int n = e - s0 < kLmlTile ? e - s0 : kLmlTile;
     auto step = [&](int i, const LmlRegs<N>& now, LmlRegs<N>& next) {
       next.load(lds + (i + 1 < n ? i + 1 : i) * LmlRec<N>::size);
       PDQ_PHASE_BOUNDARY();
@@ -412,38 +409,78 @@ __device__ __forceinline__ LmlArgs lml_shared_args(const LmlArgs& args, int fiel
   return a;
 }
 
-// A lane per (instance, tangent group): means, reverse scan, outputs.  A lane
-// beyond the last one computes it again and writes nothing.
-template <int N, int D, int TPL, int FIELD>
-__global__ void __launch_bounds__(64) lml_means_kernel(LmlArgs args) {
+#endif
+
+// The adjoint's storage per lane (doubles): interval means, node data,
+// adjoints of the interval means, checkpoints of the mean.
+template <int N, int D>
+struct LmlAdjShared {
+  static constexpr int node = N + 1 + D;
+  size_t means, nodes, xibar, ckpt, state, size;
+  __host__ __device__ LmlAdjShared(int K, int every) {
+    const size_t kobs = (size_t)(K - 1) / every + 1;
+    means = 0;
+    nodes = means + (kobs - 1) * N * D;
+    xibar = nodes + kobs * node;
+    ckpt = xibar + (kobs - 1) * N * D;
+    state = ckpt + ((size_t)(K - 2) / kLmlTile + 1) * N * D;  // m and r between two launches
+    size = state + 2 * N * D;
+  }
+};
+
+#ifndef PDQ_HOST_EMU
+// What one launch does, each part on blocks of its own: the chain of steps
+// c0 .. c1, the reverts of steps r0 .. r1, the merges of intervals j0 .. j1 and
+// the means' pass of steps m0 .. m1.  A launch's parts work on four successive
+// chunks of the grid, so that the chain, one wavefront, runs beside the lanes'
+// means; what a part reads was written by earlier launches.
+struct LmlParts {
+  int c0, c1, r0, r1, j0, j1, m0, m1;
+  __host__ __device__ int reverts() const { return (r1 - r0 + 63) / 64; }
+  __host__ __device__ int merges() const { return (j1 - j0 + 63) / 64; }
+};
+
+// The means' pass of a lane per (instance, tangent group) and, after the last
+// step, the reverse scan and the outputs.  A lane beyond the last one computes
+// it again and writes nothing.
+template <int N, int D, int TPL>
+__device__ __forceinline__ void lml_means_part(const LmlArgs& a, const LmlParts& w, int block, double* lds) {
   constexpr int MC = D * (1 + TPL);
   using SH = LmlShared<N>;
-  __shared__ double lds[LmlStage<N>::n];
-  LmlArgs a = lml_shared_args(args, FIELD);
-  const size_t n_lanes = (size_t)a.n_inst * a.G, gl = (size_t)blockIdx.x * 64 + threadIdx.x;
+  const size_t n_lanes = (size_t)a.n_inst * a.G, gl = (size_t)block * 64 + threadIdx.x;
   const bool active = gl < n_lanes;
   const size_t lane = active ? gl : n_lanes - 1;
   const int inst = (int)(lane / a.G), g = (int)(lane % a.G), q0 = g * TPL, ntan = a.n_tan;
   const LmlParams params(a.params + (size_t)inst * a.cfg.n_params, a.cfg.n_params);
   const double* const prm = params.v;
   const double* const tc = a.tcoeffs + (size_t)inst * N * D * (1 + ntan);
-  double m[N * MC];
+  double* const state = a.scratch + (size_t)((a.K - 1) / a.every) * N * MC * n_lanes + lane;
+  double m[N * MC], r[N * MC];
 #pragma unroll
   for (int i = 0; i < N; ++i)
 #pragma unroll
-    for (int k = 0; k < D; ++k) {
-      m[i * MC + k] = tc[(i * D + k) * (1 + ntan)];
-#pragma unroll
-      for (int tt = 0; tt < TPL; ++tt) m[i * MC + (1 + tt) * D + k] = tc[(i * D + k) * (1 + ntan) + 1 + q0 + tt];
+    for (int c = 0; c < MC; ++c) {
+      const int tt = c / D - 1, k = c % D, e = i * MC + c;
+      if (w.m0 == 0) m[e] = tc[(i * D + k) * (1 + ntan) + (tt < 0 ? 0 : 1 + q0 + tt)];
+      else m[e] = state[(size_t)e * n_lanes];
+      r[e] = w.m0 == 0 ? 0.0 : state[(size_t)(N * MC + e) * n_lanes];
     }
   lml_means_pass<N, D, TPL>(
-      a, a.cfg, prm, q0, lds, m, [](int, const double*) {},
-      [&](int j, const double* r) {
+      a, a.cfg, prm, q0, w.m0, w.m1, lds, m, r, [](int, const double*) {},
+      [&](int j, const double* x) {
         if (active)
 #pragma unroll
-          for (int e = 0; e < N * MC; ++e) a.scratch[((size_t)j * N * MC + e) * n_lanes + lane] = r[e];
+          for (int e = 0; e < N * MC; ++e) a.scratch[((size_t)j * N * MC + e) * n_lanes + lane] = x[e];
       });
   if (!active) return;
+  if (w.m1 < a.K - 1) {
+#pragma unroll
+    for (int e = 0; e < N * MC; ++e) {
+      state[(size_t)e * n_lanes] = m[e];
+      state[(size_t)(N * MC + e) * n_lanes] = r[e];
+    }
+    return;
+  }
   const SH lay(a.K, a.every);
   double XL[N * N];
   const double* const fin = a.shared + lay.oF + (size_t)(a.K - 1) * SH::fac;
@@ -454,28 +491,77 @@ __global__ void __launch_bounds__(64) lml_means_kernel(LmlArgs args) {
                           n_lanes};
   });
 }
-#endif
 
-// The adjoint's storage per lane (doubles): interval means, node data,
-// adjoints of the interval means, checkpoints of the mean.
+// The adjoint's: a lane per instance, with a checkpoint per tile; the mean
+// after the last step is left in the state.
 template <int N, int D>
-struct LmlAdjShared {
-  static constexpr int node = N + 1 + D;
-  size_t means, nodes, xibar, ckpt, size;
-  __host__ __device__ LmlAdjShared(int K, int every) {
-    const size_t kobs = (size_t)(K - 1) / every + 1;
-    means = 0;
-    nodes = means + (kobs - 1) * N * D;
-    xibar = nodes + kobs * node;
-    ckpt = xibar + (kobs - 1) * N * D;
-    size = ckpt + ((size_t)(K - 2) / kLmlTile + 1) * N * D;
+__device__ __forceinline__ void lml_means_part_adjoint(const LmlArgs& a, const LmlParts& w, int block, int blocks,
+                                                       double* lds) {
+  constexpr int ND = N * D;
+  const size_t n_lanes = (size_t)blocks * 64, lane = (size_t)block * 64 + threadIdx.x;
+  const int inst = lane < (size_t)a.n_inst ? (int)lane : a.n_inst - 1;
+  const LmlParams params(a.params + (size_t)inst * a.cfg.n_params, a.cfg.n_params);
+  const double* const tc = a.tcoeffs + (size_t)inst * ND * (1 + a.n_tan);
+  const LmlAdjShared<N, D> own(a.K, a.every);
+  auto at = [&](size_t off) -> double* { return a.scratch + off * n_lanes + lane; };
+  double* const state = at(own.state);
+  double m[ND], r[ND];
+#pragma unroll
+  for (int e = 0; e < ND; ++e) {
+    m[e] = w.m0 == 0 ? tc[e * (1 + a.n_tan)] : state[(size_t)e * n_lanes];
+    r[e] = w.m0 == 0 ? 0.0 : state[(size_t)(ND + e) * n_lanes];
   }
-};
+  lml_means_pass<N, D, 0>(
+      a, a.cfg, params.v, 0, w.m0, w.m1, lds, m, r,
+      [&](int s, const double* x) {
+        if (s % kLmlTile == 0) {
+          double* const c = at(own.ckpt + (size_t)(s / kLmlTile) * ND);
+#pragma unroll
+          for (int e = 0; e < ND; ++e) c[(size_t)e * n_lanes] = x[e];
+        }
+      },
+      [&](int j, const double* x) {
+        double* const c = at(own.means + (size_t)j * ND);
+#pragma unroll
+        for (int e = 0; e < ND; ++e) c[(size_t)e * n_lanes] = x[e];
+      });
+#pragma unroll
+  for (int e = 0; e < ND; ++e) {
+    state[(size_t)e * n_lanes] = m[e];
+    state[(size_t)(ND + e) * n_lanes] = r[e];
+  }
+}
 
-#ifndef PDQ_HOST_EMU
-// A lane per instance: means with a checkpoint per tile, reverse scan, its
-// adjoint, and the tiles backwards (a tile's means from its checkpoint into
-// the lane's column of LDS, then its steps' adjoints).
+template <int N, int D, int TPL, int FIELD, bool ADJOINT>
+__global__ void __launch_bounds__(64) lml_parts_kernel(LmlArgs args, LmlParts w) {
+  constexpr int lp = 64 * (2 * N + 2), ls = LmlStage<N>::n;
+  __shared__ double lds[lp > ls ? lp : ls];
+  const LmlArgs a = lml_shared_args(args, FIELD);
+  int b = blockIdx.x;
+  if (b == 0) {
+    if (w.c0 < w.c1) lml_chain<N>(a, a.cfg, w.c0, w.c1, lds);
+    return;
+  }
+  b -= 1;
+  if (b < w.reverts()) {
+    const int s = w.r0 + b * 64 + (int)threadIdx.x;
+    if (s < w.r1) lml_revert<N>(a, s);
+    return;
+  }
+  b -= w.reverts();
+  if (b < w.merges()) {
+    const int j = w.j0 + b * 64 + (int)threadIdx.x;
+    if (j < w.j1) lml_merge<N>(a, j);
+    return;
+  }
+  b -= w.merges();
+  if constexpr (ADJOINT) lml_means_part_adjoint<N, D>(a, w, b, (int)gridDim.x - 1 - w.reverts() - w.merges(), lds);
+  else lml_means_part<N, D, TPL>(a, w, b, lds);
+}
+
+// A lane per instance, after the means' pass: reverse scan, its adjoint, and
+// the tiles backwards (a tile's means from its checkpoint into the lane's
+// column of LDS, then its steps' adjoints).
 template <int N, int D, int FIELD>
 __global__ void __launch_bounds__(64) lml_adjoint_kernel(LmlArgs args) {
   using R = LmlRec<N>;
@@ -483,7 +569,7 @@ __global__ void __launch_bounds__(64) lml_adjoint_kernel(LmlArgs args) {
   constexpr int ND = N * D;
   __shared__ double lds[LmlStage<N>::n];
   __shared__ double means[kLmlTile * ND * 64];
-  LmlArgs a = lml_shared_args(args, FIELD);
+  const LmlArgs a = lml_shared_args(args, FIELD);
   const int K = a.K, every = a.every, ntan = a.n_tan;
   const size_t n_lanes = (size_t)gridDim.x * 64, lane = (size_t)blockIdx.x * 64 + threadIdx.x;
   const bool active = lane < (size_t)a.n_inst;
@@ -496,21 +582,7 @@ __global__ void __launch_bounds__(64) lml_adjoint_kernel(LmlArgs args) {
   auto at = [&](size_t off) -> double* { return a.scratch + off * n_lanes + lane; };
   double m[ND];
 #pragma unroll
-  for (int e = 0; e < ND; ++e) m[e] = tc[e * (1 + ntan)];
-  lml_means_pass<N, D, 0>(
-      a, a.cfg, prm, 0, lds, m,
-      [&](int s, const double* x) {
-        if (s % kLmlTile == 0) {
-          double* const c = at(own.ckpt + (size_t)(s / kLmlTile) * ND);
-#pragma unroll
-          for (int e = 0; e < ND; ++e) c[(size_t)e * n_lanes] = x[e];
-        }
-      },
-      [&](int j, const double* r) {
-        double* const c = at(own.means + (size_t)j * ND);
-#pragma unroll
-        for (int e = 0; e < ND; ++e) c[(size_t)e * n_lanes] = r[e];
-      });
+  for (int e = 0; e < ND; ++e) m[e] = at(own.state)[(size_t)e * n_lanes];
   double XL[N * N];
   const double* const fin = a.shared + lay.oF + (size_t)(K - 1) * SH::fac;
 #pragma unroll
@@ -539,7 +611,7 @@ __global__ void __launch_bounds__(64) lml_adjoint_kernel(LmlArgs args) {
   LmlStage<N> st;
   double ck[ND];
   auto fetch = [&](int s0) {
-    st.load(a.shared, s0, K);
+    st.load(a.shared, s0, K - 1);
     const double* const c = at(own.ckpt + (size_t)(s0 / kLmlTile) * ND);
 #pragma unroll
     for (int e = 0; e < ND; ++e) ck[e] = c[(size_t)e * n_lanes];

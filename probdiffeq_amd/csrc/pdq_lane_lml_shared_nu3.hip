@@ -23,7 +23,8 @@ size_t lml_shared_scratch(int N, int D, int tpl, int K, int every, int n_inst, i
     const size_t lanes = (size_t)((n_inst + 63) / 64) * 64;
     return (N == 4 ? LmlAdjShared<4, 2>(K, every).size : LmlAdjShared<5, 2>(K, every).size) * lanes;
   }
-  return (size_t)((K - 1) / every) * N * D * (1 + tpl) * n_inst * G;
+  // an interval's noise mean per interval; m and r between two launches
+  return ((size_t)((K - 1) / every) + 2) * N * D * (1 + tpl) * n_inst * G;
 }
 
 int launch_lml_shared(LmlArgs& a, int N, int D, int tpl, bool reverse, hipStream_t st) {
