@@ -28,9 +28,10 @@
 // 2000 steps).
 //
 // 1024 instances, nu = 3, 2000 steps, 101 observations: value 7.29 -> 2.51 ms,
-// with the gradient by tangents 7.82 -> 2.78 ms (4.46 with the chain, 2.03, before
-// the means, 2.27), by the adjoint 18.2 -> 4.49 ms (5.28); 300 instances, nu = 4,
-// 500 steps: 4.63 -> 1.53 and 10.97 -> 1.87 ms.  The chain and the means' pass are
+// with the gradient by tangents 7.82 -> 2.68 ms (4.46 with the chain, 2.03, before
+// the means, 2.27), by the adjoint 18.2 -> 4.05 ms (5.28;
+// 4.49 with the tiles' means recomputed by the wavefront that walks back); 300 instances, nu = 4,
+// 500 steps: 4.61 -> 1.49 and 10.95 -> 1.69 ms.  The chain and the means' pass are
 // bound by one wavefront's instruction issue.
 #pragma once
 
@@ -40,7 +41,10 @@
 
 namespace pdq {
 
-constexpr int kLmlTile = 16;  // grid steps staged at once, and per checkpoint of the adjoint
+// Grid steps staged at once, and per checkpoint of the adjoint (whose two tiles
+// of means, and two of records, fit the 160 KB of LDS).
+template <int N>
+constexpr int lml_tile = N == 4 ? 16 : 12;
 
 // What a step's mean recursion needs of the factors (doubles): P, PI, the
 // update's gain, the merge's T = tl_self o to_b (behind an identity: to_b), the
@@ -341,21 +345,21 @@ struct LmlParams {
 // A tile of records on its way to LDS.
 template <int N>
 struct LmlStage {
-  static constexpr int n = kLmlTile * LmlRec<N>::size, per = (n + 63) / 64;
+  static constexpr int n = lml_tile<N> * LmlRec<N>::size, per = (n + 63) / 64;
   double v[per];
   // the records of steps s0 .. end - 1, at most a tile
   __device__ __forceinline__ void load(const double* __restrict__ shared, int s0, int end) {
-    const int count = (end - s0 < kLmlTile ? end - s0 : kLmlTile) * LmlRec<N>::size;
+    const int count = (end - s0 < lml_tile<N> ? end - s0 : lml_tile<N>) * LmlRec<N>::size;
 #pragma unroll
     for (int q = 0; q < per; ++q) {
-      const int e = q * 64 + (int)threadIdx.x;
+      const int e = q * 64 + (int)(threadIdx.x & 63);
       if (e < count) v[q] = shared[(size_t)s0 * LmlRec<N>::size + e];
     }
   }
   __device__ __forceinline__ void store(double* lds) const {
 #pragma unroll
     for (int q = 0; q < per; ++q) {
-      const int e = q * 64 + (int)threadIdx.x;
+      const int e = q * 64 + (int)(threadIdx.x & 63);
       if (e < n) lds[e] = v[q];
     }
   }
@@ -371,12 +375,12 @@ __device__ __forceinline__ void lml_means_pass(const LmlArgs& a, const pdq_confi
   int in = 0, j = b / every;  // the step's place in its interval; the interval
   LmlStage<N> st;
   st.load(a.shared, b, e);
-  for (int s0 = b; s0 < e; s0 += kLmlTile) {
+  for (int s0 = b; s0 < e; s0 += lml_tile<N>) {
     Grp<64>{}.sync();
     st.store(lds);
     Grp<64>{}.sync();
-    if (s0 + kLmlTile < e) st.load(a.shared, s0 + kLmlTile, e);
-    const int n = e - s0 < kLmlTile ? e - s0 : kLmlTile;
+    if (s0 + lml_tile<N> < e) st.load(a.shared, s0 + lml_tile<N>, e);
+    const int n = e - s0 < lml_tile<N> ? e - s0 : lml_tile<N>;
     auto step = [&](int i, const LmlRegs<N>& now, LmlRegs<N>& next) {
       next.load(lds + (i + 1 < n ? i + 1 : i) * LmlRec<N>::size);
       PDQ_PHASE_BOUNDARY();
@@ -423,7 +427,7 @@ struct LmlAdjShared {
     nodes = means + (kobs - 1) * N * D;
     xibar = nodes + kobs * node;
     ckpt = xibar + (kobs - 1) * N * D;
-    state = ckpt + ((size_t)(K - 2) / kLmlTile + 1) * N * D;  // m and r between two launches
+    state = ckpt + ((size_t)(K - 2) / lml_tile<N> + 1) * N * D;  // m and r between two launches
     size = state + 2 * N * D;
   }
 };
@@ -514,8 +518,8 @@ __device__ __forceinline__ void lml_means_part_adjoint(const LmlArgs& a, const L
   lml_means_pass<N, D, 0>(
       a, a.cfg, params.v, 0, w.m0, w.m1, lds, m, r,
       [&](int s, const double* x) {
-        if (s % kLmlTile == 0) {
-          double* const c = at(own.ckpt + (size_t)(s / kLmlTile) * ND);
+        if (s % lml_tile<N> == 0) {
+          double* const c = at(own.ckpt + (size_t)(s / lml_tile<N>) * ND);
 #pragma unroll
           for (int e = 0; e < ND; ++e) c[(size_t)e * n_lanes] = x[e];
         }
@@ -559,19 +563,23 @@ __global__ void __launch_bounds__(64) lml_parts_kernel(LmlArgs args, LmlParts w)
   else lml_means_part<N, D, TPL>(a, w, b, lds);
 }
 
-// A lane per instance, after the means' pass: reverse scan, its adjoint, and
-// the tiles backwards (a tile's means from its checkpoint into the lane's
-// column of LDS, then its steps' adjoints).
+// A lane per instance, after the means' pass, in two wavefronts: 0 runs the
+// reverse scan, its adjoint and the steps' adjoints from the last to the first;
+// 1 recomputes the tiles' means from their checkpoints into the lane's column
+// of LDS, one tile ahead (beside the scan: the last one).  Both pass one
+// barrier per tile.
 template <int N, int D, int FIELD>
-__global__ void __launch_bounds__(64) lml_adjoint_kernel(LmlArgs args) {
+__global__ void __launch_bounds__(128) lml_adjoint_kernel(LmlArgs args) {
   using R = LmlRec<N>;
   using SH = LmlShared<N>;
-  constexpr int ND = N * D;
-  __shared__ double lds[LmlStage<N>::n];
-  __shared__ double means[kLmlTile * ND * 64];
+  constexpr int ND = N * D, tile = lml_tile<N>;
+  __shared__ double stage[2][LmlStage<N>::n];  // one per wavefront
+  __shared__ double means[2][tile * ND * 64];
+  const int l = threadIdx.x & 63, role = __builtin_amdgcn_readfirstlane(threadIdx.x / 64);
+  double* const lds = stage[role];
   const LmlArgs a = lml_shared_args(args, FIELD);
   const int K = a.K, every = a.every, ntan = a.n_tan;
-  const size_t n_lanes = (size_t)gridDim.x * 64, lane = (size_t)blockIdx.x * 64 + threadIdx.x;
+  const size_t n_lanes = (size_t)gridDim.x * 64, lane = (size_t)blockIdx.x * 64 + l;
   const bool active = lane < (size_t)a.n_inst;
   const int inst = active ? (int)lane : a.n_inst - 1;
   const LmlParams params(a.params + (size_t)inst * a.cfg.n_params, a.cfg.n_params);
@@ -580,6 +588,48 @@ __global__ void __launch_bounds__(64) lml_adjoint_kernel(LmlArgs args) {
   const SH lay(K, every);
   const LmlAdjShared<N, D> own(K, every);
   auto at = [&](size_t off) -> double* { return a.scratch + off * n_lanes + lane; };
+  const int last = (K - 2) / tile * tile;
+  LmlStage<N> st;
+  LmlRegs<N> ra, rb;
+  auto steps = [&](int s0) { return K - 1 - s0 < tile ? K - 1 - s0 : tile; };
+  if (role == 1) {
+    if (!a.grad) return;
+    double m[ND], r[ND], ck[ND];
+    auto fetch = [&](int s0) {
+      st.load(a.shared, s0, K - 1);
+      const double* const c = at(own.ckpt + (size_t)(s0 / tile) * ND);
+#pragma unroll
+      for (int e = 0; e < ND; ++e) ck[e] = c[(size_t)e * n_lanes];
+    };
+    fetch(last);
+    for (int s0 = last; s0 >= 0; s0 -= tile) {
+      Grp<64>{}.sync();
+      st.store(lds);
+      Grp<64>{}.sync();
+#pragma unroll
+      for (int e = 0; e < ND; ++e) {
+        m[e] = ck[e];
+        r[e] = 0.0;
+      }
+      if (s0 > 0) fetch(s0 - tile);
+      const int n = steps(s0);
+      double* const mine = means[s0 / tile & 1] + l;
+      auto again = [&](int i, const LmlRegs<N>& now, LmlRegs<N>& next) {
+        next.load(lds + (i + 1 < n ? i + 1 : i) * R::size);
+        PDQ_PHASE_BOUNDARY();
+#pragma unroll
+        for (int e = 0; e < ND; ++e) mine[(i * ND + e) * 64] = m[e];
+        lml_mean_step<N, D, 0>(a.cfg, prm, 0, now.v, true, m, r);  // (r is not used)
+      };
+      ra.load(lds);
+      for (int i = 0; i < n; i += 2) {  // (the last step's result is not used)
+        again(i, ra, rb);
+        if (i + 1 < n) again(i + 1, rb, ra);
+      }
+      __syncthreads();  // tile s0 is there, and the walk through the one after it has ended
+    }
+    return;
+  }
   double m[ND];
 #pragma unroll
   for (int e = 0; e < ND; ++e) m[e] = at(own.state)[(size_t)e * n_lanes];
@@ -607,42 +657,16 @@ __global__ void __launch_bounds__(64) lml_adjoint_kernel(LmlArgs args) {
     __device__ double tl(int) const { return 1.0; }  // (T holds both scales)
     __device__ double A(int i, int k) const { return rec[R::A + i * N + k]; }
   };
-  double* const mine = means + threadIdx.x;
-  LmlStage<N> st;
-  double ck[ND];
-  auto fetch = [&](int s0) {
-    st.load(a.shared, s0, K - 1);
-    const double* const c = at(own.ckpt + (size_t)(s0 / kLmlTile) * ND);
-#pragma unroll
-    for (int e = 0; e < ND; ++e) ck[e] = c[(size_t)e * n_lanes];
-  };
+  st.load(a.shared, last, K - 1);
   int in = 0, j = (K - 1) / every;  // the place of the step after the current one in its interval, that interval
-  const int last = (K - 2) / kLmlTile * kLmlTile;
-  fetch(last);
-  for (int s0 = last; s0 >= 0; s0 -= kLmlTile) {
+  for (int s0 = last; s0 >= 0; s0 -= tile) {
     Grp<64>{}.sync();
     st.store(lds);
     Grp<64>{}.sync();
-#pragma unroll
-    for (int e = 0; e < ND; ++e) m[e] = ck[e];
-    if (s0 > 0) fetch(s0 - kLmlTile);
-    const int n = K - 1 - s0 < kLmlTile ? K - 1 - s0 : kLmlTile;
-    double r[ND];
-#pragma unroll
-    for (int e = 0; e < ND; ++e) r[e] = 0.0;
-    LmlRegs<N> ra, rb;
-    auto again = [&](int i, const LmlRegs<N>& now, LmlRegs<N>& next) {
-      next.load(lds + (i + 1 < n ? i + 1 : i) * R::size);
-      PDQ_PHASE_BOUNDARY();
-#pragma unroll
-      for (int e = 0; e < ND; ++e) mine[(i * ND + e) * 64] = m[e];
-      lml_mean_step<N, D, 0>(a.cfg, prm, 0, now.v, true, m, r);  // (r is not used)
-    };
-    ra.load(lds);
-    for (int i = 0; i < n; i += 2) {  // (the last step's result is not used)
-      again(i, ra, rb);
-      if (i + 1 < n) again(i + 1, rb, ra);
-    }
+    if (s0 > 0) st.load(a.shared, s0 - tile, K - 1);
+    const int n = steps(s0);
+    const double* const mine = means[s0 / tile & 1] + l;
+    __syncthreads();
     auto back = [&](int i, const LmlRegs<N>& now, LmlRegs<N>& next) {
       const double* const rec = now.v;
       next.load(lds + (i > 0 ? i - 1 : 0) * R::size);

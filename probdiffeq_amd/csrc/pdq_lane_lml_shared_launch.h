@@ -14,14 +14,14 @@ int launch_lml_shared_n(LmlArgs& a, int tpl, bool reverse, hipStream_t st);
 #ifdef PDQ_LML_SHARED_DEFINE_LAUNCH
 // The factors and the means' pass, in chunks of whole intervals: launch i runs
 // the chain of chunk i, the reverts of the one before, its predecessor's merges
-// and the means of the one before that.  Sixteen chunks leave three sixteenths
-// of the chain's time uncovered; a chunk of fewer than 64 steps (70 us) would
-// not cover its launch, and with fewer than six the three launches that fill
-// and drain take what the overlap gives (nu = 4, 200 steps, gradient: 0.83 ms
-// in four chunks, 0.77 in one).
+// and the means of the one before that.  The first three launches run without
+// means (24 chunks: an eighth of the chain's time); a chunk of fewer than 64
+// steps (70 us) would not cover its launch, and with fewer than six the three
+// launches that fill and drain take what the overlap gives (nu = 4, 200 steps,
+// gradient: 0.83 ms in four chunks, 0.77 in one).
 template <int N, int TPL, int FIELD, bool ADJOINT>
 int launch_lml_parts(const LmlArgs& a, hipStream_t st) {
-  const int steps = a.K - 1, target = std::max((steps + 15) / 16, 64);
+  const int steps = a.K - 1, target = std::max((steps + 23) / 24, 64);
   int chunk = (int)std::min<long>(steps, ((long)target + a.every - 1) / a.every * a.every);
   if ((steps + chunk - 1) / chunk < 6) chunk = steps;
   const int n = (steps + chunk - 1) / chunk, lanes = (int)(((long)a.n_inst * a.G + 63) / 64);
@@ -46,7 +46,7 @@ int launch_lml_lanes(LmlArgs& a, int tpl, bool reverse, hipStream_t st) {
   }
   const int rc = launch_lml_parts<N, 0, FIELD, true>(a, st);
   if (rc) return rc;
-  hipLaunchKernelGGL((lml_adjoint_kernel<N, 2, FIELD>), dim3((a.n_inst + 63) / 64), dim3(64), 0, st, a);
+  hipLaunchKernelGGL((lml_adjoint_kernel<N, 2, FIELD>), dim3((a.n_inst + 63) / 64), dim3(128), 0, st, a);
   PDQ_HIP_TRY(hipGetLastError());
   return PDQ_OK;
 }
