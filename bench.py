@@ -36,10 +36,10 @@ HBM_PEAK_GBS = 8000.0  # MI355X HBM3E
 # profiles/lane_kernel_c2_isotropic_nu4_4096.md.  Re-measure when the kernel changes.
 C2_MEASURED_TRAFFIC_BYTES = round((228_549.9 * 2 + 940_406.3) * 1024)
 C2_TRAFFIC_SOURCE = "profiles/lane_kernel_c2_isotropic_nu4_4096.md"
-C5_MEASURED_TRAFFIC_BYTES = round((121_189.7 * 2 + 240_058.0) * 1024)
-C5_TRAFFIC_SOURCE = "profiles/lane_lml_kernel_c5_isotropic_nu3_1024.md"
-# the same for the C5 batch's reverse adjoint (lane_adj_kernel, two wavefronts)
-C5_REVERSE_MEASURED_TRAFFIC_BYTES = round((322_318.0 * 2 + 1_155_472.0) * 1024)
+# the C5 batch's LML kernels (lml_parts_kernel, all launches of a call), forward gradient and reverse adjoint
+C5_MEASURED_TRAFFIC_BYTES = round((61_450.8 * 2 + 107_398.9) * 1024)
+C5_REVERSE_MEASURED_TRAFFIC_BYTES = round(((7_889.0 + 17_991.1) * 2 + 18_316.9 + 12_112.0) * 1024)
+C5_TRAFFIC_SOURCE = "profiles/lml_parts_kernel_c5_isotropic_nu3_1024.md"
 
 
 def c2_inputs(n_inst=4096, K=200, seed=0):
@@ -170,8 +170,8 @@ def bench_c5(args, torch, capi, flops):
     res = {"lml_grads_per_s": P.shape[0] / (ms / 1e3), "lml_ms_per_batch": ms}
     n_tan = params.shape[1] + y0.shape[1]
     n_obs = data.shape[1]
-    fl = P.shape[0] * flops.lml_forward(cfg, grid.size - 1, n_obs, n_tan)
-    by = flops.lml_bytes(cfg, P.shape[0], n_obs, grid.size, n_tan)
+    fl = flops.lml_batch(cfg, P.shape[0], grid.size - 1, n_obs, n_tan)
+    by = flops.lml_batch_bytes(cfg, P.shape[0], n_obs, grid.size, n_tan)
     res["lml_roofline"] = {
         "bound": "fp64_valu",
         "achieved": fl / (ms / 1e3) / 1e12,
@@ -184,7 +184,7 @@ def bench_c5(args, torch, capi, flops):
         "traffic_source": C5_TRAFFIC_SOURCE,
         "ms_per_launch": ms,
     }
-    # the same batch through the reverse-mode adjoint (checkpoints every 50 grid steps)
+    # the same batch through the reverse-mode adjoint
     cfg_r = capi.Config(factorisation="isotropic", num_derivatives=3, ode_dim=2, strategy="fixedpoint", solver="solver", lml_gradient="reverse")
     for _ in range(max(1, args.warmup)):
         capi.lml_value_and_grad(cfg_r, P, Y0, G, 20, D, S)
@@ -196,7 +196,7 @@ def bench_c5(args, torch, capi, flops):
     e1.record()
     torch.cuda.synchronize()
     ms_r = e0.elapsed_time(e1) / reps
-    fl_r = P.shape[0] * flops.lml_reverse(cfg_r, grid.size - 1, n_obs)
+    fl_r = flops.lml_batch(cfg_r, P.shape[0], grid.size - 1, n_obs, reverse=True)
     res["lml_grads_per_s_reverse"] = P.shape[0] / (ms_r / 1e3)
     res["lml_reverse_ms_per_batch"] = ms_r
     res["lml_reverse_vs_forward_grad_max_rel"] = float(((grad_r - grad).abs().amax(dim=1) / grad.abs().amax(dim=1)).max())
@@ -207,7 +207,7 @@ def bench_c5(args, torch, capi, flops):
         "unit": "TFLOP/s",
         "frac": fl_r / (ms_r / 1e3) / 1e12 / FP64_PEAK_TFLOPS,
         "flops_per_launch": fl_r,
-        "algorithmic_bytes": flops.lml_reverse_bytes(cfg_r, P.shape[0], n_obs, grid.size),
+        "algorithmic_bytes": flops.lml_batch_bytes(cfg_r, P.shape[0], n_obs, grid.size, reverse=True),
         "traffic": C5_REVERSE_MEASURED_TRAFFIC_BYTES if P.shape[0] == 1024 else None,
         "traffic_source": C5_TRAFFIC_SOURCE,
         "ms_per_launch": ms_r,

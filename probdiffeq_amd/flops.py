@@ -127,6 +127,36 @@ def lml_reverse(cfg, grid_steps: int, observations: int) -> float:
     return nb * (3 * grid_steps * step0 + grid_steps * (step1 - step0) + scan0 + (scan1 - scan0))
 
 
+def lml_batch(cfg, n_inst: int, grid_steps: int, observations: int, n_tan: int = 0, reverse: bool = False) -> float:
+    """FLOPs of a batch of isotropic lane LMLs without calibration (PDQ_SOLVER): the grid steps' factors
+    once for the batch, and per instance the mean columns through them and the reverse scan (whose
+    factors depend on the observation stds).  Per step and column: the transition N^2 + 3 N, the revert's
+    and the merge's matrix-vector products 2 N^2 + 2 N each, the update 2 N + 1.  The reverse adjoint
+    recomputes the means once and its step costs what a step of the means does."""
+    N, d = cfg.num_derivatives + 1, cfg.ode_dim
+    factors = lml_forward(cfg, grid_steps, 0, 0)
+    column = 5 * N * N + 9 * N + 1
+    per_inst = lml_forward(cfg, 0, observations, n_tan) + grid_steps * column * d * (1 + n_tan)
+    if reverse:
+        per_inst = 2 * lml_forward(cfg, 0, observations, 0) + 3 * grid_steps * column * d
+    return factors + n_inst * per_inst
+
+
+def lml_batch_bytes(cfg, n_inst: int, observations: int, grid_points: int, n_tan: int = 0, reverse: bool = False) -> float:
+    """Algorithmic HBM bytes of the same: inputs and outputs (the Taylor coefficients carry their
+    sensitivities), the shared records written and read once, and per instance the intervals' noise
+    means (with their tangents), and for the adjoint node data, the means' adjoints and a checkpoint of
+    the mean every 16 steps, each written and read once."""
+    N, d = cfg.num_derivatives + 1, cfg.ode_dim
+    n_theta = cfg.n_params + d
+    shared = (grid_points - 1) * (4 * N + 2 * N * N + 1 + N * (N + 1)) + (observations - 1) * (N * N + N * (N + 1) // 2 + 2 * N)
+    per_inst = (observations - 1) * N * d * (1 + n_tan)
+    if reverse:
+        per_inst = 2 * (observations - 1) * N * d + observations * (N + 1 + d) + (grid_points - 1) / 16 * N * d
+    inputs = n_inst * (cfg.n_params + d + observations * (d + 1) + N * d * (1 + n_theta)) + grid_points
+    return 8.0 * (inputs + n_inst * (1 + n_theta) + 2 * shared + 2 * n_inst * per_inst)
+
+
 def lml_reverse_bytes(cfg, n_inst: int, observations: int, grid_points: int) -> float:
     """Algorithmic HBM bytes of the reverse adjoint: inputs and outputs as in the forward LML
     (the Taylor coefficients carry their n_params + d sensitivities), and per instance its storage
