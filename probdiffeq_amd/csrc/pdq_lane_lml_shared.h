@@ -31,7 +31,7 @@
 // with the gradient by tangents 7.82 -> 2.68 ms (4.46 with the chain, 2.03, before
 // the means, 2.27), by the adjoint 18.2 -> 4.05 ms (5.28;
 // 4.49 with the tiles' means recomputed by the wavefront that walks back); 300 instances, nu = 4,
-// 500 steps: 4.61 -> 1.49 and 10.95 -> 1.69 ms.  The chain and the means' pass are
+// 500 steps: 4.61 -> 1.33 and 10.95 -> 1.69 ms.  The chain and the means' pass are
 // bound by one wavefront's instruction issue.
 #pragma once
 
@@ -271,7 +271,7 @@ __device__ __forceinline__ void lml_merge(const LmlArgs& a, int j) {
 // the step's record.
 template <int N, int D, int TPL>
 __device__ __forceinline__ void lml_mean_step(const pdq_config& cfg, const double* prm, int q0, const double* rec,
-                                              bool ident, double* m, double* r) {
+                                              const double* A, bool ident, double* m, double* r) {
   constexpr int MC = D * (1 + TPL);
   using R = LmlRec<N>;
   double tmp[N * MC], Pm[N * MC], b[MC], mv[N * MC];
@@ -309,7 +309,7 @@ __device__ __forceinline__ void lml_mean_step(const pdq_config& cfg, const doubl
       for (int c = 0; c < MC; ++c) {
         double acc = 0.0;
 #pragma unroll
-        for (int k = 0; k < N; ++k) acc += rec[R::A + i * N + k] * mv[k * MC + c];
+        for (int k = 0; k < N; ++k) acc += A[i * N + k] * mv[k * MC + c];
         r[i * MC + c] = acc + r[i * MC + c];
       }
   }
@@ -321,13 +321,15 @@ __device__ __forceinline__ void lml_mean_step(const pdq_config& cfg, const doubl
   }
 }
 
-// A step's record in registers, read a step ahead of its use.
-template <int N>
+// A step's record in registers, read a step ahead of its use (without A: read
+// where it is used, where the registers do not hold it).
+template <int N, bool WITH_A = true>
 struct LmlRegs {
   double v[LmlRec<N>::size];
   __device__ __forceinline__ void load(const double* rec) {
 #pragma unroll
-    for (int e = 0; e < LmlRec<N>::size; ++e) v[e] = rec[e];
+    for (int e = 0; e < LmlRec<N>::size; ++e)
+      if (WITH_A || e < LmlRec<N>::A || e >= LmlRec<N>::t) v[e] = rec[e];
   }
 };
 
@@ -381,18 +383,21 @@ __device__ __forceinline__ void lml_means_pass(const LmlArgs& a, const pdq_confi
     Grp<64>{}.sync();
     if (s0 + lml_tile<N> < e) st.load(a.shared, s0 + lml_tile<N>, e);
     const int n = e - s0 < lml_tile<N> ? e - s0 : lml_tile<N>;
-    auto step = [&](int i, const LmlRegs<N>& now, LmlRegs<N>& next) {
+    constexpr bool with_a = !(N == 5 && TPL == 1);  // (two records with it and four columns: 172 bytes of scratch)
+    using Regs = LmlRegs<N, with_a>;
+    auto step = [&](int i, const Regs& now, Regs& next) {
       next.load(lds + (i + 1 < n ? i + 1 : i) * LmlRec<N>::size);
       PDQ_PHASE_BOUNDARY();
       at_step(s0 + i, m);
-      lml_mean_step<N, D, TPL>(cfg, prm, q0, now.v, in == 0, m, r);
+      lml_mean_step<N, D, TPL>(cfg, prm, q0, now.v,
+                               with_a ? now.v + LmlRec<N>::A : lds + i * LmlRec<N>::size + LmlRec<N>::A, in == 0, m, r);
       if (++in == every) {
         at_node(j, r);
         in = 0;
         ++j;
       }
     };
-    LmlRegs<N> ra, rb;
+    Regs ra, rb;
     ra.load(lds);
     for (int i = 0; i < n; i += 2) {
       step(i, ra, rb);
@@ -619,7 +624,7 @@ __global__ void __launch_bounds__(128) lml_adjoint_kernel(LmlArgs args) {
         PDQ_PHASE_BOUNDARY();
 #pragma unroll
         for (int e = 0; e < ND; ++e) mine[(i * ND + e) * 64] = m[e];
-        lml_mean_step<N, D, 0>(a.cfg, prm, 0, now.v, true, m, r);  // (r is not used)
+        lml_mean_step<N, D, 0>(a.cfg, prm, 0, now.v, now.v + R::A, true, m, r);  // (r is not used)
       };
       ra.load(lds);
       for (int i = 0; i < n; i += 2) {  // (the last step's result is not used)
