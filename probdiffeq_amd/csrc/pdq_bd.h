@@ -852,6 +852,18 @@ __device__ __forceinline__ void bd_solve_instance(const BdArgs& a, const BdGroup
   }
 }
 
+// A group's instances first, first + stride, ...  Every instance begins with
+// the first of the alternating buffers, so the next one waits until every
+// wavefront has read the last one's (on a fixed grid its last barrier is the
+// one before those reads).
+template <int N, int STRATEGY>
+__device__ __forceinline__ void bd_solve_instances(const BdArgs& a, const BdGroup& g, int first, int stride) {
+  for (int inst = first; inst < a.n_inst; inst += stride) {
+    bd_solve_instance<N, STRATEGY>(a, g, inst);
+    if (g.multi) g.sync();
+  }
+}
+
 // Whether the filter's kernels without OPTS take a solve: the options that
 // they fold in.  The kernels for every option hold five times the code
 // (burgers, d = 512: 13 900 instructions against 2 800) and keep twice as many
@@ -898,9 +910,7 @@ __global__ void __launch_bounds__(64) bd_wave_kernel(BdArgs args) {
   g.multi = false;
   g.y = y + (threadIdx.x / G) * 2 * G;
   g.red = nullptr;
-  const int stride = gridDim.x * gpw;
-  for (int inst = blockIdx.x * gpw + threadIdx.x / G; inst < a.n_inst; inst += stride)
-    bd_solve_instance<N, STRATEGY>(a, g, inst);
+  bd_solve_instances<N, STRATEGY>(a, g, blockIdx.x * gpw + threadIdx.x / G, gridDim.x * gpw);
 }
 
 // One workgroup of G = 64 * ceil(d / 64) <= 512 lanes per instance, grid-
@@ -919,7 +929,7 @@ __global__ void __launch_bounds__(512) bd_block_kernel(BdArgs args) {
   g.multi = true;
   g.y = y;
   g.red = red;
-  for (int inst = blockIdx.x; inst < a.n_inst; inst += gridDim.x) bd_solve_instance<N, STRATEGY>(a, g, inst);
+  bd_solve_instances<N, STRATEGY>(a, g, blockIdx.x, gridDim.x);
 }
 #endif
 

@@ -3,6 +3,7 @@
 // every instance with one lane (G = 1) so that the kernel logic can be
 // compared with the oracle on the CPU.
 #include <barrier>
+#include <chrono>
 #include <cstring>
 #include <thread>
 #include <type_traits>
@@ -32,9 +33,20 @@ namespace {
 std::barrier<>* g_group_barrier = nullptr;
 double g_group_xchg[pdq::kBdMaxDim];
 thread_local int t_group_lane = 0;
+// Lanes from g_lag_lane on leave every barrier g_lag_us late (a wavefront that
+// the others run ahead of); 0 us: none does.
+int g_lag_lane = 0, g_lag_us = 0;
 }  // namespace
 
-void pdq_emu_group_barrier() { g_group_barrier->arrive_and_wait(); }
+extern "C" void pdqemu_set_lag(int first_lane, int microseconds) {
+  g_lag_lane = first_lane;
+  g_lag_us = microseconds;
+}
+
+void pdq_emu_group_barrier() {
+  g_group_barrier->arrive_and_wait();
+  if (g_lag_us > 0 && t_group_lane >= g_lag_lane) std::this_thread::sleep_for(std::chrono::microseconds(g_lag_us));
+}
 
 double pdq_emu_shfl_xor(double v, int mask, int width) {
   const int self = t_group_lane;
@@ -57,8 +69,10 @@ double pdq_emu_shfl(double v, int src, int width) {
 }
 
 namespace {
+// A lane group's threads over the instances first, first + stride, ...: a
+// workgroup of several wavefronts keeps its LDS from one to the next.
 template <int N, int S>
-void bd_emu_instance(const pdq::BdArgs& a, int inst) {
+void bd_emu_group(const pdq::BdArgs& a, int first, int stride) {
   const int G = a.G;
   std::vector<double> y(2 * G, 0.0), red(pdq::kBdRedSize, 0.0);
   std::barrier<> bar(G);
@@ -74,18 +88,18 @@ void bd_emu_instance(const pdq::BdArgs& a, int inst) {
       g.multi = G > 64;
       g.y = y.data();
       g.red = red.data();
-      pdq::bd_solve_instance<N, S>(a, g, inst);
+      pdq::bd_solve_instances<N, S>(a, g, first, stride);
     });
   for (auto& t : th) t.join();
   g_group_barrier = nullptr;
 }
 
 template <int N>
-void bd_emu_n(const pdq::BdArgs& a, int inst) {
+void bd_emu_n(const pdq::BdArgs& a) {
   switch (a.cfg.strategy) {
-    case PDQ_FILTER: return bd_emu_instance<N, PDQ_FILTER>(a, inst);
-    case PDQ_FIXEDPOINT: return bd_emu_instance<N, PDQ_FIXEDPOINT>(a, inst);
-    default: return bd_emu_instance<N, PDQ_FIXEDINTERVAL>(a, inst);
+    case PDQ_FILTER: return bd_emu_group<N, PDQ_FILTER>(a, 0, 1);
+    case PDQ_FIXEDPOINT: return bd_emu_group<N, PDQ_FIXEDPOINT>(a, 0, 1);
+    default: return bd_emu_group<N, PDQ_FIXEDINTERVAL>(a, 0, 1);
   }
 }
 }  // namespace
@@ -241,8 +255,8 @@ int pdqemu_solve(const pdq_config* cfg, int n_inst, const double* params, const 
                  int K, const pdq_solution* out, int mode) {
   int queue = 0;
   if (cfg->factorisation == PDQ_BLOCKDIAG) {
-    // the block-diagonal kernel's code, one instance at a time, each as a
-    // group of G threads (one per block)
+    // the block-diagonal kernel's code: a group of G threads (one per block)
+    // that takes every instance
     std::vector<double> A1, Q1;
     pdq::iwp_matrices(cfg->num_derivatives, A1, Q1);
     pdq::BdArgs a{};
@@ -257,15 +271,13 @@ int pdqemu_solve(const pdq_config* cfg, int n_inst, const double* params, const 
     a.Q = Q1.data();
     a.out = *out;
     if (cfg->ode_dim > pdq::kBdMaxDim) return 2;
-    for (int i = 0; i < n_inst; ++i) {
-      switch (cfg->num_derivatives + 1) {
-        case 2: bd_emu_n<2>(a, i); break;
-        case 3: bd_emu_n<3>(a, i); break;
-        case 4: bd_emu_n<4>(a, i); break;
-        case 5: bd_emu_n<5>(a, i); break;
-        case 6: bd_emu_n<6>(a, i); break;
-        default: return 2;
-      }
+    switch (cfg->num_derivatives + 1) {
+      case 2: bd_emu_n<2>(a); break;
+      case 3: bd_emu_n<3>(a); break;
+      case 4: bd_emu_n<4>(a); break;
+      case 5: bd_emu_n<5>(a); break;
+      case 6: bd_emu_n<6>(a); break;
+      default: return 2;
     }
     return 0;
   }
