@@ -1849,14 +1849,10 @@ __global__ void __launch_bounds__(64) solve_kernel(KArgs args) {
   double* const lds = pdq_coop_lds;
   const KArgs& a = args;
   const Ctx<G> c = coop_setup<G>(a, lds);
-  for (;;) {
-    int inst = 0;
-    if (c.g.l == 0) inst = atomicAdd(a.queue, 1);
-    inst = c.g.bcast(inst);
-    if (inst >= a.n_inst) break;
+  queue_for_each(c.g, a.queue, a.n_inst, [&](int inst) {
     if (a.mode == MODE_LML) lml_instance(c, inst);
     else solve_instance(c, inst);
-  }
+  });
 }
 
 

@@ -469,9 +469,27 @@ struct Grp {
   }
 #endif
   __device__ __forceinline__ int bcast(int v) const {
+#ifdef PDQ_HOST_EMU
+    return G > 1 ? (int)pdq_emu_shfl(v, 0, G) : v;
+#else
     if constexpr (G > 1) return __shfl(v, 0, G);
     return v;
+#endif
   }
 };
+
+// f(i) for the work queue's instances i < n that this group draws.  Every lane
+// takes part in a draw (lane 0 adds one, the others nothing).  Under a branch
+// for lane 0 alone, the other lanes' index is a constant of the loop, and the
+// compiler may split the loop by lane: lane 0 leaves for the next draw while
+// the others go round with their constant, for ever.
+template <int G, class F>
+__device__ __forceinline__ void queue_for_each(const Grp<G>& g, int* queue, int n, F&& f) {
+  for (;;) {
+    const int i = g.bcast(atomicAdd(queue, g.l == 0 ? 1 : 0));
+    if (i >= n) break;
+    f(i);
+  }
+}
 
 }  // namespace pdq

@@ -26,10 +26,10 @@ inline void __threadfence_block() {}
 inline double __shfl_xor(double v, int, int) { return v; }
 inline int __shfl(int v, int, int) { return v; }
 inline double __shfl(double v, int, int) { return v; }
+inline int pdq_emu_atomics = 0;  // atomic operations issued, by all lanes
 inline int atomicAdd(int* p, int v) {
-  const int old = *p;
-  *p += v;
-  return old;
+  __atomic_fetch_add(&pdq_emu_atomics, 1, __ATOMIC_RELAXED);
+  return __atomic_fetch_add(p, v, __ATOMIC_RELAXED);
 }
 #define __builtin_amdgcn_fence(a, b) ((void)0)
 #define __builtin_amdgcn_wave_barrier() ((void)0)

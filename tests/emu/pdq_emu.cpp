@@ -104,7 +104,38 @@ void bd_emu_n(const pdq::BdArgs& a) {
 }
 }  // namespace
 
+namespace {
+template <int G>
+int queue_emu(int n, int* taken) {
+  int queue = 0;
+  std::barrier<> bar(G);
+  g_group_barrier = &bar;
+  pdq_emu_atomics = 0;
+  std::vector<std::thread> th;
+  for (int l = 0; l < G; ++l)
+    th.emplace_back([&, l] {
+      t_group_lane = l;
+      pdq::queue_for_each(pdq::Grp<G>{l}, &queue, n, [&](int i) { ++taken[(size_t)i * G + l]; });
+    });
+  for (auto& t : th) t.join();
+  g_group_barrier = nullptr;
+  return pdq_emu_atomics;
+}
+}  // namespace
+
 extern "C" {
+
+// One group of G lanes draws n instances from the work queue (queue_for_each):
+// taken[i G + l] counts lane l's calls with instance i.  Returns the atomic
+// operations issued.
+int pdqemu_queue(int G, int n, int* taken) {
+  switch (G) {
+    case 4: return queue_emu<4>(n, taken);
+    case 16: return queue_emu<16>(n, taken);
+    case 64: return queue_emu<64>(n, taken);
+  }
+  return -1;
+}
 
 // Entries where the lane kernel's compile-time IWP transition (pdq_lane.h:
 // lane_iwp_a) differs from the host's iwp_matrices, for nu = 1..7.
