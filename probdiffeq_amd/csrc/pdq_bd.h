@@ -47,14 +47,6 @@
 #include "pdq_lane.h"
 #include "pdq_wave.h"
 
-#ifdef PDQ_HOST_EMU
-// The CPU build runs a group as G threads (tests/emu): these hooks are the
-// harness's barrier and lane exchange.
-void pdq_emu_group_barrier();
-double pdq_emu_shfl_xor(double v, int mask, int width);
-double pdq_emu_shfl(double v, int src, int width);
-#endif
-
 namespace pdq {
 
 // Largest block-diagonal dimension (one lane per block, <= 512 lanes per
@@ -90,17 +82,8 @@ struct BdGroup {
   mutable int ybuf = 0, rbuf = 0;
 
   __device__ __forceinline__ void sync() const {
-#ifdef PDQ_HOST_EMU
-    pdq_emu_group_barrier();
-#else
-    if (multi) {
-      __syncthreads();
-    } else {
-      __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-      __builtin_amdgcn_wave_barrier();
-      __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-    }
-#endif
+    if (multi) __syncthreads();
+    else Grp<64>{}.sync();
   }
   __device__ __forceinline__ double shfl_xor(double v, int m, int w) const {
 #ifdef PDQ_HOST_EMU
@@ -852,18 +835,6 @@ __device__ __forceinline__ void bd_solve_instance(const BdArgs& a, const BdGroup
   }
 }
 
-// A group's instances first, first + stride, ...  Every instance begins with
-// the first of the alternating buffers, so the next one waits until every
-// wavefront has read the last one's (on a fixed grid its last barrier is the
-// one before those reads).
-template <int N, int STRATEGY>
-__device__ __forceinline__ void bd_solve_instances(const BdArgs& a, const BdGroup& g, int first, int stride) {
-  for (int inst = first; inst < a.n_inst; inst += stride) {
-    bd_solve_instance<N, STRATEGY>(a, g, inst);
-    if (g.multi) g.sync();
-  }
-}
-
 // Whether the filter's kernels without OPTS take a solve: the options that
 // they fold in.  The kernels for every option hold five times the code
 // (burgers, d = 512: 13 900 instructions against 2 800) and keep twice as many
@@ -894,7 +865,6 @@ __device__ __forceinline__ BdArgs bd_args(const BdArgs& args, int strategy) {
   return a;
 }
 
-#ifndef PDQ_HOST_EMU
 // Groups of G <= 64 lanes, 64 / G instances per wavefront, grid-stride over
 // instances.  A group's instances and its exits depend only on values the
 // whole group shares, so each group leaves the loop as a unit.
@@ -910,7 +880,9 @@ __global__ void __launch_bounds__(64) bd_wave_kernel(BdArgs args) {
   g.multi = false;
   g.y = y + (threadIdx.x / G) * 2 * G;
   g.red = nullptr;
-  bd_solve_instances<N, STRATEGY>(a, g, blockIdx.x * gpw + threadIdx.x / G, gridDim.x * gpw);
+  const int stride = gridDim.x * gpw;
+  for (int inst = blockIdx.x * gpw + threadIdx.x / G; inst < a.n_inst; inst += stride)
+    bd_solve_instance<N, STRATEGY>(a, g, inst);
 }
 
 // One workgroup of G = 64 * ceil(d / 64) <= 512 lanes per instance, grid-
@@ -929,9 +901,14 @@ __global__ void __launch_bounds__(512) bd_block_kernel(BdArgs args) {
   g.multi = true;
   g.y = y;
   g.red = red;
-  bd_solve_instances<N, STRATEGY>(a, g, blockIdx.x, gridDim.x);
+  for (int inst = blockIdx.x; inst < a.n_inst; inst += gridDim.x) {
+    bd_solve_instance<N, STRATEGY>(a, g, inst);
+    // Every instance begins with the first of the alternating buffers: the next
+    // one waits until all wavefronts have read this one's (on a fixed grid its
+    // last barrier is the one before those reads).
+    __syncthreads();
+  }
 }
-#endif
 
 // Lanes per instance for dimension d (the launcher and the CPU build agree).
 inline int bd_group_lanes(int d) {

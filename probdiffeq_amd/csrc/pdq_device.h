@@ -420,8 +420,7 @@ __device__ __forceinline__ double factorial_d(int k) {
 #ifdef PDQ_HOST_EMU
 }  // namespace pdq
 // The CPU build runs a group of more than one lane as threads (tests/emu):
-// these hooks are the harness's barrier and lane exchange.
-void pdq_emu_group_barrier();
+// these hooks are the harness's lane exchange.
 double pdq_emu_shfl_xor(double v, int mask, int width);
 double pdq_emu_shfl(double v, int src, int width);
 namespace pdq {
@@ -433,7 +432,7 @@ struct Grp {
   __device__ __forceinline__ void sync() const {
     if constexpr (G > 1) {
 #ifdef PDQ_HOST_EMU
-      pdq_emu_group_barrier();
+      pdq_emu_wave_barrier();
 #else
       __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
       __builtin_amdgcn_wave_barrier();

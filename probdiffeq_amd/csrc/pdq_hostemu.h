@@ -1,7 +1,9 @@
 // Host build of the device sources (test infrastructure): compiled with g++
 // and PDQ_HOST_EMU defined, the kernels' per-instance code runs on the CPU
-// with one lane per group (G = 1) and one thread per workgroup, so that the
-// kernel logic can be checked against the oracle without a GPU.
+// with one lane per group (G = 1) and one thread per workgroup, or a whole
+// workgroup as one thread per lane with the harness's barriers (tests/emu), so
+// that the kernel logic can be checked against the oracle without a GPU.
+// LDS arrays are static: shared by the threads of the one workgroup that runs.
 #pragma once
 
 #include <cmath>
@@ -12,16 +14,20 @@
 #define __host__
 #define __global__
 #define __forceinline__ inline
-#define __launch_bounds__(x)
-#define __shared__
+#define __launch_bounds__(...)
+#define __shared__ static
 
 struct PdqEmuDim {
   unsigned x = 0;
 };
-static PdqEmuDim threadIdx;
-static PdqEmuDim blockDim{1};
+inline thread_local PdqEmuDim threadIdx, blockIdx;
+inline PdqEmuDim blockDim{1}, gridDim{1};
 
-inline void __syncthreads() {}
+// The barriers of a workgroup's lanes and of one wavefront's (nothing outside a group).
+void pdq_emu_group_barrier();
+void pdq_emu_wave_barrier();
+
+inline void __syncthreads() { pdq_emu_group_barrier(); }
 inline void __threadfence_block() {}
 inline double __shfl_xor(double v, int, int) { return v; }
 inline int __shfl(int v, int, int) { return v; }

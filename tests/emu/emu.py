@@ -13,9 +13,19 @@ BUILD = os.path.join(HERE, "_build")
 LIB = os.path.join(BUILD, "libpdqemu.so")
 
 
+def _sources():
+    root = os.path.dirname(os.path.dirname(HERE))
+    for folder in (HERE, os.path.join(root, "probdiffeq_amd", "csrc"), os.path.join(root, "include")):
+        for name in os.listdir(folder):
+            if name.endswith((".cpp", ".h", ".hip")):
+                yield os.path.join(folder, name)
+
+
 def build(extra=()) -> str:
     os.makedirs(BUILD, exist_ok=True)
     src = os.path.join(HERE, "pdq_emu.cpp")
+    if not extra and os.path.exists(LIB) and os.path.getmtime(LIB) > max(os.path.getmtime(f) for f in _sources()):
+        return LIB
     # compiled to a private name and renamed into place, so that concurrent
     # test processes never load a half-written library
     tmp = f"{LIB}.{os.getpid()}.tmp"

@@ -5,6 +5,7 @@
 #include <barrier>
 #include <chrono>
 #include <cstring>
+#include <memory>
 #include <thread>
 #include <type_traits>
 #include <vector>
@@ -25,16 +26,17 @@ int host_error(int code, const char*, ...) { return code; }
 int num_cus() { return 1; }
 }  // namespace pdq
 
-// The block-diagonal kernel's lane group on the CPU: one thread per lane, a
-// real barrier, and lane exchanges through a shared array with HIP's
-// __shfl_xor / __shfl semantics (a source lane outside the caller's width
-// segment reads the caller's own value).
+// A lane group on the CPU: one thread per lane, real barriers (one for the
+// group and, in a workgroup of several wavefronts, one per wavefront), and lane
+// exchanges through a shared array with HIP's __shfl_xor / __shfl semantics (a
+// source lane outside the caller's width segment reads the caller's own value).
 namespace {
 std::barrier<>* g_group_barrier = nullptr;
 double g_group_xchg[pdq::kBdMaxDim];
 thread_local int t_group_lane = 0;
-// Lanes from g_lag_lane on leave every barrier g_lag_us late (a wavefront that
-// the others run ahead of); 0 us: none does.
+thread_local std::barrier<>* t_wave_barrier = nullptr;
+// Lanes from g_lag_lane on leave every barrier of the group g_lag_us late (a
+// wavefront that the others run ahead of); 0 us: none does.
 int g_lag_lane = 0, g_lag_us = 0;
 }  // namespace
 
@@ -44,8 +46,14 @@ extern "C" void pdqemu_set_lag(int first_lane, int microseconds) {
 }
 
 void pdq_emu_group_barrier() {
+  if (!g_group_barrier) return;
   g_group_barrier->arrive_and_wait();
   if (g_lag_us > 0 && t_group_lane >= g_lag_lane) std::this_thread::sleep_for(std::chrono::microseconds(g_lag_us));
+}
+
+void pdq_emu_wave_barrier() {
+  if (t_wave_barrier) t_wave_barrier->arrive_and_wait();
+  else if (g_group_barrier) g_group_barrier->arrive_and_wait();
 }
 
 double pdq_emu_shfl_xor(double v, int mask, int width) {
@@ -69,37 +77,70 @@ double pdq_emu_shfl(double v, int src, int width) {
 }
 
 namespace {
-// A lane group's threads over the instances first, first + stride, ...: a
-// workgroup of several wavefronts keeps its LDS from one to the next.
-template <int N, int S>
-void bd_emu_group(const pdq::BdArgs& a, int first, int stride) {
-  const int G = a.G;
-  std::vector<double> y(2 * G, 0.0), red(pdq::kBdRedSize, 0.0);
-  std::barrier<> bar(G);
+// Runs f on a group of `lanes` threads.
+template <class F>
+void emu_group(int lanes, F&& f) {
+  std::barrier<> bar(lanes);
   g_group_barrier = &bar;
   std::vector<std::thread> th;
-  th.reserve(G);
-  for (int l = 0; l < G; ++l)
+  th.reserve(lanes);
+  for (int l = 0; l < lanes; ++l)
     th.emplace_back([&, l] {
       t_group_lane = l;
-      pdq::BdGroup g;
-      g.G = G;
-      g.lane = l;
-      g.multi = G > 64;
-      g.y = y.data();
-      g.red = red.data();
-      pdq::bd_solve_instances<N, S>(a, g, first, stride);
+      f(l);
     });
   for (auto& t : th) t.join();
   g_group_barrier = nullptr;
 }
 
+// Runs a kernel's workgroups one after another, each as `lanes` threads (a
+// multiple of 64).
+template <class F>
+void emu_launch(int blocks, int lanes, F&& kernel) {
+  gridDim.x = blocks;
+  blockDim.x = lanes;
+  for (int b = 0; b < blocks; ++b) {
+    std::vector<std::unique_ptr<std::barrier<>>> waves;
+    for (int w = 0; w < lanes / 64; ++w) waves.push_back(std::make_unique<std::barrier<>>(64));
+    emu_group(lanes, [&](int l) {
+      threadIdx.x = l;
+      blockIdx.x = b;
+      t_wave_barrier = waves[l / 64].get();
+      kernel();
+    });
+  }
+  gridDim.x = blockDim.x = 1;
+}
+
+// One instance on a group of a single wavefront's lanes (of G threads).
+template <int N, int S>
+void bd_emu_wave(const pdq::BdArgs& a, int inst) {
+  const int G = a.G;
+  std::vector<double> y(2 * G, 0.0);
+  emu_group(G, [&](int l) {
+    pdq::BdGroup g;
+    g.G = G;
+    g.lane = l;
+    g.multi = false;
+    g.y = y.data();
+    g.red = nullptr;
+    pdq::bd_solve_instance<N, S>(a, g, inst);
+  });
+}
+
+// Every instance; above 64 lanes the kernel itself, one workgroup for all.
+template <int N, int S>
+void bd_emu_ns(const pdq::BdArgs& a) {
+  if (a.G > 64) return emu_launch(1, a.G, [&] { pdq::bd_block_kernel<N, S, true>(a); });
+  for (int i = 0; i < a.n_inst; ++i) bd_emu_wave<N, S>(a, i);
+}
+
 template <int N>
 void bd_emu_n(const pdq::BdArgs& a) {
   switch (a.cfg.strategy) {
-    case PDQ_FILTER: return bd_emu_group<N, PDQ_FILTER>(a, 0, 1);
-    case PDQ_FIXEDPOINT: return bd_emu_group<N, PDQ_FIXEDPOINT>(a, 0, 1);
-    default: return bd_emu_group<N, PDQ_FIXEDINTERVAL>(a, 0, 1);
+    case PDQ_FILTER: return bd_emu_ns<N, PDQ_FILTER>(a);
+    case PDQ_FIXEDPOINT: return bd_emu_ns<N, PDQ_FIXEDPOINT>(a);
+    default: return bd_emu_ns<N, PDQ_FIXEDINTERVAL>(a);
   }
 }
 }  // namespace
@@ -108,17 +149,10 @@ namespace {
 template <int G>
 int queue_emu(int n, int* taken) {
   int queue = 0;
-  std::barrier<> bar(G);
-  g_group_barrier = &bar;
   pdq_emu_atomics = 0;
-  std::vector<std::thread> th;
-  for (int l = 0; l < G; ++l)
-    th.emplace_back([&, l] {
-      t_group_lane = l;
-      pdq::queue_for_each(pdq::Grp<G>{l}, &queue, n, [&](int i) { ++taken[(size_t)i * G + l]; });
-    });
-  for (auto& t : th) t.join();
-  g_group_barrier = nullptr;
+  emu_group(G, [&](int l) {
+    pdq::queue_for_each(pdq::Grp<G>{l}, &queue, n, [&](int i) { ++taken[(size_t)i * G + l]; });
+  });
   return pdq_emu_atomics;
 }
 }  // namespace
@@ -287,7 +321,6 @@ int pdqemu_solve(const pdq_config* cfg, int n_inst, const double* params, const 
   int queue = 0;
   if (cfg->factorisation == PDQ_BLOCKDIAG) {
     // the block-diagonal kernel's code: a group of G threads (one per block)
-    // that takes every instance
     std::vector<double> A1, Q1;
     pdq::iwp_matrices(cfg->num_derivatives, A1, Q1);
     pdq::BdArgs a{};
@@ -345,20 +378,12 @@ namespace {
 template <class SH>
 void wave_emu_instance(const pdq::KArgs& a, int inst) {
   std::vector<double> lds(SH::fixed_size + a.cfg.n_params, 0.0);
-  std::barrier<> bar(64);
-  g_group_barrier = &bar;
-  std::vector<std::thread> th;
-  th.reserve(64);
-  for (int l = 0; l < 64; ++l)
-    th.emplace_back([&, l] {
-      t_group_lane = l;
-      pdq::WCtx<SH> c(&a, lds.data(), l);
-      c.inst = inst;
-      pdq::w_setup<SH>(a, lds.data(), l);
-      pdq::w_solve_instance(c);
-    });
-  for (auto& t : th) t.join();
-  g_group_barrier = nullptr;
+  emu_group(64, [&](int l) {
+    pdq::WCtx<SH> c(&a, lds.data(), l);
+    c.inst = inst;
+    pdq::w_setup<SH>(a, lds.data(), l);
+    pdq::w_solve_instance(c);
+  });
 }
 
 template <int N, bool DENSE>
