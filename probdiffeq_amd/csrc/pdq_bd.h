@@ -100,12 +100,16 @@ struct BdGroup {
 #endif
   }
   // Whether this lane's wavefront takes the step's scalar decisions (sum).
-  __device__ __forceinline__ bool first_wave() const { return !multi || lane < 64; }
+  template <bool LEAD>
+  __device__ __forceinline__ bool decides() const {
+    return !LEAD || !multi || lane < 64;
+  }
   __device__ __forceinline__ double* ctl() const { return red + 2 * kBdRedStride; }
   // Group sum: a butterfly per wavefront, whose total is the bitwise same in
   // every lane (each stage adds the same two values in both lanes), then the
-  // wavefronts' totals added in wavefront order.  With several wavefronts only
-  // the first one's lanes get the total.
+  // wavefronts' totals added in wavefront order.  With LEAD and several
+  // wavefronts only the first one's lanes get the total.
+  template <bool LEAD>
   __device__ __forceinline__ double sum(double v) const {
     if (!multi) return wave_total(v, G);
     v = wave_total(v, 64);
@@ -114,7 +118,12 @@ struct BdGroup {
     rbuf ^= 1;
     if ((lane & 63) == 0) r[w] = v;
     sync();
-    if (!first_wave()) return 0.0;
+    if (!decides<LEAD>()) return 0.0;
+    if constexpr (!LEAD) {
+      double s = 0.0;
+      for (int i = 0; i < nw; ++i) s += r[i];
+      return s;
+    }
     // all reads at once; the entries beyond nw stay 0
     double p[kBdRedStride], s = 0.0;
 #pragma unroll
@@ -202,6 +211,19 @@ __device__ __forceinline__ LCondView<N> cv(LCond<N, 1>& c) {
   return LCondView<N>{&c};
 }
 
+// Whether a group's first wavefront takes the step's scalar decisions for all.
+// The filter's does (bd_control).  The smoothers' slots and conditionals spill
+// (24 to 3 000 bytes of scratch per lane), and the other wavefronts' wait, the
+// partial sums read at once and the shared result cost more there than the
+// roots and powers they save: ms with the first wavefront deciding / every one,
+// fixed-interval nu = 3, d = 200 (64 instances): 12.0 / 7.9, nu = 5: 53.7 / 51.1;
+// fixed-point nu = 2, d = 512 (256 instances): 9.09 / 8.2, nu = 5, d = 200: 225 / 203.
+// What is spilled where also depends on how the decision is written, with the same
+// scratch sizes: through bd_control the fixed-interval nu = 3 takes 9.0 ms, and
+// without it the fixed-point nu = 2 takes 10.1, hence one of the two for each.
+template <int STRATEGY>
+constexpr bool bd_lead = STRATEGY == PDQ_FILTER;
+
 // Group-uniform scalars of a slot.
 struct BdScal {
   double t;
@@ -219,7 +241,7 @@ __device__ __forceinline__ void bd_rounded(double (&x)[n]) {
   for (int i = 0; i < n; ++i) x[i] = wave_rounded(x[i]);
 }
 
-template <int N, int STRATEGY>
+template <int N, int STRATEGY, bool OPTS>
 struct BdCtx {
   const BdArgs* a;
   const double* prm;
@@ -236,8 +258,8 @@ struct BdCtx {
 // Burgers' component k (the registry's formula, vf_component in
 // pdq_device.h): the periodic neighbours without an integer modulo, the two
 // quotients from the instance's reciprocals.  Bitwise the registry's value.
-template <int N, int STRATEGY>
-__device__ __forceinline__ double bd_burgers(const BdCtx<N, STRATEGY>& c, const double* y, int d, int k) {
+template <int N, int STRATEGY, bool OPTS>
+__device__ __forceinline__ double bd_burgers(const BdCtx<N, STRATEGY, OPTS>& c, const double* y, int d, int k) {
   const double visc = c.prm[0];
   const int km = k == 0 ? d - 1 : k - 1, kp = k + 1 == d ? 0 : k + 1;
   const double um = y[km], u0 = y[k], up = y[kp];
@@ -252,8 +274,8 @@ __device__ __forceinline__ double bd_burgers(const BdCtx<N, STRATEGY>& c, const 
 // jacobian_monte_carlo_rev and _fwd, jacobians.py:250-271, 171-192) h0 is minus
 // the probe mean of (v^T J)_k v_k or (J v)_k v_k over the probe set c.lin_set.  Every lane of the group calls it (it
 // synchronises twice).
-template <int N, int STRATEGY>
-__device__ __forceinline__ void bd_linearize(const BdCtx<N, STRATEGY>& c, const double* Xm, double t, double& b,
+template <int N, int STRATEGY, bool OPTS>
+__device__ __forceinline__ void bd_linearize(const BdCtx<N, STRATEGY, OPTS>& c, const double* Xm, double t, double& b,
                                              double& h0, uint32_t set_offset = 0) {
   const pdq_config& cfg = c.a->cfg;
   const int d = cfg.ode_dim, k = c.g.lane;
@@ -286,8 +308,8 @@ __device__ __forceinline__ void bd_linearize(const BdCtx<N, STRATEGY>& c, const 
 // whole instance from group sums (error_norm_scale_then_rms /
 // _rms_then_scale, solvers.py:770-811, over d errors and d references): in the
 // group's first wavefront, 0 in the others (bd_control).
-template <int N, int STRATEGY>
-__device__ __forceinline__ double bd_error_power(const BdCtx<N, STRATEGY>& c, double err, int row, const double* prev_m,
+template <int N, int STRATEGY, bool OPTS>
+__device__ __forceinline__ double bd_error_power(const BdCtx<N, STRATEGY, OPTS>& c, double err, int row, const double* prev_m,
                                                  const double* prop_m, double dt, int nord) {
   const pdq_config& cfg = c.a->cfg;
   const double e = nord == 1 ? err * dt / 1.0 : err * pow(dt, (double)nord) / factorial_d(nord);
@@ -299,13 +321,13 @@ __device__ __forceinline__ double bd_error_power(const BdCtx<N, STRATEGY>& c, do
   double norm;
   if (cfg.error_norm == PDQ_NORM_SCALE_THEN_RMS) {
     const double rr = e / (cfg.atol + cfg.rtol * fabs(ref));
-    const double tot = c.g.sum(c.act ? rr * rr : 0.0);
-    if (!c.g.first_wave()) return 0.0;
+    const double tot = c.g.template sum<bd_lead<STRATEGY>>(c.act ? rr * rr : 0.0);
+    if (!c.g.template decides<bd_lead<STRATEGY>>()) return 0.0;
     norm = lane_div(sqrt(tot), c.sqd, c.rsqd);  // sqrt(tot) / sqrt(d)
   } else {
-    const double sa = c.g.sum(c.act ? e * e : 0.0);
-    const double sr = c.g.sum(c.act ? ref * ref : 0.0);
-    if (!c.g.first_wave()) return 0.0;
+    const double sa = c.g.template sum<bd_lead<STRATEGY>>(c.act ? e * e : 0.0);
+    const double sr = c.g.template sum<bd_lead<STRATEGY>>(c.act ? ref * ref : 0.0);
+    if (!c.g.template decides<bd_lead<STRATEGY>>()) return 0.0;
     norm = (sqrt(sa) / sqrt(d)) / (cfg.atol + cfg.rtol * (sqrt(sr) / sqrt(d)));
   }
   return lane_root_inv<N>(norm);  // pow(norm, -1/N), as the lane kernel's error power takes it
@@ -314,12 +336,12 @@ __device__ __forceinline__ double bd_error_power(const BdCtx<N, STRATEGY>& c, do
 // The controller on the error power.  With several wavefronts the first one
 // takes the roots and powers for all (they would run one after another on the
 // SIMDs that hold two of them) and hands ep and the new dt over in LDS.
-template <int N, int STRATEGY>
-__device__ __forceinline__ double bd_control(const BdCtx<N, STRATEGY>& c, double h, double& cstate, double& ep) {
+template <int N, int STRATEGY, bool OPTS>
+__device__ __forceinline__ double bd_control(const BdCtx<N, STRATEGY, OPTS>& c, double h, double& cstate, double& ep) {
   const pdq_config& cfg = c.a->cfg;
-  if (!c.g.multi) return lane_control(cfg, h, cstate, ep);
+  if (!bd_lead<STRATEGY> || !c.g.multi) return lane_control(cfg, h, cstate, ep);
   double* const r = c.g.ctl();
-  if (c.g.first_wave()) {
+  if (c.g.template decides<true>()) {
     const double dt = lane_control(cfg, h, cstate, ep);
     if (c.g.lane == 0) {
       r[0] = ep;
@@ -415,8 +437,8 @@ __device__ __forceinline__ void bd_write_normal(const double* m, const double* L
 }
 
 // Backward conditional j of block k (identity when `ident`).
-template <int N, int STRATEGY>
-__device__ __forceinline__ void bd_write_cond(const BdCtx<N, STRATEGY>& c, bool ident, const LCond<N, 1>& s, int j) {
+template <int N, int STRATEGY, bool OPTS>
+__device__ __forceinline__ void bd_write_cond(const BdCtx<N, STRATEGY, OPTS>& c, bool ident, const LCond<N, 1>& s, int j) {
   const pdq_solution& o = c.a->out;
   const int d = c.a->cfg.ode_dim, k = c.g.lane;
   const size_t idx = ((size_t)c.inst * (c.a->K - 1) + j) * d + k;
@@ -437,8 +459,8 @@ __device__ __forceinline__ void bd_write_cond(const BdCtx<N, STRATEGY>& c, bool 
 
 // Checkpoint k: the filter's marginal, or the smoothers' filtering marginal
 // (and, with `cond`, the backward conditional that leads to it).
-template <int N, int STRATEGY>
-__device__ __forceinline__ void bd_write_checkpoint(const BdCtx<N, STRATEGY>& c, int k, double t, const double* m,
+template <int N, int STRATEGY, bool OPTS>
+__device__ __forceinline__ void bd_write_checkpoint(const BdCtx<N, STRATEGY, OPTS>& c, int k, double t, const double* m,
                                                     const double* L, double os, double nsteps,
                                                     const LCond<N, 1>* cond, bool cond_ident) {
   const pdq_solution& o = c.a->out;
@@ -454,16 +476,16 @@ __device__ __forceinline__ void bd_write_checkpoint(const BdCtx<N, STRATEGY>& c,
   const size_t mo = (row * d + blk) * N, co = (row * d + blk) * N * N;
   if (STRATEGY != PDQ_FILTER) {
     bd_write_normal<N>(m, L, o.filt_mean ? o.filt_mean + mo : nullptr, o.filt_chol ? o.filt_chol + co : nullptr);
-    if (k > 0 && cond) bd_write_cond<N, STRATEGY>(c, cond_ident, *cond, k - 1);
+    if (k > 0 && cond) bd_write_cond<N, STRATEGY, OPTS>(c, cond_ident, *cond, k - 1);
   } else {
     bd_write_normal<N>(m, L, o.mean ? o.mean + mo : nullptr, o.chol ? o.chol + co : nullptr);
   }
 }
 
-template <int N, int STRATEGY>
-__device__ __forceinline__ void bd_write_slot(const BdCtx<N, STRATEGY>& c, int k, const BdSlot<N>& s,
+template <int N, int STRATEGY, bool OPTS>
+__device__ __forceinline__ void bd_write_slot(const BdCtx<N, STRATEGY, OPTS>& c, int k, const BdSlot<N>& s,
                                               const BdScal& z) {
-  bd_write_checkpoint<N, STRATEGY>(c, k, z.t, s.m, s.L, s.os, z.nsteps, &s.c, z.ident);
+  bd_write_checkpoint<N, STRATEGY, OPTS>(c, k, z.t, s.m, s.L, s.os, z.nsteps, &s.c, z.ident);
 }
 
 template <int N>
@@ -482,8 +504,8 @@ __device__ __forceinline__ void bd_copy(BdSlot<N>& dst, const BdSlot<N>& src) {
 // (solvers.py:549-599), solver.step (:702-733) or solver_mle.step
 // (:395-437), with the error estimate.  Returns error_power (with
 // `estimate`).  Every lane of the group calls it.
-template <int N, int STRATEGY>
-__device__ __forceinline__ double bd_step(const BdCtx<N, STRATEGY>& c, const BdSlot<N>& sf, const BdScal& zs,
+template <int N, int STRATEGY, bool OPTS>
+__device__ __forceinline__ double bd_step(const BdCtx<N, STRATEGY, OPTS>& c, const BdSlot<N>& sf, const BdScal& zs,
                                           BdSlot<N>& pr, BdScal& zp, double h, bool estimate) {
   const pdq_config& cfg = c.a->cfg;
   const double* __restrict__ Q = c.a->Q;
@@ -501,10 +523,12 @@ __device__ __forceinline__ double bd_step(const BdCtx<N, STRATEGY>& c, const BdS
     for (int i = 0; i < N; ++i)
 #pragma unroll
       for (int j = 0; j < N; ++j) UL[i * N + j] = fabs(P[i]) * (s1 * lane_iwp_q<N>(Q, i, j));
-    bd_rounded(Um);
-    bd_rounded(UL);
-    bd_linearize<N, STRATEGY>(c, Um, tn, b, h0);
-    b = wave_rounded(b);
+    if constexpr (!OPTS) {
+      bd_rounded(Um);
+      bd_rounded(UL);
+    }
+    bd_linearize<N, STRATEGY, OPTS>(c, Um, tn, b, h0);
+    if constexpr (!OPTS) b = wave_rounded(b);
     double om, oL;
     lane_marginalise_fx<N, 1>(cfg, &b, h0, Um, UL, &om, oL);
     sigma = lane_rms_zero<1>(&om, oL);
@@ -522,20 +546,22 @@ __device__ __forceinline__ double bd_step(const BdCtx<N, STRATEGY>& c, const BdS
     PDQ_PHASE_BOUNDARY();
     if (STRATEGY == PDQ_FIXEDPOINT) lane_merge<N, 1>(zs.ident, sf.c, cv<N>(pr.c), cv<N>(pr.c));
   }
-  Pm[0] = wave_rounded(Pm[0]);  // the rows that the linearisation reads; the others' products are the update's
-  Pm[1] = wave_rounded(Pm[1]);
-  bd_rounded(PL);
+  if constexpr (!OPTS) {
+    Pm[0] = wave_rounded(Pm[0]);  // the rows that the linearisation reads; the others' products are the update's
+    Pm[1] = wave_rounded(Pm[1]);
+    bd_rounded(PL);
+  }
   PDQ_PHASE_BOUNDARY();
   // (3) the update, the MLE running scale and the error estimate
   double Rm[N], RL[N * N], mo, oLu;
   if (cfg.solver == PDQ_SOLVER_DYNAMIC) {
     double bu = b, hu = h0;
-    if (cfg.re_linearize_after_calibration) bd_linearize<N, STRATEGY>(c, Pm, tn, bu, hu, 1);
+    if (cfg.re_linearize_after_calibration) bd_linearize<N, STRATEGY, OPTS>(c, Pm, tn, bu, hu, 1);
     lane_update<N, 1>(cfg, &bu, hu, Pm, PL, Rm, RL, &mo, oLu);
     pr.mle_run = 0.0;
     zp.mle_n = 0.0;
   } else {
-    bd_linearize<N, STRATEGY>(c, Pm, tn, b, h0);
+    bd_linearize<N, STRATEGY, OPTS>(c, Pm, tn, b, h0);
     if (estimate) {
       double Um[N], UL[N * N], be = b, he = h0;
       lane_apply_flat_mean<N, 1>(P, PI, sf.m, Um);
@@ -545,7 +571,7 @@ __device__ __forceinline__ double bd_step(const BdCtx<N, STRATEGY>& c, const BdS
         for (int j = 0; j < N; ++j) UL[i * N + j] = fabs(P[i]) * (s1 * lane_iwp_q<N>(Q, i, j));
       // re_linearize_before_error (solvers.py:951-956): a new linearisation
       // at the extrapolation
-      if (cfg.error_re_linearize) bd_linearize<N, STRATEGY>(c, Um, tn, be, he);
+      if (cfg.error_re_linearize) bd_linearize<N, STRATEGY, OPTS>(c, Um, tn, be, he);
       if (state_std) {
         err = lane_state_err<N, 1>(cfg, &be, he, Um, UL, cfg.error_derivative_idx);
       } else {
@@ -570,15 +596,15 @@ __device__ __forceinline__ double bd_step(const BdCtx<N, STRATEGY>& c, const BdS
       sigma = 1.0;
     }
   }
-  sigma = wave_rounded(sigma);
-  err = wave_rounded(err);
-
-
+  if constexpr (!OPTS) {
+    sigma = wave_rounded(sigma);
+    err = wave_rounded(err);
+  }
   double ep = 0.0;
   if (estimate) {
     const int err_row = state_std ? cfg.error_derivative_idx : 0;
     const int nord = (state_std ? cfg.error_derivative_idx : 1) + (cfg.error_per_unit_step ? 1 : 0);
-    ep = bd_error_power<N, STRATEGY>(c, err, err_row, sf.m, Rm, h, nord);
+    ep = bd_error_power<N, STRATEGY, OPTS>(c, err, err_row, sf.m, Rm, h, nord);
   }
 #pragma unroll
   for (int i = 0; i < N; ++i) pr.m[i] = Rm[i];
@@ -593,8 +619,8 @@ __device__ __forceinline__ double bd_step(const BdCtx<N, STRATEGY>& c, const BdS
 
 // ProbabilisticSolver.interpolate_fwd (solvers.py:205-269) from interp_from
 // `fr` to step_from `sf` at t1: writes checkpoint k, updates both slots.
-template <int N, int STRATEGY>
-__device__ __forceinline__ void bd_interp_beyond(const BdCtx<N, STRATEGY>& c, int k, double t1, BdSlot<N>& fr,
+template <int N, int STRATEGY, bool OPTS>
+__device__ __forceinline__ void bd_interp_beyond(const BdCtx<N, STRATEGY, OPTS>& c, int k, double t1, BdSlot<N>& fr,
                                                  BdScal& zf, BdSlot<N>& sf, BdScal& zs) {
   const pdq_config& cfg = c.a->cfg;
   const double* __restrict__ Q = c.a->Q;
@@ -605,7 +631,7 @@ __device__ __forceinline__ void bd_interp_beyond(const BdCtx<N, STRATEGY>& c, in
   const double s0 = lane_noise_scale(cfg, dt0, os);
   if (STRATEGY == PDQ_FILTER) {
     bd_marginalise_prior<N>(Q, P, PI, s0, fr.m, fr.L, Pm, PL);
-    bd_write_checkpoint<N, STRATEGY>(c, k, t1, Pm, PL, os, zs.nsteps, nullptr, false);
+    bd_write_checkpoint<N, STRATEGY, OPTS>(c, k, t1, Pm, PL, os, zs.nsteps, nullptr, false);
   } else {
     // ext_t = (Pm, PL) with the conditional interp_from.cond o bw (fixed
     // point; bw staged in step_from's conditional, rewritten below) or bw
@@ -625,7 +651,7 @@ __device__ __forceinline__ void bd_interp_beyond(const BdCtx<N, STRATEGY>& c, in
     double Ym[N], YL[N * N];
     lane_revert_prior<N, 1>(Q, P, PI, s1, Pm, PL, Ym, YL, cv<N>(sf.c));
     if (STRATEGY == PDQ_FIXEDPOINT) lane_merge<N, 1>(true, cv<N>(sf.c), cv<N>(sf.c), cv<N>(sf.c));
-    bd_write_checkpoint<N, STRATEGY>(c, k, t1, Pm, PL, os, zs.nsteps, &fr.c, false);
+    bd_write_checkpoint<N, STRATEGY, OPTS>(c, k, t1, Pm, PL, os, zs.nsteps, &fr.c, false);
     zf.ident = STRATEGY == PDQ_FIXEDPOINT;
     zs.ident = false;
   }
@@ -638,8 +664,8 @@ __device__ __forceinline__ void bd_interp_beyond(const BdCtx<N, STRATEGY>& c, in
 
 // userfriendly_output + strategy.finalize (solvers.py:439-480, 601-633,
 // 735-767; estimators_and_losses.py:380-391, 437-470), per block.
-template <int N, int STRATEGY>
-__device__ __forceinline__ void bd_finalize(const BdCtx<N, STRATEGY>& c, BdSlot<N>& sf, const BdScal& zs) {
+template <int N, int STRATEGY, bool OPTS>
+__device__ __forceinline__ void bd_finalize(const BdCtx<N, STRATEGY, OPTS>& c, BdSlot<N>& sf, const BdScal& zs) {
   const pdq_config& cfg = c.a->cfg;
   const pdq_solution& o = c.a->out;
   const int K = c.a->K, Km1 = K - 1, d = cfg.ode_dim, blk = c.g.lane;
@@ -720,11 +746,11 @@ __device__ __forceinline__ void bd_finalize(const BdCtx<N, STRATEGY>& c, BdSlot<
 // One instance on its lane group: init, the save_at / fixed-grid loop,
 // finalize, counters.  Every lane of the group runs it with the same
 // control flow.
-template <int N, int STRATEGY>
+template <int N, int STRATEGY, bool OPTS>
 __device__ __forceinline__ void bd_solve_instance(const BdArgs& a, const BdGroup& g, int inst) {
   const pdq_config& cfg = a.cfg;
   const int d = cfg.ode_dim, K = a.K, blk = g.lane;
-  BdCtx<N, STRATEGY> c;
+  BdCtx<N, STRATEGY, OPTS> c;
   c.a = &a;
   c.prm = a.params + (size_t)inst * cfg.n_params;
   c.g = g;
@@ -767,16 +793,16 @@ __device__ __forceinline__ void bd_solve_instance(const BdArgs& a, const BdGroup
   bd_copy<N>(pr, sf);
   zf = zs;
   zp = zs;
-  bd_write_checkpoint<N, STRATEGY>(c, 0, ts[0], sf.m, sf.L, 1.0, 0.0, nullptr, false);
+  bd_write_checkpoint<N, STRATEGY, OPTS>(c, 0, ts[0], sf.m, sf.L, 1.0, 0.0, nullptr, false);
   long attempts = 0, accepted = 0;
   int status = PDQ_STATUS_OK;
   if (a.mode == LMODE_FIXED_GRID) {
     for (int k = 1; k < K; ++k) {
       c.lin_set = pdq_lin_set(cfg, k - 1);
-      bd_step<N, STRATEGY>(c, sf, zs, pr, zp, ts[k] - ts[k - 1], false);
+      bd_step<N, STRATEGY, OPTS>(c, sf, zs, pr, zp, ts[k] - ts[k - 1], false);
       ++attempts;
       ++accepted;
-      bd_write_slot<N, STRATEGY>(c, k, pr, zp);
+      bd_write_slot<N, STRATEGY, OPTS>(c, k, pr, zp);
       bd_copy<N>(sf, pr);
       zs = zp;
     }
@@ -790,8 +816,10 @@ __device__ __forceinline__ void bd_solve_instance(const BdArgs& a, const BdGroup
         double h = dt;
         if (cfg.clip_dt) h = fmin(h, t1 - zs.t);
         c.lin_set = pdq_lin_set(cfg, accepted);
-        double ep = bd_step<N, STRATEGY>(c, sf, zs, pr, zp, h, true);
-        dt = bd_control(c, h, cstate, ep);
+        double ep = bd_step<N, STRATEGY, OPTS>(c, sf, zs, pr, zp, h, true);
+        // (the smoothers' two forms are the same computation: bd_lead)
+        if constexpr (STRATEGY == PDQ_FIXEDINTERVAL) dt = lane_control(cfg, h, cstate, ep);
+        else dt = bd_control(c, h, cstate, ep);
         ++att;
         ++attempts;
         if (!isfinite(ep) || !isfinite(dt)) {
@@ -811,11 +839,11 @@ __device__ __forceinline__ void bd_solve_instance(const BdArgs& a, const BdGroup
           zs = zp;
         }
       } else if (zs.t > t1 + cfg.eps) {
-        bd_interp_beyond<N, STRATEGY>(c, k, t1, fr, zf, sf, zs);
+        bd_interp_beyond<N, STRATEGY, OPTS>(c, k, t1, fr, zf, sf, zs);
         ++k;
       } else {
         // interpolate_fwd_at_t1 (solvers.py:271-315)
-        bd_write_slot<N, STRATEGY>(c, k, sf, zs);
+        bd_write_slot<N, STRATEGY, OPTS>(c, k, sf, zs);
         bd_copy<N>(fr, sf);
         zf = zs;
         if (STRATEGY == PDQ_FIXEDPOINT) {
@@ -826,7 +854,7 @@ __device__ __forceinline__ void bd_solve_instance(const BdArgs& a, const BdGroup
       }
     }
   }
-  if (status == PDQ_STATUS_OK) bd_finalize<N, STRATEGY>(c, sf, zs);
+  if (status == PDQ_STATUS_OK) bd_finalize<N, STRATEGY, OPTS>(c, sf, zs);
   if (blk == 0) {
     const pdq_solution& o = a.out;
     if (o.attempts) o.attempts[inst] = attempts;
@@ -882,7 +910,7 @@ __global__ void __launch_bounds__(64) bd_wave_kernel(BdArgs args) {
   g.red = nullptr;
   const int stride = gridDim.x * gpw;
   for (int inst = blockIdx.x * gpw + threadIdx.x / G; inst < a.n_inst; inst += stride)
-    bd_solve_instance<N, STRATEGY>(a, g, inst);
+    bd_solve_instance<N, STRATEGY, OPTS>(a, g, inst);
 }
 
 // One workgroup of G = 64 * ceil(d / 64) <= 512 lanes per instance, grid-
@@ -892,9 +920,11 @@ __global__ void __launch_bounds__(512) bd_block_kernel(BdArgs args) {
   __shared__ double y[2 * kBdMaxDim];
   __shared__ double red[kBdRedSize];
   const BdArgs a = bd_args<OPTS>(args, STRATEGY);
-  // zero: the partial sums of wavefronts that the workgroup does not have
-  if (threadIdx.x < kBdRedSize) red[threadIdx.x] = 0.0;
-  __syncthreads();
+  if constexpr (bd_lead<STRATEGY>) {
+    // zero: the partial sums of wavefronts that the workgroup does not have
+    if (threadIdx.x < kBdRedSize) red[threadIdx.x] = 0.0;
+    __syncthreads();
+  }
   BdGroup g;
   g.G = a.G;
   g.lane = threadIdx.x;
@@ -902,7 +932,7 @@ __global__ void __launch_bounds__(512) bd_block_kernel(BdArgs args) {
   g.y = y;
   g.red = red;
   for (int inst = blockIdx.x; inst < a.n_inst; inst += gridDim.x) {
-    bd_solve_instance<N, STRATEGY>(a, g, inst);
+    bd_solve_instance<N, STRATEGY, OPTS>(a, g, inst);
     // Every instance begins with the first of the alternating buffers: the next
     // one waits until all wavefronts have read this one's (on a fixed grid its
     // last barrier is the one before those reads).

@@ -124,7 +124,7 @@ void bd_emu_wave(const pdq::BdArgs& a, int inst) {
     g.multi = false;
     g.y = y.data();
     g.red = nullptr;
-    pdq::bd_solve_instance<N, S>(a, g, inst);
+    pdq::bd_solve_instance<N, S, true>(a, g, inst);
   });
 }
 
