@@ -867,7 +867,12 @@ __device__ __forceinline__ void bd_solve_instance(const BdArgs& a, const BdGroup
 // they fold in.  The kernels for every option hold five times the code
 // (burgers, d = 512: 13 900 instructions against 2 800) and keep twice as many
 // scalars as there are scalar registers.  The smoothers have no such kernels:
-// their slots' conditionals fill the vector registers either way.
+// built with the options folded in, the fixed-point kernel of nu = 5 (2.7 KB of
+// scratch per lane) gave results that differed from run to run on the device,
+// while all others and all kernels for every option reproduced.  On the CPU the
+// folded code equals the other bit for bit, does not depend on what its
+// variables start with, and shows no race between its lanes; the cause was not
+// found, so the smoothers are not folded.
 inline bool bd_default_options(const pdq_config& c, int mode) {
   return c.strategy == PDQ_FILTER && mode == LMODE_SAVE_AT && c.solver == PDQ_SOLVER_DYNAMIC &&
          c.constraint == PDQ_TS0 && c.error_estimator == PDQ_ERROR_RESIDUAL_STD &&

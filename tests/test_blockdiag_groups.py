@@ -7,6 +7,10 @@ Whatever it writes for the next instance must not reach the last reads of this o
 import numpy as np
 import pytest
 
+import test_gpu_parity as T
+
+torch = pytest.importorskip("torch")
+
 
 @pytest.fixture(scope="module")
 def emu():
@@ -37,3 +41,51 @@ def test_the_next_instance_waits_for_the_last_reads(emu, strategy, solver, K):
         emu.lib().pdqemu_set_lag(0, 0)
     for key, x in together.items():
         assert np.array_equal(x, np.concatenate([a[key] for a in alone]), equal_nan=True), key
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("d", [2, 33, 65, 130])
+@pytest.mark.parametrize("nu", [4, 5])
+@pytest.mark.parametrize("strategy", ["fixedpoint", "fixedinterval"])
+def test_high_order_smoothers(oracle, strategy, nu, d):
+    """The kernels with the most scratch memory per lane: against the oracle, and the same bits again."""
+    from probdiffeq_amd import capi
+
+    capi.require_device()
+    print(f"blockdiag smoother case: {strategy} nu={nu} d={d}", flush=True)
+    rng = np.random.default_rng(d)
+    B = 3
+    params, y0, times = np.full((B, 1), 1.5), rng.uniform(0.1, 0.9, size=(B, d)), np.tile(np.linspace(0.0, 3.0, 5), (B, 1))
+    cfg = capi.Config(factorisation="blockdiag", num_derivatives=nu, ode_dim=d, vector_field="logistic", n_params=1, strategy=strategy,
+                      rtol=1e-5, atol=1e-7)
+    T._compare(oracle, capi, cfg, params, y0, times)
+    P, S = T._dev(params), T._dev(times)
+    tc = capi.taylor_coefficients("logistic", P, T._dev(y0), 0.0, nu)
+    once = {k: v.cpu().numpy() for k, v in capi.solve(cfg, P, tc, S).items() if v is not None}
+    for _ in range(3):
+        for key, x in capi.solve(cfg, P, tc, S).items():
+            if x is not None:
+                assert np.array_equal(x.cpu().numpy(), once[key], equal_nan=once[key].dtype.kind == "f"), key
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("strategy", ["filter", "fixedinterval"])
+def test_more_instances_than_workgroups_on_a_fixed_grid(strategy):
+    """Workgroups that take several instances on a fixed grid (an odd number of steps): an instance's
+    result is the same bits as alone."""
+    from probdiffeq_amd import capi
+
+    capi.require_device()
+    print(f"blockdiag fixed grid case: {strategy}", flush=True)
+    d, nu, B = 130, 2, 3000
+    rng = np.random.default_rng(7)
+    y0 = rng.normal(size=(B, d))
+    cfg = capi.Config(factorisation="blockdiag", num_derivatives=nu, ode_dim=d, vector_field="burgers", n_params=2, strategy=strategy)
+    P, Y, S = T._dev(np.tile([0.05, 1.0 / d], (B, 1))), T._dev(y0), T._dev(np.tile(np.linspace(0.0, 1e-4, 4), (B, 1)))
+    tc = capi.taylor_coefficients("burgers", P, Y, 0.0, nu)
+    run = lambda rows: capi.solve(cfg, P[rows], tc[rows], S[rows], fixed_grid=True)
+    together = run(slice(None))
+    for rows in (slice(0, 64), slice(B - 64, B)):
+        alone = run(rows)
+        for key in ("mean", "chol"):
+            assert torch.equal(together[key][rows], alone[key]), (key, rows)
