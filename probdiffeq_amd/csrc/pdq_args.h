@@ -100,7 +100,7 @@ int launch_lane_adj(LmlArgs& a, int N, int D, hipStream_t st);
 // The same with the factors computed once for the batch (pdq_lane_lml_shared.h):
 // whether a solve takes that form, the doubles of the shared buffer and of the
 // lanes' scratch, the launch.
-bool lml_shared_takes(const pdq_config& c, int N, int D, int K, bool reverse);
+bool lml_shared_takes(const pdq_config& c, int N, int D);
 size_t lml_shared_doubles(int N, int K, int every);
 size_t lml_shared_scratch(int N, int D, int tpl, int K, int every, int n_inst, int G, bool reverse);
 int launch_lml_shared(LmlArgs& a, int N, int D, int tpl, bool reverse, hipStream_t st);

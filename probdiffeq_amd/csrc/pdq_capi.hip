@@ -602,14 +602,13 @@ int32_t pdq_lml_value_and_grad(const pdq_config* cfg, int32_t n_inst, const doub
     if (rc) return rc;
     CallBuffers bufs(st);
     double* tinit = nullptr;
-    double* adj_buf = nullptr;  // conditionals, node data, checkpoints and one segment per lane
-    HIP_TRY(bufs.alloc(&tinit, sizeof(double) * (size_t)n_inst * N * d * (1 + n_tan)));
-    const bool shared = pdq::lml_shared_takes(*cfg, N, d, K_grid, true);
-    double* shared_buf = nullptr;
-    if (shared) HIP_TRY(bufs.alloc(&shared_buf, sizeof(double) * pdq::lml_shared_doubles(N, K_grid, every)));
-    HIP_TRY(bufs.alloc(&adj_buf,
-                       sizeof(double) * (shared ? pdq::lml_shared_scratch(N, d, 0, K_grid, every, n_inst, 1, true)
-                                                : pdq::lane_adj_scratch_doubles(N, d, K_grid, every, n_inst))));
+    const size_t n_tinit = (size_t)n_inst * N * d * (1 + n_tan);
+    const bool shared = pdq::lml_shared_takes(*cfg, N, d);
+    const size_t n_shared = shared ? pdq::lml_shared_doubles(N, K_grid, every) : 0;
+    // conditionals, node data, checkpoints and one segment per lane
+    const size_t n_scratch = shared ? pdq::lml_shared_scratch(N, d, 0, K_grid, every, n_inst, 1, true)
+                                    : pdq::lane_adj_scratch_doubles(N, d, K_grid, every, n_inst);
+    HIP_TRY(bufs.alloc(&tinit, sizeof(double) * (n_tinit + n_shared + n_scratch)));
     rc = pdq::launch_taylor_tangents(cfg->vector_field, d, cfg->n_params, n_inst, cfg->num_derivatives, n_tan, params,
                                      y0, grid, tinit, st);
     if (rc) return rc;
@@ -629,8 +628,8 @@ int32_t pdq_lml_value_and_grad(const pdq_config* cfg, int32_t n_inst, const doub
     la.Q = m.Q;
     la.value = value;
     la.grad = grad;
-    la.scratch = adj_buf;
-    la.shared = shared_buf;
+    la.shared = tinit + n_tinit;
+    la.scratch = la.shared + n_shared;
     return shared ? pdq::launch_lml_shared(la, N, d, 0, true, st) : pdq::launch_lane_adj(la, N, d, st);
   }
   if (lane_ok && cfg->lanes_per_instance <= 1) {
@@ -644,14 +643,13 @@ int32_t pdq_lml_value_and_grad(const pdq_config* cfg, int32_t n_inst, const doub
     if (rc) return rc;
     CallBuffers bufs(st);
     double* tinit = nullptr;
-    double* cond_buf = nullptr;  // backward conditionals between observation nodes
-    HIP_TRY(bufs.alloc(&tinit, sizeof(double) * (size_t)n_inst * N * d * (1 + n_tan)));
-    const bool shared = pdq::lml_shared_takes(*cfg, N, d, K_grid, false);
-    double* shared_buf = nullptr;
-    if (shared) HIP_TRY(bufs.alloc(&shared_buf, sizeof(double) * pdq::lml_shared_doubles(N, K_grid, every)));
-    HIP_TRY(bufs.alloc(&cond_buf,
-                       sizeof(double) * (shared ? pdq::lml_shared_scratch(N, d, tpl, K_grid, every, n_inst, G, false)
-                                                : csz * (size_t)std::max(1, Kobs - 1) * n_lanes)));
+    const size_t n_tinit = (size_t)n_inst * N * d * (1 + n_tan);
+    const bool shared = pdq::lml_shared_takes(*cfg, N, d);
+    const size_t n_shared = shared ? pdq::lml_shared_doubles(N, K_grid, every) : 0;
+    // backward conditionals between observation nodes
+    const size_t n_scratch = shared ? pdq::lml_shared_scratch(N, d, tpl, K_grid, every, n_inst, G, false)
+                                    : csz * (size_t)std::max(1, Kobs - 1) * n_lanes;
+    HIP_TRY(bufs.alloc(&tinit, sizeof(double) * (n_tinit + n_shared + n_scratch)));
     rc = pdq::launch_taylor_tangents(cfg->vector_field, d, cfg->n_params, n_inst, cfg->num_derivatives, n_tan, params,
                                      y0, grid, tinit, st);
     if (rc) return rc;
@@ -671,8 +669,8 @@ int32_t pdq_lml_value_and_grad(const pdq_config* cfg, int32_t n_inst, const doub
     la.Q = m.Q;
     la.value = value;
     la.grad = grad;
-    la.scratch = cond_buf;
-    la.shared = shared_buf;
+    la.shared = tinit + n_tinit;
+    la.scratch = la.shared + n_shared;
     return shared ? pdq::launch_lml_shared(la, N, d, tpl, false, st) : pdq::launch_lane_lml(la, N, d, tpl, st);
   }
   pdq::Layout L = pdq::make_layout(*cfg, n_tan);

@@ -44,8 +44,7 @@ int launch_lml_nd(LmlArgs& a, hipStream_t st) {
 
 template <int N, int D, int TPL>
 int launch_lml_tpl(LmlArgs& a, hipStream_t st) {
-  if (a.cfg.solver == PDQ_SOLVER_DYNAMIC) return launch_lml_nd<N, D, TPL, PDQ_SOLVER_DYNAMIC>(a, st);
-  return launch_lml_nd<N, D, TPL, PDQ_SOLVER>(a, st);
+  return launch_lml_nd<N, D, TPL, PDQ_SOLVER_DYNAMIC>(a, st);
 }
 
 template <int N, int D>
@@ -97,10 +96,11 @@ int launch_lane_adj(LmlArgs& a, int N, int D, hipStream_t st) {
   return host_error(PDQ_ERR_UNSUPPORTED, "no adjoint LML kernel for nu + 1 = %d, d = %d", N, D);
 }
 
-// One tangent column per lane: G = n_tan lanes per instance.  Against three
-// per lane (G = 2) this is 1.44x faster on the C5 batch (13.9 vs 20.0 ms):
-// the extra lanes are free (the batch occupies a fraction of the CUs) and each
-// lane's mean recursions shrink from 8 to 4 columns.
+// One tangent column per lane: G = n_tan lanes per instance.  The extra lanes
+// are free (1024 instances occupy a fraction of the CUs) and each lane's mean
+// recursions shrink from 8 to 4 columns: against three per lane (G = 2), when
+// every lane still computed its own factors, 13.9 against 20.0 ms (1024
+// instances, nu = 3, 2000 steps).
 int lane_lml_tangents_per_lane(int n_tan) { return n_tan == 0 ? 0 : 1; }
 
 bool lane_lml_supported(int N, int D, int solver) {
@@ -113,7 +113,8 @@ size_t lane_lml_cond_size(int N, int D, int tpl) {
 }
 
 int launch_lane_lml(LmlArgs& a, int N, int D, int tpl, hipStream_t st) {
-  if (D == 2) {
+  // (PDQ_SOLVER's factors are the batch's: pdq_lane_lml_shared.h)
+  if (D == 2 && a.cfg.solver == PDQ_SOLVER_DYNAMIC) {
     if (N == 4) return launch_lml_shape<4, 2>(a, tpl, st);
     if (N == 5) return launch_lml_shape<5, 2>(a, tpl, st);
   }

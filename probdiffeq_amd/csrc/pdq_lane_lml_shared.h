@@ -445,6 +445,9 @@ struct LmlAdjShared {
 // means; what a part reads was written by earlier launches.
 struct LmlParts {
   int c0, c1, r0, r1, j0, j1, m0, m1;
+  // block 0 runs the chain, then the reverts and the merges of the same steps
+  // (at most 64: one per lane); there are no other blocks for them
+  int together;
   __host__ __device__ int reverts() const { return (r1 - r0 + 63) / 64; }
   __host__ __device__ int merges() const { return (j1 - j0 + 63) / 64; }
 };
@@ -547,17 +550,22 @@ __global__ void __launch_bounds__(64) lml_parts_kernel(LmlArgs args, LmlParts w)
   __shared__ double lds[lp > ls ? lp : ls];
   const LmlArgs a = lml_shared_args(args, FIELD);
   int b = blockIdx.x;
+  const bool together = w.together != 0;
   if (b == 0) {
     if (w.c0 < w.c1) lml_chain<N>(a, a.cfg, w.c0, w.c1, lds);
-    return;
+    if (!together) return;
+    __syncthreads();  // (the lanes' stores are the other lanes' loads)
+  } else {
+    b -= 1;
   }
-  b -= 1;
   if (b < w.reverts()) {
     const int s = w.r0 + b * 64 + (int)threadIdx.x;
     if (s < w.r1) lml_revert<N>(a, s);
-    return;
+    if (!together) return;
+    __syncthreads();
+  } else {
+    b -= w.reverts();
   }
-  b -= w.reverts();
   if (b < w.merges()) {
     const int j = w.j0 + b * 64 + (int)threadIdx.x;
     if (j < w.j1) lml_merge<N>(a, j);

@@ -12,7 +12,9 @@ template <int N>
 int launch_lml_shared_n(LmlArgs& a, int tpl, bool reverse, hipStream_t st);
 
 #ifdef PDQ_LML_SHARED_DEFINE_LAUNCH
-// The factors and the means' pass, in chunks of whole intervals: launch i runs
+// The factors and the means' pass.  Up to 64 steps: the factors in one launch
+// (a step, or an interval, per lane of one wavefront), the means in a second:
+// what such a call costs is its launches.  Beyond, in chunks of whole intervals: launch i runs
 // the chain of chunk i, the reverts of the one before, its predecessor's merges
 // and the means of the one before that.  The first three launches run without
 // means (24 chunks: an eighth of the chain's time); a chunk of fewer than 64
@@ -27,12 +29,20 @@ int launch_lml_parts(const LmlArgs& a, hipStream_t st) {
   const int n = (steps + chunk - 1) / chunk, lanes = (int)(((long)a.n_inst * a.G + 63) / 64);
   auto from = [&](int i) { return i < 0 || i >= n ? 0 : i * chunk; };
   auto to = [&](int i) { return i < 0 || i >= n ? 0 : std::min(steps, (i + 1) * chunk); };
-  for (int i = 0; i < n + 3; ++i) {
-    const LmlParts w{from(i),     to(i),     from(i - 1), to(i - 1), from(i - 2) / a.every, to(i - 2) / a.every,
-                     from(i - 3), to(i - 3)};
-    const int grid = 1 + w.reverts() + w.merges() + (w.m0 < w.m1 ? lanes : 0);
+  auto launch = [&](const LmlParts& w, int grid) {
     hipLaunchKernelGGL((lml_parts_kernel<N, 2, TPL, FIELD, ADJOINT>), dim3(grid), dim3(64), 0, st, a, w);
     PDQ_HIP_TRY(hipGetLastError());
+    return (int)PDQ_OK;
+  };
+  if (steps <= 64) {
+    const int rc = launch(LmlParts{0, steps, 0, steps, 0, steps / a.every, 0, 0, 1}, 1);
+    return rc ? rc : launch(LmlParts{0, 0, 0, 0, 0, 0, 0, steps, 0}, 1 + lanes);
+  }
+  for (int i = 0; i < n + 3; ++i) {
+    const LmlParts w{from(i),     to(i),     from(i - 1), to(i - 1), from(i - 2) / a.every, to(i - 2) / a.every,
+                     from(i - 3), to(i - 3), 0};
+    const int rc = launch(w, 1 + w.reverts() + w.merges() + (w.m0 < w.m1 ? lanes : 0));
+    if (rc) return rc;
   }
   return PDQ_OK;
 }

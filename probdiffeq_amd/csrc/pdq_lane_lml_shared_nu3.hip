@@ -6,12 +6,15 @@ namespace pdq {
 
 template int launch_lml_shared_n<4>(LmlArgs&, int, bool, hipStream_t);
 
-// Four launches against one: below 8 grid steps the value and the forward
-// gradient of the lane kernels are as fast or faster (nu = 3, gradient of 1..5
-// instances: 2 steps 79 us against 99, 6 steps 94 / 95, 16 steps 132 / 128, 34
-// steps 280 / 200); the adjoint's never is (2 steps: 122 / 97).
-bool lml_shared_takes(const pdq_config& c, int N, int D, int K, bool reverse) {
-  return D == 2 && (N == 4 || N == 5) && c.solver == PDQ_SOLVER && (reverse || K > 8);
+// PDQ_SOLVER takes this form at every size.  Us of a call, the lane kernels that
+// compute every lane's own factors / this form (the factors of up to 64 steps in
+// one launch, the call's buffers in one allocation): nu = 3, value, 1 step 55 / 49
+// (1 instance), 64 / 50 (1024), 8 steps 68 / 56, 64 steps 261 / 183; gradient by
+// tangents, 1 step 64 / 55, 8 steps of 8192 instances 164 / 76; nu = 4, 8 steps
+// 131 / 95; the adjoint, nu = 3, 1 step 66 / 58, 4 steps 94 / 67, nu = 4, 1 step
+// 81 / 61.
+bool lml_shared_takes(const pdq_config& c, int N, int D) {
+  return D == 2 && (N == 4 || N == 5) && c.solver == PDQ_SOLVER;
 }
 
 size_t lml_shared_doubles(int N, int K, int every) {
