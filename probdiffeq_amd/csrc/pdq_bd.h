@@ -938,10 +938,11 @@ __global__ void __launch_bounds__(512) bd_block_kernel(BdArgs args) {
   g.red = red;
   for (int inst = blockIdx.x; inst < a.n_inst; inst += gridDim.x) {
     bd_solve_instance<N, STRATEGY, OPTS>(a, g, inst);
-    // Every instance begins with the first of the alternating buffers: the next
-    // one waits until all wavefronts have read this one's (on a fixed grid its
-    // last barrier is the one before those reads).
-    __syncthreads();
+    // Every instance begins with the first of the alternating buffers.  In an
+    // adaptive solve a group sum's barrier lies behind the last reads of them;
+    // on a fixed grid the last barrier is the one before those reads, and the
+    // next instance waits until all wavefronts have made them.
+    if (a.mode == LMODE_FIXED_GRID) __syncthreads();
   }
 }
 

@@ -21,8 +21,12 @@ def emu():
     return M
 
 
-@pytest.mark.parametrize("strategy,solver,K", [("filter", "solver", 2), ("filter", "dynamic", 4), ("fixedinterval", "mle", 2)])
-def test_the_next_instance_waits_for_the_last_reads(emu, strategy, solver, K):
+@pytest.mark.parametrize(
+    "strategy,solver,K,grid",
+    [("filter", "solver", 2, True), ("filter", "dynamic", 4, True), ("fixedinterval", "mle", 2, True),
+     ("filter", "dynamic", 2, False), ("fixedpoint", "dynamic", 2, False), ("fixedinterval", "solver", 2, False)],
+)
+def test_the_next_instance_waits_for_the_last_reads(emu, strategy, solver, K, grid):
     from probdiffeq_amd import capi
 
     d, nu, B = 66, 1, 3
@@ -32,11 +36,13 @@ def test_the_next_instance_waits_for_the_last_reads(emu, strategy, solver, K):
     f = -y0 * (np.roll(y0, -1, 1) - np.roll(y0, 1, 1)) / (2 * dx) + 0.05 * (np.roll(y0, -1, 1) - 2 * y0 + np.roll(y0, 1, 1)) / dx**2
     tc = np.stack([y0, f], axis=1).reshape(B, -1)
     p, t = np.tile([0.05, dx], (B, 1)), np.tile(np.linspace(0.0, 1e-4, K), (B, 1))
-    cfg = capi.Config(factorisation="blockdiag", num_derivatives=nu, ode_dim=d, vector_field="burgers", n_params=2, strategy=strategy, solver=solver)
-    alone = [emu.solve(cfg, p[i : i + 1], tc[i : i + 1], t[i : i + 1], fixed_grid=True) for i in range(B)]
+    cfg = capi.Config(factorisation="blockdiag", num_derivatives=nu, ode_dim=d, vector_field="burgers", n_params=2, strategy=strategy, solver=solver,
+                      dt0=4e-5, rtol=1e-3, atol=1e-4)
+    alone = [emu.solve(cfg, p[i : i + 1], tc[i : i + 1], t[i : i + 1], fixed_grid=grid) for i in range(B)]
     emu.lib().pdqemu_set_lag(64, 20000)
     try:
-        together = emu.solve(cfg, p, tc, t, fixed_grid=True)
+        together = emu.solve(cfg, p, tc, t, fixed_grid=grid)
+        print(together["attempts"])
     finally:
         emu.lib().pdqemu_set_lag(0, 0)
     for key, x in together.items():
