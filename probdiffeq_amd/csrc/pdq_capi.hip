@@ -351,6 +351,11 @@ int solve_run(const pdq_config* cfg, int n_inst, const double* params, const dou
   return rc;
 }
 
+// Doubles rounded up to whole 256 bytes: where one buffer holds several parts,
+// each begins as an allocation of its own would (a wavefront's row of 64 lanes'
+// doubles then covers whole cache lines).
+size_t whole_lines(size_t doubles) { return (doubles + 31) / 32 * 32; }
+
 int solve_common(const pdq_config* cfg, int n_inst, const double* params, const double* tcoeffs,
                  const double* times, int K, const pdq_solution* out, void* stream, int mode) {
   int rc = solve_validate(cfg, n_inst, params, tcoeffs, times, K, out);
@@ -602,9 +607,9 @@ int32_t pdq_lml_value_and_grad(const pdq_config* cfg, int32_t n_inst, const doub
     if (rc) return rc;
     CallBuffers bufs(st);
     double* tinit = nullptr;
-    const size_t n_tinit = (size_t)n_inst * N * d * (1 + n_tan);
+    const size_t n_tinit = whole_lines((size_t)n_inst * N * d * (1 + n_tan));
     const bool shared = pdq::lml_shared_takes(*cfg, N, d);
-    const size_t n_shared = shared ? pdq::lml_shared_doubles(N, K_grid, every) : 0;
+    const size_t n_shared = shared ? whole_lines(pdq::lml_shared_doubles(N, K_grid, every)) : 0;
     // conditionals, node data, checkpoints and one segment per lane
     const size_t n_scratch = shared ? pdq::lml_shared_scratch(N, d, 0, K_grid, every, n_inst, 1, true)
                                     : pdq::lane_adj_scratch_doubles(N, d, K_grid, every, n_inst);
@@ -643,9 +648,9 @@ int32_t pdq_lml_value_and_grad(const pdq_config* cfg, int32_t n_inst, const doub
     if (rc) return rc;
     CallBuffers bufs(st);
     double* tinit = nullptr;
-    const size_t n_tinit = (size_t)n_inst * N * d * (1 + n_tan);
+    const size_t n_tinit = whole_lines((size_t)n_inst * N * d * (1 + n_tan));
     const bool shared = pdq::lml_shared_takes(*cfg, N, d);
-    const size_t n_shared = shared ? pdq::lml_shared_doubles(N, K_grid, every) : 0;
+    const size_t n_shared = shared ? whole_lines(pdq::lml_shared_doubles(N, K_grid, every)) : 0;
     // backward conditionals between observation nodes
     const size_t n_scratch = shared ? pdq::lml_shared_scratch(N, d, tpl, K_grid, every, n_inst, G, false)
                                     : csz * (size_t)std::max(1, Kobs - 1) * n_lanes;
