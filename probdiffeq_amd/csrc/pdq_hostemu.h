@@ -37,6 +37,12 @@ inline int atomicAdd(int* p, int v) {
   __atomic_fetch_add(&pdq_emu_atomics, 1, __ATOMIC_RELAXED);
   return __atomic_fetch_add(p, v, __ATOMIC_RELAXED);
 }
+template <class T>
+inline void pdq_emu_store(T v, T* p) {
+  *p = v;
+}
+#define __builtin_nontemporal_store pdq_emu_store
+#define __builtin_amdgcn_readfirstlane(x) (x)
 #define __builtin_amdgcn_fence(a, b) ((void)0)
 #define __builtin_amdgcn_wave_barrier() ((void)0)
 

@@ -121,7 +121,6 @@ __device__ __forceinline__ void lml_chain_step(const pdq_config& cfg, const doub
   lane_update<N, 1>(cfg, &b, 0.0, none, PL, Xm, L, &mo, oL, gain);
 }
 
-#ifndef PDQ_HOST_EMU
 // The factors' chain from step b to step e (one wavefront; the factor before a
 // later step than the first is where the previous call left it).
 template <int N>
@@ -265,7 +264,6 @@ __device__ __forceinline__ void lml_merge(const LmlArgs& a, int j) {
     c[SH::cto + i] = self.to(i);
   }
 }
-#endif
 
 // One step of the means: m and the running conditional's noise mean r, from
 // the step's record.
@@ -343,7 +341,6 @@ struct LmlParams {
   }
 };
 
-#ifndef PDQ_HOST_EMU
 // A tile of records on its way to LDS.
 template <int N>
 struct LmlStage {
@@ -418,7 +415,6 @@ __device__ __forceinline__ LmlArgs lml_shared_args(const LmlArgs& args, int fiel
   return a;
 }
 
-#endif
 
 // The adjoint's storage per lane (doubles): interval means, node data,
 // adjoints of the interval means, checkpoints of the mean.
@@ -437,7 +433,20 @@ struct LmlAdjShared {
   }
 };
 
-#ifndef PDQ_HOST_EMU
+// The doubles of the shared buffer and of the lanes' scratch.
+inline size_t lml_shared_size(int N, int K, int every) {
+  return N == 4 ? LmlShared<4>(K, every).size : LmlShared<5>(K, every).size;
+}
+
+inline size_t lml_shared_scratch_size(int N, int D, int tpl, int K, int every, int n_inst, int G, bool reverse) {
+  if (reverse) {
+    const size_t lanes = (size_t)((n_inst + 63) / 64) * 64;
+    return (N == 4 ? LmlAdjShared<4, 2>(K, every).size : LmlAdjShared<5, 2>(K, every).size) * lanes;
+  }
+  // an interval's noise mean per interval; m and r between two launches
+  return ((size_t)((K - 1) / every) + 2) * N * D * (1 + tpl) * n_inst * G;
+}
+
 // What one launch does, each part on blocks of its own: the chain of steps
 // c0 .. c1, the reverts of steps r0 .. r1, the merges of intervals j0 .. j1 and
 // the means' pass of steps m0 .. m1.  A launch's parts work on four successive
@@ -445,12 +454,40 @@ struct LmlAdjShared {
 // means; what a part reads was written by earlier launches.
 struct LmlParts {
   int c0, c1, r0, r1, j0, j1, m0, m1;
-  // block 0 runs the chain, then the reverts and the merges of the same steps
-  // (at most 64: one per lane); there are no other blocks for them
-  int together;
   __host__ __device__ int reverts() const { return (r1 - r0 + 63) / 64; }
   __host__ __device__ int merges() const { return (j1 - j0 + 63) / 64; }
 };
+
+// The launches of `steps` grid steps with `lanes` workgroups of means, until one
+// fails (not 0).  Up to 64 steps: factors() for all of them (lml_factors_kernel),
+// then the means; what such a call costs is its launches.  Beyond, run(parts,
+// workgroups) in chunks of whole intervals: launch i runs the chain of chunk i, the reverts of the one before,
+// its predecessor's merges and the means of the one before that.  The first three
+// launches run without means (24 chunks: an eighth of the chain's time); a chunk
+// of fewer than 64 steps (70 us) would not cover its launch, and with fewer than
+// six the three launches that fill and drain take what the overlap gives (nu = 4,
+// 200 steps, gradient: 0.83 ms in four chunks, 0.77 in one).
+template <class F0, class F>
+int lml_for_launches(int steps, int every, int lanes, F0&& factors, F&& run) {
+  if (steps <= 64) {
+    const int rc = factors();
+    return rc ? rc : run(LmlParts{0, 0, 0, 0, 0, 0, 0, steps}, 1 + lanes);
+  }
+  const int target = (steps + 23) / 24 > 64 ? (steps + 23) / 24 : 64;
+  const long whole = ((long)target + every - 1) / every * every;
+  int chunk = whole < steps ? (int)whole : steps;
+  if ((steps + chunk - 1) / chunk < 6) chunk = steps;
+  const int n = (steps + chunk - 1) / chunk;
+  auto from = [&](int i) { return i < 0 || i >= n ? 0 : i * chunk; };
+  auto to = [&](int i) { return i < 0 || i >= n ? 0 : (steps - from(i) < chunk ? steps : from(i) + chunk); };
+  for (int i = 0; i < n + 3; ++i) {
+    const LmlParts w{from(i),     to(i),     from(i - 1), to(i - 1), from(i - 2) / every, to(i - 2) / every,
+                     from(i - 3), to(i - 3)};
+    const int rc = run(w, 1 + w.reverts() + w.merges() + (w.m0 < w.m1 ? lanes : 0));
+    if (rc) return rc;
+  }
+  return 0;
+}
 
 // The means' pass of a lane per (instance, tangent group) and, after the last
 // step, the reverse scan and the outputs.  A lane beyond the last one computes
@@ -544,28 +581,37 @@ __device__ __forceinline__ void lml_means_part_adjoint(const LmlArgs& a, const L
   }
 }
 
+// All factors of at most 64 steps by one wavefront: the chain, then a step, then
+// an interval, per lane (the barriers: a lane's stores are other lanes' loads).
+template <int N>
+__global__ void __launch_bounds__(64) lml_factors_kernel(LmlArgs args) {
+  __shared__ double lds[64 * (2 * N + 2)];
+  const LmlArgs a = lml_shared_args(args, args.cfg.vector_field);
+  const int steps = a.K - 1, i = threadIdx.x;
+  lml_chain<N>(a, a.cfg, 0, steps, lds);
+  __syncthreads();
+  if (i < steps) lml_revert<N>(a, i);
+  __syncthreads();
+  if (i < steps / a.every) lml_merge<N>(a, i);
+}
+
 template <int N, int D, int TPL, int FIELD, bool ADJOINT>
 __global__ void __launch_bounds__(64) lml_parts_kernel(LmlArgs args, LmlParts w) {
   constexpr int lp = 64 * (2 * N + 2), ls = LmlStage<N>::n;
   __shared__ double lds[lp > ls ? lp : ls];
   const LmlArgs a = lml_shared_args(args, FIELD);
   int b = blockIdx.x;
-  const bool together = w.together != 0;
   if (b == 0) {
     if (w.c0 < w.c1) lml_chain<N>(a, a.cfg, w.c0, w.c1, lds);
-    if (!together) return;
-    __syncthreads();  // (the lanes' stores are the other lanes' loads)
-  } else {
-    b -= 1;
+    return;
   }
+  b -= 1;
   if (b < w.reverts()) {
     const int s = w.r0 + b * 64 + (int)threadIdx.x;
     if (s < w.r1) lml_revert<N>(a, s);
-    if (!together) return;
-    __syncthreads();
-  } else {
-    b -= w.reverts();
+    return;
   }
+  b -= w.reverts();
   if (b < w.merges()) {
     const int j = w.j0 + b * 64 + (int)threadIdx.x;
     if (j < w.j1) lml_merge<N>(a, j);
@@ -720,6 +766,5 @@ __global__ void __launch_bounds__(128) lml_adjoint_kernel(LmlArgs args) {
     if (active) a.grad[(size_t)inst * ntan + q] = g;
   }
 }
-#endif
 
 }  // namespace pdq

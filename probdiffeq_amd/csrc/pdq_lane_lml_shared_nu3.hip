@@ -17,17 +17,10 @@ bool lml_shared_takes(const pdq_config& c, int N, int D) {
   return D == 2 && (N == 4 || N == 5) && c.solver == PDQ_SOLVER;
 }
 
-size_t lml_shared_doubles(int N, int K, int every) {
-  return N == 4 ? LmlShared<4>(K, every).size : LmlShared<5>(K, every).size;
-}
+size_t lml_shared_doubles(int N, int K, int every) { return lml_shared_size(N, K, every); }
 
 size_t lml_shared_scratch(int N, int D, int tpl, int K, int every, int n_inst, int G, bool reverse) {
-  if (reverse) {
-    const size_t lanes = (size_t)((n_inst + 63) / 64) * 64;
-    return (N == 4 ? LmlAdjShared<4, 2>(K, every).size : LmlAdjShared<5, 2>(K, every).size) * lanes;
-  }
-  // an interval's noise mean per interval; m and r between two launches
-  return ((size_t)((K - 1) / every) + 2) * N * D * (1 + tpl) * n_inst * G;
+  return lml_shared_scratch_size(N, D, tpl, K, every, n_inst, G, reverse);
 }
 
 int launch_lml_shared(LmlArgs& a, int N, int D, int tpl, bool reverse, hipStream_t st) {

@@ -54,31 +54,11 @@ __device__ __forceinline__ void lane_offgrid_marginal(const OffgridArgs& a, doub
   }
 }
 
-#ifdef PDQ_HOST_EMU
-template <int N, int D, int STRATEGY>
-void lane_offgrid(const OffgridArgs& a, size_t q) {
-  const int K = a.K;
-  const size_t inst = q / (size_t)a.n_query;
-  const double* ts = a.times + inst * K;
-  const double t = a.t_query[q];
-  const int i = lane_offgrid_interval(ts, K, t);
-  const size_t r0 = inst * K + (i - 1), r1 = inst * K + i;
-  lane_offgrid_marginal<N, D, STRATEGY>(
-      a, t, ts[i - 1], ts[i], a.output_scale[r1], (STRATEGY == PDQ_FILTER ? a.mean : a.filt_mean) + r0 * N * D,
-      (STRATEGY == PDQ_FILTER ? a.chol : a.filt_chol) + r0 * N * N,
-      [&](double* m1, double* L1) {
-        for (int e = 0; e < N * D; ++e) m1[e] = a.mean[r1 * N * D + e];
-        for (int e = 0; e < N * N; ++e) L1[e] = a.chol[r1 * N * N + e];
-      },
-      a.mean_out + q * N * D, a.chol_out + q * N * N);
-}
-#else
-
 // Two neighbouring doubles (8-byte aligned).
 struct alignas(8) OffgridPair {
   double v[2];
 };
-typedef double OffgridVec __attribute__((ext_vector_type(2), aligned(8)));
+typedef double OffgridVec __attribute__((vector_size(16), aligned(8)));
 
 // One wavefront's 64 queries.  What bounds them beside the smoother's two
 // reverts per query (2650 FP64 instructions at nu = 4) is the memory
@@ -222,6 +202,5 @@ __global__ void __launch_bounds__(64, 2) lane_offgrid_kernel(OffgridArgs a) {
   for (size_t q = (size_t)blockIdx.x * 64; q < total; q += stride)
     wave_offgrid<N, D, STRATEGY>(a, q, (int)(total - q < 64 ? total - q : 64), lds, rows);
 }
-#endif
 
 }  // namespace pdq

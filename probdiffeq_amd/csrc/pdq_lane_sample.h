@@ -22,7 +22,7 @@ struct alignas(8) SamplePair {
   double v[2];
 };
 // the same as a vector, for stores that leave the L2 to the reads
-typedef double SampleVec __attribute__((ext_vector_type(2), aligned(8)));
+typedef double SampleVec __attribute__((vector_size(16), aligned(8)));
 template <int n>
 __device__ __forceinline__ void sample_load(const double* __restrict__ src, double* dst) {
 #pragma unroll
@@ -106,20 +106,6 @@ __device__ __forceinline__ void lane_sample_steps(const SampleArgs& a, size_t c0
   }
 }
 
-// The whole scan that way.
-template <int N, int D>
-__device__ __forceinline__ void lane_sample(const SampleArgs& a, size_t gid) {
-  const int K = a.K;
-  const size_t inst = gid / (size_t)a.n_samples, c0 = inst * (size_t)(K - 1);
-  const double* __restrict__ z = a.base + gid * K * N;
-  double* __restrict__ out = a.samples + gid * K * N * D;
-  double x[N * D];
-  lane_sample_terminal<N, D>(a, inst, z + (size_t)(K - 1) * N, x);
-  sample_store<N * D>(out + (size_t)(K - 1) * N * D, x);
-  lane_sample_steps<N, D>(a, c0, K - 2, 0, z, out, x);
-}
-
-#ifndef PDQ_HOST_EMU
 // One wavefront's 64 samples, kSampleTile points at a time.  What bounds the
 // scan is memory: it reads the draws and writes the samples once, but a lane's
 // own accesses to them are rows apart (a cache line per lane and instruction,
@@ -309,6 +295,5 @@ __global__ void __launch_bounds__(64) lane_sample_kernel(SampleArgs a) {
   for (size_t g = (size_t)blockIdx.x * 64; g < total; g += stride)
     wave_sample<N, D, STAGED>(a, g, (int)(total - g < 64 ? total - g : 64), lds);
 }
-#endif
 
 }  // namespace pdq

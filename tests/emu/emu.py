@@ -116,6 +116,21 @@ def lml(cfg, params, y0, grid, every, data, stds, average=True, grad=True, kerne
     return value, g
 
 
+def lml_shared(cfg, params, y0, grid, every, data, stds, average=True, grad=True, reverse=False):
+    """The kernels of the LML with the batch's factors computed once (pdq_lane_lml_shared.h), in the
+    device library's launches."""
+    params, y0, grid, data, stds = (np.ascontiguousarray(x, dtype=np.float64) for x in (params, y0, grid, data, stds))
+    B = params.shape[0]
+    value = np.zeros(B)
+    g = np.zeros((B, params.shape[1] + y0.shape[1])) if grad else None
+    c = cfg.c(host=True)
+    P = ctypes.c_void_p
+    rc = lib().pdqemu_lml_shared(ctypes.byref(c), B, P(params.ctypes.data), P(y0.ctypes.data), P(grid.ctypes.data), grid.size, every, P(data.ctypes.data), P(stds.ctypes.data), int(average), P(value.ctypes.data), P(g.ctypes.data) if grad else None, int(reverse))
+    if rc:
+        raise RuntimeError(f"emulation rc {rc}")
+    return value, g
+
+
 def lml_adjoint(cfg, params, y0, grid, every, data, stds, average=True, grad=True, lanes=3):
     """The reverse-mode adjoint LML kernel's code (pdq_lane_adjoint.h) on the CPU; `lanes` scratch
     columns shared by the instances in grid-stride order, as on the device."""
@@ -154,18 +169,22 @@ def offgrid(cfg, times, sol, t_query):
     return mean_out, chol_out
 
 
-def sample(cfg, sol, base):
-    """The posterior sampler's code on the CPU: sol = one instance's term_*/cond_* (solve()'s layouts),
-    base (S, K, n) with n the covariance dimension.  Returns (S, K, mean_size)."""
+def sample(cfg, sol, base, staged=None):
+    """The posterior sampler's code on the CPU: sol = instances' term_*/cond_* (solve()'s layouts, without
+    the batch axis for one instance), base (S, K, n) or (B, S, K, n) with n the covariance dimension.
+    Returns (S, K, mean_size) or (B, S, K, mean_size).  staged: the lane kernel reads a tile's
+    conditionals together (default: from 16 samples on)."""
     arr = lambda x: np.ascontiguousarray(x, dtype=np.float64)
     base = arr(base)
-    S, K, _ = base.shape
-    out = np.zeros((S, K, cfg.mean_size))
+    B = base.shape[0] if base.ndim == 4 else 1
+    S, K, _ = base.shape[-3:]
+    out = np.zeros((*base.shape[:-1], cfg.mean_size))
     keys = ("term_mean", "term_chol", "cond_A", "cond_mean", "cond_chol", "cond_tl", "cond_to")
     arrs = [arr(sol[k]) for k in keys]
     P = ctypes.c_void_p
     c = cfg.c(host=True)
-    rc = lib().pdqemu_sample(ctypes.byref(c), 1, K, *[P(a.ctypes.data) for a in arrs], S, P(base.ctypes.data), P(out.ctypes.data))
+    staged = S >= 16 if staged is None else staged
+    rc = lib().pdqemu_sample(ctypes.byref(c), B, K, *[P(a.ctypes.data) for a in arrs], S, P(base.ctypes.data), P(out.ctypes.data), int(staged))
     if rc:
         raise RuntimeError(f"emulation rc {rc}")
     return out

@@ -17,6 +17,7 @@
 #include "../../probdiffeq_amd/csrc/pdq_lane.h"
 #include "../../probdiffeq_amd/csrc/pdq_lane_adjoint.h"
 #include "../../probdiffeq_amd/csrc/pdq_lane_lml.h"
+#include "../../probdiffeq_amd/csrc/pdq_lane_lml_shared.h"
 #include "../../probdiffeq_amd/csrc/pdq_lane_offgrid.h"
 #include "../../probdiffeq_amd/csrc/pdq_lane_sample.h"
 #include "../../probdiffeq_amd/csrc/pdq_sample_generic.h"
@@ -35,20 +36,22 @@ std::barrier<>* g_group_barrier = nullptr;
 double g_group_xchg[pdq::kBdMaxDim];
 thread_local int t_group_lane = 0;
 thread_local std::barrier<>* t_wave_barrier = nullptr;
-// Lanes from g_lag_lane on leave every barrier of the group g_lag_us late (a
-// wavefront that the others run ahead of); 0 us: none does.
-int g_lag_lane = 0, g_lag_us = 0;
+// Lanes g_lag_first .. g_lag_end - 1 leave every barrier of the group g_lag_us
+// late (a wavefront that the others run ahead of); 0 us: none does.
+int g_lag_first = 0, g_lag_end = 0, g_lag_us = 0;
 }  // namespace
 
-extern "C" void pdqemu_set_lag(int first_lane, int microseconds) {
-  g_lag_lane = first_lane;
+extern "C" void pdqemu_set_lag(int first_lane, int end_lane, int microseconds) {
+  g_lag_first = first_lane;
+  g_lag_end = end_lane;
   g_lag_us = microseconds;
 }
 
 void pdq_emu_group_barrier() {
   if (!g_group_barrier) return;
   g_group_barrier->arrive_and_wait();
-  if (g_lag_us > 0 && t_group_lane >= g_lag_lane) std::this_thread::sleep_for(std::chrono::microseconds(g_lag_us));
+  if (g_lag_us > 0 && t_group_lane >= g_lag_first && t_group_lane < g_lag_end)
+    std::this_thread::sleep_for(std::chrono::microseconds(g_lag_us));
 }
 
 void pdq_emu_wave_barrier() {
@@ -609,8 +612,70 @@ int pdqemu_lml_adjoint(const pdq_config* cfg, int n_inst, const double* params, 
   return 0;
 }
 
-// The off-grid marginal kernel (pdq_lane_offgrid.h) on the CPU, one query
-// after another.  Returns 2 for a shape or strategy it does not cover.
+}  // extern "C"
+
+namespace {
+template <int N, int FIELD>
+void lml_shared_emu(pdq::LmlArgs& a, bool reverse) {
+  const int lanes = (int)(((size_t)a.n_inst * a.G + 63) / 64);
+  auto factors = [&] {
+    emu_launch(1, 64, [&] { pdq::lml_factors_kernel<N>(a); });
+    return 0;
+  };
+  pdq::lml_for_launches(a.K - 1, a.every, lanes, factors, [&](const pdq::LmlParts& w, int grid) {
+    emu_launch(grid, 64, [&] {
+      if (reverse) pdq::lml_parts_kernel<N, 2, 0, FIELD, true>(a, w);
+      else if (a.n_tan) pdq::lml_parts_kernel<N, 2, 1, FIELD, false>(a, w);
+      else pdq::lml_parts_kernel<N, 2, 0, FIELD, false>(a, w);
+    });
+    return 0;
+  });
+  if (reverse) emu_launch((a.n_inst + 63) / 64, 128, [&] { pdq::lml_adjoint_kernel<N, 2, FIELD>(a); });
+}
+}  // namespace
+
+extern "C" {
+
+// The LML with the batch's factors computed once (pdq_lane_lml_shared.h): its
+// kernels, in the device library's launches.  Lotka-Volterra, nu = 3, 4.
+int pdqemu_lml_shared(const pdq_config* cfg, int n_inst, const double* params, const double* y0, const double* grid,
+                      int K, int every, const double* data, const double* stds, int average, double* value,
+                      double* grad, int reverse) {
+  const int n_tan = grad ? cfg->n_params + cfg->ode_dim : 0;
+  const int N = cfg->num_derivatives + 1, D = cfg->ode_dim;
+  if (cfg->factorisation != PDQ_ISOTROPIC || D != 2 || (N != 4 && N != 5) || cfg->solver != PDQ_SOLVER ||
+      cfg->vector_field != PDQ_VF_LOTKA_VOLTERRA)
+    return 2;
+  std::vector<double> A, Q;
+  pdq::iwp_matrices(cfg->num_derivatives, A, Q);
+  std::vector<double> tinit = emu_taylor_tangents(cfg, n_inst, params, y0, grid, n_tan);
+  const int tpl = n_tan && !reverse ? 1 : 0, G = tpl ? n_tan : 1;
+  std::vector<double> shared(pdq::lml_shared_size(N, K, every));
+  std::vector<double> scratch(pdq::lml_shared_scratch_size(N, D, tpl, K, every, n_inst, G, reverse != 0));
+  pdq::LmlArgs a{};
+  a.cfg = *cfg;
+  a.n_inst = n_inst;
+  a.K = K;
+  a.every = every;
+  a.n_tan = n_tan;
+  a.average_pdfs = average;
+  a.G = G;
+  a.params = params;
+  a.tcoeffs = tinit.data();
+  a.times = grid;
+  a.data = data;
+  a.stds = stds;
+  a.Q = Q.data();
+  a.value = value;
+  a.grad = grad;
+  a.scratch = scratch.data();
+  a.shared = shared.data();
+  if (N == 4) lml_shared_emu<4, PDQ_VF_LOTKA_VOLTERRA>(a, reverse != 0);
+  else lml_shared_emu<5, PDQ_VF_LOTKA_VOLTERRA>(a, reverse != 0);
+  return 0;
+}
+
+// The off-grid marginal kernel (pdq_lane_offgrid.h) on the CPU.  Returns 2 for a shape or strategy it does not cover.
 int pdqemu_offgrid(const pdq_config* cfg, int n_inst, int K, const double* times, const double* mean,
                    const double* chol, const double* filt_mean, const double* filt_chol, const double* output_scale,
                    int n_query, const double* t_query, double* mean_out, double* chol_out) {
@@ -658,22 +723,23 @@ int pdqemu_offgrid(const pdq_config* cfg, int n_inst, int K, const double* times
   a.Q = Q.data();
   a.mean_out = mean_out;
   a.chol_out = chol_out;
-  const size_t total = (size_t)n_inst * n_query;
-  for (size_t q = 0; q < total; ++q) {
-    if (N == 4 && cfg->strategy == PDQ_FILTER) pdq::lane_offgrid<4, 2, PDQ_FILTER>(a, q);
-    else if (N == 4) pdq::lane_offgrid<4, 2, PDQ_FIXEDINTERVAL>(a, q);
-    else if (cfg->strategy == PDQ_FILTER) pdq::lane_offgrid<5, 2, PDQ_FILTER>(a, q);
-    else pdq::lane_offgrid<5, 2, PDQ_FIXEDINTERVAL>(a, q);
-  }
+  // the kernel, on two workgroups that stride over the queries
+  const int blocks = (int)(((size_t)n_inst * n_query + 63) / 64) > 1 ? 2 : 1;
+  emu_launch(blocks, 64, [&] {
+    if (N == 4 && cfg->strategy == PDQ_FILTER) pdq::lane_offgrid_kernel<4, 2, PDQ_FILTER>(a);
+    else if (N == 4) pdq::lane_offgrid_kernel<4, 2, PDQ_FIXEDINTERVAL>(a);
+    else if (cfg->strategy == PDQ_FILTER) pdq::lane_offgrid_kernel<5, 2, PDQ_FILTER>(a);
+    else pdq::lane_offgrid_kernel<5, 2, PDQ_FIXEDINTERVAL>(a);
+  });
   return 0;
 }
 
 
-// The posterior sampler (pdq_lane_sample.h) on the CPU, one (instance,
-// sample) lane after another.
+// The posterior sampler (pdq_lane_sample.h) on the CPU.  staged: the conditionals
+// of a tile read together (16 samples and more).
 int pdqemu_sample(const pdq_config* cfg, int n_inst, int K, const double* term_mean, const double* term_chol,
                   const double* cA, const double* cm, const double* cL, const double* ctl, const double* cto,
-                  int n_samples, const double* base, double* samples) {
+                  int n_samples, const double* base, double* samples, int staged) {
   const int N = cfg->num_derivatives + 1, D = cfg->ode_dim;
   if (cfg->factorisation == PDQ_BLOCKDIAG) return 2;
   const bool lane = cfg->factorisation == PDQ_ISOTROPIC && D == 2 && (N == 4 || N == 5) && cfg->lanes_per_instance <= 1;
@@ -700,10 +766,14 @@ int pdqemu_sample(const pdq_config* cfg, int n_inst, int K, const double* term_m
     for (size_t g = 0; g < (size_t)n_inst * n_samples; ++g) pdq::sample_generic(a, g, n, mc, dense, v.data(), 1);
     return 0;
   }
-  for (size_t g = 0; g < (size_t)n_inst * n_samples; ++g) {
-    if (N == 4) pdq::lane_sample<4, 2>(a, g);
-    else pdq::lane_sample<5, 2>(a, g);
-  }
+  // the kernel, on two workgroups that stride over the samples
+  const int blocks = (int)(((size_t)n_inst * n_samples + 63) / 64) > 1 ? 2 : 1;
+  emu_launch(blocks, 64, [&] {
+    if (N == 4 && staged) pdq::lane_sample_kernel<4, 2, true>(a);
+    else if (N == 4) pdq::lane_sample_kernel<4, 2, false>(a);
+    else if (staged) pdq::lane_sample_kernel<5, 2, true>(a);
+    else pdq::lane_sample_kernel<5, 2, false>(a);
+  });
   return 0;
 }
 

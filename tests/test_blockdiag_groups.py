@@ -39,12 +39,12 @@ def test_the_next_instance_waits_for_the_last_reads(emu, strategy, solver, K, gr
     cfg = capi.Config(factorisation="blockdiag", num_derivatives=nu, ode_dim=d, vector_field="burgers", n_params=2, strategy=strategy, solver=solver,
                       dt0=4e-5, rtol=1e-3, atol=1e-4)
     alone = [emu.solve(cfg, p[i : i + 1], tc[i : i + 1], t[i : i + 1], fixed_grid=grid) for i in range(B)]
-    emu.lib().pdqemu_set_lag(64, 20000)
+    emu.lib().pdqemu_set_lag(64, 128, 20000)
     try:
         together = emu.solve(cfg, p, tc, t, fixed_grid=grid)
         print(together["attempts"])
     finally:
-        emu.lib().pdqemu_set_lag(0, 0)
+        emu.lib().pdqemu_set_lag(0, 0, 0)
     for key, x in together.items():
         assert np.array_equal(x, np.concatenate([a[key] for a in alone]), equal_nan=True), key
 
