@@ -32,7 +32,11 @@
 // Storage per lane, in HBM element-major across the launch's lanes:
 // conditionals (Kobs - 1) x |cond|, nodes Kobs x (N + 1 + D), adjoints of the
 // conditional means (Kobs - 1) x N D, checkpoints ceil((K - 1) / C) x |slot|,
-// and two segment buffers of C slots.
+// two segment buffers of C slots, and the K - 1 output scales.  The scales are
+// replayed, not calibrated again: a calibration is the rest of a cancellation
+// (|m_1 - f(m_0)|), so that a last-bit difference between the forward pass's code
+// and the recomputation's moves it by 1e-8, and the walk back then belonged to
+// another trajectory (nu = 3, 40 steps: a gradient 2e-9 off its tangents').
 //
 // Two-wavefront form (SPLIT).  The forward pass is the LML kernel's split one
 // (lane_lml_forward_split: wavefront 1 runs each step's merge and the copy of
@@ -59,7 +63,7 @@ struct AdjLayout {
   using SL = SlotLayout<N, D>;
   static constexpr int node = N + 1 + D;  // gain, r00, whitened residuals
   static constexpr bool conds_first = true;  // conds sits at offset 0 (the split forward pass relies on it)
-  size_t conds, nodes, xibar, ckpt, seg, size;
+  size_t conds, nodes, xibar, ckpt, seg, scales, size;
   __device__ __host__ AdjLayout(int K, int every) {
     const size_t kobs = (size_t)(K - 1) / every + 1;
     const size_t nck = (size_t)(K - 2) / kAdjSegment + 1;
@@ -74,6 +78,8 @@ struct AdjLayout {
     o += nck * SL::size;
     seg = o;
     o += 2 * (size_t)kAdjSegment * SL::size;
+    scales = o;
+    o += (size_t)(K - 1);
     size = o;
   }
 };
@@ -124,7 +130,7 @@ __device__ __forceinline__ void adj_recompute_segment(const LaneCtx<N, D>& c, co
   for (int k = k0; k < k1; ++k) {
     adj_slot_out<N, D>(w, sf, at(lay.seg + ((size_t)buf * kAdjSegment + (k - k0)) * SL::size), n_lanes);
     if (k + 1 == k1) break;
-    lane_lml_step<N, D, 0>(c, 0, sf, pr, a.times[k + 1] - a.times[k]);
+    lane_lml_step<N, D, 0>(c, 0, sf, pr, a.times[k + 1] - a.times[k], at(lay.scales + k));
     const int tmp = sf;
     sf = pr;
     pr = tmp;
@@ -132,8 +138,8 @@ __device__ __forceinline__ void adj_recompute_segment(const LaneCtx<N, D>& c, co
   }
 }
 
-// The quantities of one forward step (from slot `from`, step h) that its
-// adjoint needs, recomputed from the slot: the transition's preconditioner,
+// The quantities of one forward step (from slot `from`, step h, the forward
+// pass's output scale sigma) that its adjoint needs, recomputed from the slot: the transition's preconditioner,
 // the revert's gain G_b and its output scales to_b, the prediction mean Pm
 // and the update's gain (solver.step / solver_dynamic.step, solvers.py:
 // 549-599, 702-733, with the operations of lane_lml_step).
@@ -143,29 +149,14 @@ struct AdjStep {
 };
 
 template <int N, int D>
-__device__ __forceinline__ void adj_recompute_step(const LaneCtx<N, D>& c, int from, double h, AdjStep<N, D>& s) {
+__device__ __forceinline__ void adj_recompute_step(const LaneCtx<N, D>& c, int from, double h, double sigma,
+                                                   AdjStep<N, D>& s) {
   const pdq_config& cfg = c.a->cfg;
   const double* __restrict__ Q = c.a->Q;
   const LaneWs<N, D>& w = c.w;
   double Sm[N * D], SLf[N * N];
   w.load_mL(from, Sm, SLf);
-  const double tn = w.at(from, LS_T) + h;
   lane_precon<N>(h, s.P, s.PI);
-  double sigma = 1.0, b[D];
-  if (cfg.solver == PDQ_SOLVER_DYNAMIC) {
-    const double s1 = lane_noise_scale(cfg, h, 1.0);
-    double Um[N * D], col[N + 1];
-    lane_apply_flat_mean<N, D>(s.P, s.PI, Sm, Um);
-    lane_lml_linearize<N, D, 0>(cfg, c.prm, 0, Um, tn, b);
-#pragma unroll
-    for (int r = 0; r < N; ++r) col[r] = fabs(s.P[1]) * (s1 * lane_iwp_q<N>(Q, 1, r));
-    col[N] = cfg.damp;
-    double om[D];
-#pragma unroll
-    for (int k = 0; k < D; ++k) om[k] = Um[1 * D + k] + b[k];
-    lane_qr<N + 1, 1, FxColumnRows<N>>(col);
-    sigma = lane_rms_zero<D>(om, col[0]);
-  }
   LCond<N, D> bw;
   double PL[N * N];
   lane_revert_prior<N, D>(Q, s.P, s.PI, lane_noise_scale(cfg, h, sigma), Sm, SLf, s.Pm, PL, LCondViewD<N, D>{&bw});
@@ -465,7 +456,8 @@ __device__ __forceinline__ void lane_adj_instance(const LArgs& la, const LmlArgs
     // the interval conditionals land where the LML kernel puts them: lay.conds
     // is the storage's first region
     static_assert(AdjLayout<N, D>::conds_first, "the split forward pass writes the conditionals at offset 0");
-    sf = lane_lml_forward_split<N, D, 0>(c, a, 0, lane, n_lanes, true, req, kAdjSegment, at(lay.ckpt), stage_tail);
+    sf = lane_lml_forward_split<N, D, 0>(c, a, 0, lane, n_lanes, true, req, kAdjSegment, at(lay.ckpt), stage_tail,
+                                         at(lay.scales));
 #endif
   } else {
     for (int k = 0; k < K - 1; ++k) {
@@ -474,6 +466,7 @@ __device__ __forceinline__ void lane_adj_instance(const LArgs& la, const LmlArgs
       const int tmp = sf;
       sf = pr;
       pr = tmp;
+      at(lay.scales + k)[0] = w.at(sf, LS_OS);
       if ((k + 1) % every == 0) {
         const CondStrided<N, D> dst{at(lay.conds + (size_t)((k + 1) / every - 1) * CL::size), n_lanes};
         cond_copy<N, D>(dst, w.cond(sf));
@@ -566,7 +559,7 @@ __device__ __forceinline__ void lane_adj_instance(const LArgs& la, const LmlArgs
       }
       adj_slot_in<N, D>(w, sf, at(lay.seg + ((size_t)buf * kAdjSegment + (k - k0)) * SL::size), n_lanes);
       AdjStep<N, D> s;
-      adj_recompute_step<N, D>(c, sf, a.times[k + 1] - a.times[k], s);
+      adj_recompute_step<N, D>(c, sf, a.times[k + 1] - a.times[k], *at(lay.scales + k), s);
       const bool ident = w.at(sf, LS_IDENT) != 0.0;
       adj_back_step<N, D>(cfg, c.prm, np, s.P, s.PI, s.Gb, s.tob, s.gain, s.Pm, ident, w.cond(sf), mbar, cbar, tbar);
     }

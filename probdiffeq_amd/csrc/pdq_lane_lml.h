@@ -94,11 +94,12 @@ struct LmlStepVals {
 // With `defer` the revert stops after its left half (lane_revert_left): the
 // conditional of slot `to` is finished by lane_revert_right from the stage
 // left in its storage and `stage_tail` (lane_lml_forward_split's second
-// wavefront).
+// wavefront).  `replay`: the step's output scale, recorded when it was first
+// taken, instead of a calibration.
 template <int N, int D, int TPL>
 __device__ __forceinline__ void lane_lml_step_part1(const LaneCtx<N, D * (1 + TPL)>& c, int q0, int from, int to,
                                                     double h, LmlStepVals<N, D * (1 + TPL)>& v, bool defer = false,
-                                                    double* stage_tail = nullptr) {
+                                                    double* stage_tail = nullptr, const double* replay = nullptr) {
   constexpr int MC = D * (1 + TPL);
   const pdq_config& cfg = c.a->cfg;
   const double* __restrict__ Q = c.a->Q;
@@ -111,18 +112,23 @@ __device__ __forceinline__ void lane_lml_step_part1(const LaneCtx<N, D * (1 + TP
   if (cfg.solver == PDQ_SOLVER_DYNAMIC) {
     // calibration at the output-scale-1 extrapolation; sigma is a constant
     // for the tangents (stop_gradient)
-    const double s1 = lane_noise_scale(cfg, h, 1.0);
-    double Um[N * MC], col[N + 1];
+    double Um[N * MC];
     lane_apply_flat_mean<N, MC>(v.P, v.PI, Sm, Um);
     lane_lml_linearize<N, D, TPL>(cfg, c.prm, q0, Um, v.tn, v.b);
+    if (replay) {
+      v.sigma = *replay;
+    } else {
+      const double s1 = lane_noise_scale(cfg, h, 1.0);
+      double col[N + 1];
 #pragma unroll
-    for (int r = 0; r < N; ++r) col[r] = fabs(v.P[1]) * (s1 * lane_iwp_q<N>(Q, 1, r));
-    col[N] = cfg.damp;
-    double om[D];
+      for (int r = 0; r < N; ++r) col[r] = fabs(v.P[1]) * (s1 * lane_iwp_q<N>(Q, 1, r));
+      col[N] = cfg.damp;
+      double om[D];
 #pragma unroll
-    for (int k = 0; k < D; ++k) om[k] = Um[1 * MC + k] + v.b[k];
-    lane_qr<N + 1, 1, FxColumnRows<N>>(col);
-    v.sigma = lane_rms_zero<D>(om, col[0]);
+      for (int k = 0; k < D; ++k) om[k] = Um[1 * MC + k] + v.b[k];
+      lane_qr<N + 1, 1, FxColumnRows<N>>(col);
+      v.sigma = lane_rms_zero<D>(om, col[0]);
+    }
   }
   PDQ_PHASE_BOUNDARY();
   if (defer)
@@ -152,11 +158,11 @@ __device__ __forceinline__ void lane_lml_step_part2(const LaneCtx<N, D * (1 + TP
 
 template <int N, int D, int TPL>
 __device__ __forceinline__ void lane_lml_step(const LaneCtx<N, D * (1 + TPL)>& c, int q0, int from, int to,
-                                              double h) {
+                                              double h, const double* replay = nullptr) {
   constexpr int MC = D * (1 + TPL);
   const LaneWs<N, MC>& w = c.w;
   LmlStepVals<N, MC> v;
-  lane_lml_step_part1<N, D, TPL>(c, q0, from, to, h, v);
+  lane_lml_step_part1<N, D, TPL>(c, q0, from, to, h, v, false, nullptr, replay);
   lane_merge<N, MC>(w.at(from, LS_IDENT) != 0.0, w.cond(from), w.cond(to), w.cond(to));
   PDQ_PHASE_BOUNDARY();
   lane_lml_step_part2<N, D, TPL>(c, q0, from, to, v);
@@ -180,12 +186,12 @@ __device__ __forceinline__ void lane_lml_step(const LaneCtx<N, D * (1 + TPL)>& c
 // > 0 wavefront 0 also stores step_from's whole slot before every
 // ckpt_every-th step (checkpoint j, before step j ckpt_every, at ckpt + j |slot|
 // n_lanes, element-major with stride n_lanes), once the previous step's merge
-// has completed.
+// has completed, and every step's output scale at scales (stride n_lanes).
 template <int N, int D, int TPL>
 __device__ __forceinline__ int lane_lml_forward_split(const LaneCtx<N, D * (1 + TPL)>& c, const LmlArgs& a, int q0,
                                                       size_t glane, size_t n_lanes, bool active, int* req,
                                                       int ckpt_every = 0, double* ckpt = nullptr,
-                                                      double* stage_tail = nullptr) {
+                                                      double* stage_tail = nullptr, double* scales = nullptr) {
   constexpr int MC = D * (1 + TPL);
   using CL = CondLayout<N, MC>;
   const bool defer = RevertStage<N, MC>::tail == 0 || stage_tail != nullptr;
@@ -221,6 +227,7 @@ __device__ __forceinline__ int lane_lml_forward_split(const LaneCtx<N, D * (1 + 
 #pragma unroll
         for (int e = 0; e < SlotLayout<N, MC>::size; ++e) dst[(size_t)e * n_lanes] = w.at(sf, e);
       }
+      if (scales && active) scales[(size_t)(k - 1) * n_lanes] = v.sigma;
       last[0] = 0;
       last[1] = -1;
       if (active) {

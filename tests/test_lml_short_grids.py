@@ -53,3 +53,12 @@ def test_edges_of_the_dispatch(nu, B, steps, every):
     _close(_run(nu, args, every, obs, lanes_per_instance=16), forward, steps)
     _close(_run(nu, args, every, obs, lml_gradient="reverse"), forward, steps)
     _close(_run(nu, args, every, obs, grad=False), forward, steps)
+
+
+@pytest.mark.parametrize("nu,steps,every", [(3, 40, 10), (4, 30, 3), (4, 1, 1)])
+def test_calibrated_adjoint_on_a_partial_segment(nu, steps, every):
+    """solver_dynamic keeps the lane kernels: its adjoint with one segment of fewer than 50 steps."""
+    print(f"lml dynamic case: nu={nu} steps={steps} every={every}", flush=True)
+    args, obs = _inputs(65, steps, every)
+    forward = _run(nu, args, every, obs, solver="dynamic")
+    _close(_run(nu, args, every, obs, solver="dynamic", lml_gradient="reverse"), forward, steps)
