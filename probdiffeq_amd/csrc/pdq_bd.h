@@ -37,7 +37,8 @@
 // at run time, sums by LDS exchanges and the controller in every wavefront,
 // 86.6 ms (8 100 cycles per attempt) with the filter's default options folded
 // in, sums by register moves and the controller in one wavefront; d = 64: 1.38
-// and 0.99 ms, d = 200: 6.9 and 5.1 ms.
+// and 0.99 ms, d = 200: 6.9 and 5.1 ms.  The smoothers spill; what their kernels
+// take from this is at bd_lead.
 //
 // The loops follow _ivpsolve/solvers_via_adaptive_steps.py:46-375 and
 // solvers.py:205-767 in the order of the lane-per-instance kernel

@@ -267,7 +267,7 @@ __device__ __forceinline__ void w_gemm_cols(int l, const double* X, const double
 // eliminates all of them at once, and the back substitution runs on the
 // right-hand sides' lanes.  Its time is the instructions of one wavefront, a
 // few thousand in sequence; the run-time-shape form waited for LDS operands.
-// 200 Matern solves (nu = 4, d = 2, 20 points): 142 -> 23.5 ms, the same bits.
+// 200 Matern solves (nu = 4, d = 2, 20 points): 154 -> 24.5 ms, the same bits.
 template <class SH>
 __device__ __forceinline__ void w_exp_transition(const WCtx<SH>& c, double dt) {
   constexpr int n = SH::nc, d = SH::d, N = SH::N, nn = SH::nn, m10 = SH::m10;

@@ -1,6 +1,6 @@
 // Kernel and launcher of one fixed shape of the cooperative solver
-// (pdq_coop_wave.h).  The shapes are compiled in two translation units, by
-// strategy, so that they build in parallel.
+// (pdq_coop_wave.h).  The shapes are compiled in three translation units
+// (filter, smoothers, exponential prior), so that they build in parallel.
 #pragma once
 
 #include <algorithm>

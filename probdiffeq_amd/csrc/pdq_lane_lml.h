@@ -1,4 +1,6 @@
-// Lane-per-instance marginal log-likelihood and its gradient (isotropic).
+// Lane-per-instance marginal log-likelihood and its gradient (isotropic;
+// solver_dynamic on the device: the uncalibrated solver's factors are the batch's,
+// pdq_lane_lml_shared.h).
 //
 // loss_lml_timeseries (estimators_and_losses.py:53-105) on the fixed-point
 // smoother's Markov sequence: a forward pass on a fixed grid with a reset

@@ -111,22 +111,6 @@ def lml_forward(cfg, grid_steps: int, observations: int, n_tan: int = 0) -> floa
     return nb * (grid_steps * step) + nb * lml
 
 
-ADJ_SEGMENT = 50  # grid steps per checkpoint segment of the reverse adjoint
-
-
-def lml_reverse(cfg, grid_steps: int, observations: int) -> float:
-    """FLOPs the reverse-mode adjoint of the isotropic lane LML executes: the forward pass, the
-    recomputation of every checkpoint segment and of every step's factors in the backward sweep
-    (three forward passes' worth of factor work), and the adjoint of the mean recursions, which
-    costs what one more set of mean columns costs in the forward direction (step and scan)."""
-    nc, mc, ko, nb = dims(cfg)
-    step0 = lml_forward(cfg, grid_steps, 0, 0) / max(1, grid_steps)
-    step1 = lml_forward(cfg, grid_steps, 0, 1) / max(1, grid_steps)
-    scan0 = lml_forward(cfg, 0, observations, 0)
-    scan1 = lml_forward(cfg, 0, observations, 1)
-    return nb * (3 * grid_steps * step0 + grid_steps * (step1 - step0) + scan0 + (scan1 - scan0))
-
-
 def lml_batch(cfg, n_inst: int, grid_steps: int, observations: int, n_tan: int = 0, reverse: bool = False) -> float:
     """FLOPs of a batch of isotropic lane LMLs without calibration (PDQ_SOLVER): the grid steps' factors
     once for the batch, and per instance the mean columns through them and the reverse scan (whose
@@ -146,34 +130,15 @@ def lml_batch_bytes(cfg, n_inst: int, observations: int, grid_points: int, n_tan
     """Algorithmic HBM bytes of the same: inputs and outputs (the Taylor coefficients carry their
     sensitivities), the shared records written and read once, and per instance the intervals' noise
     means (with their tangents), and for the adjoint node data, the means' adjoints and a checkpoint of
-    the mean every 16 steps, each written and read once."""
+    the mean every 16 (nu = 3) or 12 (nu = 4) steps, each written and read once."""
     N, d = cfg.num_derivatives + 1, cfg.ode_dim
     n_theta = cfg.n_params + d
     shared = (grid_points - 1) * (4 * N + 2 * N * N + 1 + N * (N + 1)) + (observations - 1) * (N * N + N * (N + 1) // 2 + 2 * N)
     per_inst = (observations - 1) * N * d * (1 + n_tan)
     if reverse:
-        per_inst = 2 * (observations - 1) * N * d + observations * (N + 1 + d) + (grid_points - 1) / 16 * N * d
+        per_inst = 2 * (observations - 1) * N * d + observations * (N + 1 + d) + (grid_points - 1) / (16 if N == 4 else 12) * N * d
     inputs = n_inst * (cfg.n_params + d + observations * (d + 1) + N * d * (1 + n_theta)) + grid_points
     return 8.0 * (inputs + n_inst * (1 + n_theta) + 2 * shared + 2 * n_inst * per_inst)
-
-
-def lml_reverse_bytes(cfg, n_inst: int, observations: int, grid_points: int) -> float:
-    """Algorithmic HBM bytes of the reverse adjoint: inputs and outputs as in the forward LML
-    (the Taylor coefficients carry their n_params + d sensitivities), and per instance its storage
-    written once and read once: the interval conditionals, each observation node's gain, factor
-    and residuals, the adjoints of the conditional means, the checkpoints every 50 steps, and
-    every step's slot within its segment."""
-    N, d = cfg.num_derivatives + 1, cfg.ode_dim
-    tri = N * (N + 1) // 2
-    slot = 8 + N * d + tri + N * N + N * d + tri + 2 * N
-    cond = N * N + N * d + tri + 2 * N
-    steps = grid_points - 1
-    per_inst = (observations - 1) * cond + observations * (N + 1 + d) + (observations - 1) * N * d
-    per_inst += ((steps - 1) // ADJ_SEGMENT + 1) * slot + steps * slot
-    n_theta = cfg.n_params + d
-    inputs = n_inst * (cfg.n_params + d + observations * (d + 1) + N * d * (1 + n_theta)) + grid_points
-    outputs = n_inst * (1 + n_theta)
-    return 8.0 * (inputs + outputs + 2 * n_inst * per_inst)
 
 
 def solve_bytes(cfg, n_inst: int, K: int) -> float:
@@ -191,19 +156,6 @@ def solve_bytes(cfg, n_inst: int, K: int) -> float:
         per_ckpt += ms + cs + cond                   # filtering marginal + backward conditional
         reread = (K - 1) * cond
     return 8.0 * n_inst * (inputs + K * per_ckpt + reread)
-
-
-def lml_bytes(cfg, n_inst: int, observations: int, grid_points: int, n_tan: int = 0) -> float:
-    """Algorithmic HBM bytes of one batched LML (+ gradient): inputs (params, y0, the grid, data
-    and one std per observation), outputs (value, gradient), and the backward conditional of every
-    interval between observations (factors once, mean columns with their tangents) written by the
-    forward pass and read back by the reverse scan."""
-    nc, mc, _, nb = dims(cfg, n_tan)
-    d = cfg.ode_dim
-    cond = nb * (2 * nc * nc + 2 * nc) + nc * mc  # A, noise factor, to_latent, to_observed; noise mean
-    inputs = n_inst * (cfg.n_params + d + observations * (d + 1)) + grid_points
-    outputs = n_inst * (1 + n_tan)
-    return 8.0 * (inputs + outputs + 2 * n_inst * (observations - 1) * cond)
 
 
 def offgrid(cfg) -> float:
